@@ -323,7 +323,7 @@ EwaldDev stage_ewald(Store &S, FourierSum &fs, const Bins &B, const Modes &M, co
     d.real = S.make<double>(n);
     d.far = S.make<double>(n);
     d.phi = S.make<double>(n);
-    fs.setup(theta, n, 2 * M.mmax[0] + 1, 2 * M.mmax[1] + 1, 2 * M.mmax[2] + 1, M.mijk, M.mw, S.arena, max_blocks);
+    fs.setup(theta, n, M.mijk, M.mw, S.arena, max_blocks);
     return d;
 }
 
@@ -494,7 +494,7 @@ void ewald_sum_targets(const double *cell, int n, const double *pos, const doubl
     d_real.alloc(sizeof(double) * (size_t)m);
     d_far.alloc(sizeof(double) * (size_t)m);
     FourierSum fs;
-    fs.setup(theta, n, 2 * M.mmax[0] + 1, 2 * M.mmax[1] + 1, 2 * M.mmax[2] + 1, M.mijk, M.mw);
+    fs.setup(theta, n, M.mijk, M.mw);
     fs.run_at(d_q.as<double>(), d_ttheta.as<double>(), m, d_far.as<double>(), st);
     hipLaunchKernelGGL(k_ewald_real_targets, dim3(m), dim3(EW_THREADS), 0, st, d_pts.as<double4>(), d_bstart.as<int>(),
                        d_nptr.as<int>(), d_nbin.as<int>(), d_nshift.as<double4>(), d_tsorted.as<int>(),

@@ -2379,214 +2379,311 @@ __global__ void k_fill(R *__restrict__ p, R v, int n) {
 }
 
 // ------------------------------------------------------------------ far field
-// Half-space modes with nonzero weight are grouped in lines of constant (j, k) with i
-// contiguous; each line is cut into chunks of up to FF_CHUNK consecutive i.  Chunk c
-// covers modes chunk_m0[c] .. + chunk_len[c] - 1 with indices (chunk_i0[c] + r, j, k).
-// All far-field arithmetic is FP64.
-constexpr int FF_CHUNK = 8;
-constexpr int FF_TP = 16;  // points per LDS tile
-constexpr int FF_QUAD = 4;  // structure factors per scalar load in the evaluation
-constexpr int FF_MANY_S = 4;  // vectors per workgroup of a many-vector structure-factor launch
-constexpr int FF_MANY_E = 2;  // vectors per workgroup of a many-vector evaluation
+// Half-space modes with nonzero weight come in lines of constant (j, k) with i contiguous.
+// All far-field arithmetic is FP64, on the matrix cores: along i the phases are real,
+//   sum_i f_i e^{-+ i i th1} = sum_{i >= 0} (combinations of f_i, f_-i) x (cos i th1, sin i th1),
+// so both directions are products of a real table trig[point][2 i + (0 cos, 1 sin)] with the
+// lines' complex parts, 2 multiply-adds per mode and point where a recurrence per mode takes
+// 6 (structure factors) and a Horner step 4 (evaluation).  Lines are sorted by their largest
+// |i| and taken 16 at a time (line tiles), so that a tile only spends the columns it needs.
+// The rows of a tile of points (trig along axis 0, e^{i m th} for m >= 0 along axes 1 and 2:
+// negative m by conjugation) are tabulated in LDS by recurrence from one sincos per axis.
+// The vector kernels these replace ran a lane per mode chunk or per point and were bound by
+// latency (one point per lane of a 4-workgroup launch at N = 1e3) and FP64 issue.
+constexpr int FF_UNITS = 16;  // most (line tile, 16 trig columns) units of a structure-factor workgroup
+constexpr int FF_MANY = 2;    // vectors per workgroup of a many-vector launch
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
     return make_double2(fma(a.x, b.x, -a.y * b.y), fma(a.x, b.y, a.y * b.x));
 }
 
-// Partial structure factors per workgroup of points:
-//   Sp[blk][m] = sum_{points of blk} q e^{-i(i th1 + j th2 + k th3)}.
-// Per point tile, e^{-i m th} for every axis index m is tabulated in LDS (FP64 recurrence
-// from one sincos per axis), with the tile's charges beside it.  A lane owns one chunk: per
-// point it gathers its first mode's factor from the three tables, walks the chunk by
-// multiplying with e^{-i th1} and adds q times each factor.  Workgroup z of a many-vector
-// launch takes vectors V z .. V z + V - 1 (< nv; vector v's charges at q + v vs_q, its partial
-// sums at Sp + v vs_sp): the factors are formed once for its V vectors, and each vector's sums
-// are those of a one-vector launch, bit for bit.
-template <int V>
-__global__ __launch_bounds__(256) void k_ff_structure(const double *__restrict__ theta, const double *__restrict__ q, int n,
-                                                       int ms, int mt, int mu, const int *__restrict__ chunk_ijk,
-                                                       const int *__restrict__ chunk_m0, const int *__restrict__ chunk_len,
-                                                       int n_chunks, int n_modes, double2 *__restrict__ Sp,
-                                                       long long vs_q = 0, long long vs_sp = 0, int nv = 1) {
-    extern __shared__ double2 ff_lds[];
-    const int v0 = blockIdx.z * V;
-    double2 *E1 = ff_lds, *E2 = E1 + FF_TP * ms, *E3 = E2 + FF_TP * mt, *Est = E3 + FF_TP * mu;
-    double *Qs = reinterpret_cast<double *>(Est + FF_TP);  // [V][FF_TP]
-    const int c = blockIdx.y * blockDim.x + threadIdx.x;
-    const bool active = c < n_chunks;
-    const int ci = active ? chunk_ijk[3 * c] + ms / 2 : 0;
-    const int cj = active ? chunk_ijk[3 * c + 1] + mt / 2 : 0;
-    const int ck = active ? chunk_ijk[3 * c + 2] + mu / 2 : 0;
-    const int len = active ? chunk_len[c] : 0;
-    double2 acc[V][FF_CHUNK];
-#pragma unroll
-    for (int v = 0; v < V; ++v)
-#pragma unroll
-        for (int r = 0; r < FF_CHUNK; ++r) acc[v][r] = make_double2(0, 0);
-    for (int p0 = blockIdx.x * FF_TP; p0 < n; p0 += gridDim.x * FF_TP) {
-        __syncthreads();
-        for (int t = threadIdx.x; t < FF_TP * 3; t += blockDim.x) {
-            const int pp = t % FF_TP, ax = t / FF_TP, gp = p0 + pp;
-            const int cnt = ax == 0 ? ms : (ax == 1 ? mt : mu);
-            const int lo = -(cnt / 2);
-            double2 *row = (ax == 0 ? E1 : (ax == 1 ? E2 : E3)) + pp * cnt;
-            const double th = gp < n ? theta[3 * (size_t)gp + ax] : 0.0;
-            double s1, c1, sl, cl;
-            sincos(th, &s1, &c1);
-            sincos(-th * lo, &sl, &cl);
-            const double2 step = make_double2(c1, -s1);  // e^{-i th}
-            if (ax == 0) Est[pp] = step;
-            double2 cur = make_double2(cl, sl);  // e^{-i lo th}
-            for (int m = 0; m < cnt; ++m) {
+// Index bounds of the listed modes: |i| <= I, |j| <= J, |k| <= K.  LDS row of a point:
+// ts() doubles of trig (an odd count: the evaluation reads 16 points' rows at once), then
+// J + 1 and K + 1 complex phases.
+struct FfDims {
+    int I, J, K;
+    __host__ __device__ int ts() const { return 2 * I + 3; }
+    __host__ __device__ size_t lds_bytes(int tp) const {
+        return (size_t)tp * (sizeof(double) * ts() + sizeof(double2) * (J + 1 + K + 1));
+    }
+};
+
+// LDS tables of points p0 .. p0 + tp - 1 (phases e^{sgn i m th}; points past n: theta 0).  The
+// pad column of trig is 0.
+__device__ __forceinline__ void ff_tables(double *trig, double2 *E2, double2 *E3, const double *__restrict__ theta, int n,
+                                          int p0, int tp, FfDims d, double sgn) {
+    for (int t = threadIdx.x; t < tp * 3; t += blockDim.x) {
+        const int pp = t % tp, ax = t / tp, gp = p0 + pp;
+        double s1, c1;
+        sincos(gp < n ? theta[3 * (size_t)gp + ax] : 0.0, &s1, &c1);
+        if (ax == 0) {
+            double *row = trig + (size_t)pp * d.ts();
+            double2 cur = make_double2(1, 0);
+            for (int m = 0; m <= d.I; ++m) {
+                row[2 * m] = cur.x;
+                row[2 * m + 1] = cur.y;
+                cur = cmul(cur, make_double2(c1, s1));
+            }
+            row[2 * d.I + 2] = 0;
+        } else {
+            const int cnt = ax == 1 ? d.J : d.K;
+            double2 *row = (ax == 1 ? E2 : E3) + (size_t)pp * (cnt + 1);
+            const double2 step = make_double2(c1, sgn * s1);
+            double2 cur = make_double2(1, 0);
+            for (int m = 0; m <= cnt; ++m) {
                 row[m] = cur;
                 cur = cmul(cur, step);
             }
         }
-        for (int t = threadIdx.x; t < FF_TP * V; t += blockDim.x) {
-            const int pp = t % FF_TP, v = t / FF_TP, gp = p0 + pp;
-            Qs[t] = gp < n && v0 + v < nv ? q[(long long)(v0 + v) * vs_q + gp] : 0.0;
+    }
+}
+
+// Partial structure factors per workgroup column of points:
+//   Sp[blk][m] = sum_{points of blk} q e^{-i(i th1 + j th2 + k th3)}.
+// Unit (line tile, ct): the 16 x 16 products of 16 lines' a = e^{-i(j th2 + k th3)} (real and
+// imaginary part, one accumulator each) with 16 trig columns times q, summed over points 4 at a time
+// by v_mfma_f64_16x16x4f64 (lane l supplies A[l % 16][l / 16] = its line's a at point l / 16 and
+// B[l / 16][l % 16] = q trig, and holds D[l / 16 + 4 e][l % 16]).  A wave owns U units (those
+// past the last are formed and not stored: with a test per unit the compiler cannot have the
+// LDS reads of all U in flight), a workgroup 4 U (grid y).  At the end the cos and sin columns
+// of a line (neighbouring lanes) combine into modes +i and -i.  Workgroup z of a many-vector
+// launch takes vectors V z .. V z + V - 1 (< nv; vector v's charges at q + v vs_q, its sums at
+// Sp + v vs_sp) on one set of tables and phases; each vector's sums are those of a one-vector
+// launch, bit for bit.
+template <int U, int V>
+__global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restrict__ theta, const double *__restrict__ q, int n,
+                                                       int tp, FfDims d, const int4 *__restrict__ lines,
+                                                       const int *__restrict__ line_m0, const int2 *__restrict__ units,
+                                                       int n_units, int n_modes, double2 *__restrict__ Sp,
+                                                       long long vs_q = 0, long long vs_sp = 0, int nv = 1) {
+    extern __shared__ double2 ff_lds[];
+    __shared__ double Qs[V][32];
+    const int v0 = blockIdx.z * V;
+    double *trig = reinterpret_cast<double *>(ff_lds);
+    const int ts = d.ts();
+    double2 *E2 = reinterpret_cast<double2 *>(trig + (size_t)tp * ts), *E3 = E2 + (size_t)tp * (d.J + 1);
+    const int lane = threadIdx.x & 63, kk = lane >> 4, jj = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int u0 = (blockIdx.y * 4 + w) * U;
+    int o2[U], o3[U], oc[U];  // LDS offsets of the lane's j and k phases, and of its trig column
+    double s2[U], s3[U];      // signs of j and k
+    c2p_d4 are[V][U], aim[V][U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int2 un = units[min(u0 + u, n_units - 1)];
+        const int4 ln = lines[un.x * 16 + jj];
+        o2[u] = abs(ln.x);
+        o3[u] = abs(ln.y);
+        s2[u] = ln.x < 0 ? -1.0 : 1.0;
+        s3[u] = ln.y < 0 ? -1.0 : 1.0;
+        oc[u] = 16 * un.y + jj;
+#pragma unroll
+        for (int v = 0; v < V; ++v) are[v][u] = aim[v][u] = c2p_d4{0, 0, 0, 0};
+    }
+    for (int p0 = blockIdx.x * tp; p0 < n; p0 += gridDim.x * tp) {
+        __syncthreads();
+        ff_tables(trig, E2, E3, theta, n, p0, tp, d, -1.0);
+        // (from the last threads down: the first ones are busy with the tables)
+        for (int t = 255 - (int)threadIdx.x; t < tp * V; t += 256) {
+            const int pp = t % tp, v = t / tp;
+            Qs[v][pp] = p0 + pp < n && v0 + v < nv ? q[(long long)(v0 + v) * vs_q + p0 + pp] : 0.0;
         }
         __syncthreads();
-        if (active) {
-            const int np = min(FF_TP, n - p0);
-            for (int pp = 0; pp < np; ++pp) {
-                const double2 st = Est[pp];
-                double qq[V];
+        for (int k0 = 0; k0 < tp; k0 += 4) {  // (a wave-uniform count: the accumulators stay in place)
+            const int p = k0 + kk;
+            const double *tr = trig + (size_t)p * ts;
+            const double2 *r2 = E2 + (size_t)p * (d.J + 1), *r3 = E3 + (size_t)p * (d.K + 1);
+            double b[U];
+            double2 x[U], y[U];
+            double qq[V];
 #pragma unroll
-                for (int v = 0; v < V; ++v) qq[v] = Qs[v * FF_TP + pp];
-                double2 cur = cmul(cmul(E1[pp * ms + ci], E2[pp * mt + cj]), E3[pp * mu + ck]);
+            for (int v = 0; v < V; ++v) qq[v] = Qs[v][p];
 #pragma unroll
-                for (int r = 0; r < FF_CHUNK; ++r) {
+            for (int u = 0; u < U; ++u) {
+                b[u] = tr[oc[u]];
+                x[u] = r2[o2[u]];
+                y[u] = r3[o3[u]];
+            }
 #pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        acc[v][r].x = fma(qq[v], cur.x, acc[v][r].x);
-                        acc[v][r].y = fma(qq[v], cur.y, acc[v][r].y);
-                    }
-                    cur = cmul(cur, st);
+            for (int u = 0; u < U; ++u) {
+                const double xi = s2[u] * x[u].y, yi = s3[u] * y[u].y;
+                const double ar = fma(x[u].x, y[u].x, -xi * yi), ai = fma(x[u].x, yi, xi * y[u].x);
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const double qb = qq[v] * b[u];
+                    are[v][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, qb, are[v][u], 0, 0, 0);
+                    aim[v][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, qb, aim[v][u], 0, 0, 0);
                 }
             }
         }
     }
-    if (active) {
-        const int m0 = chunk_m0[c];
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
-            if (v0 + v >= nv) break;
-            double2 *out = Sp + (long long)(v0 + v) * vs_sp + (size_t)blockIdx.x * n_modes + m0;
+    for (int u = 0; u < U; ++u) {
+        if (u0 + u >= n_units) break;
+        const int2 un = units[u0 + u];
+        const int c = 16 * un.y + jj, i = (c & 1) ? -(c >> 1) : (c >> 1);  // even: cos, mode +i; odd: sin, mode -i
 #pragma unroll
-            for (int r = 0; r < FF_CHUNK; ++r)
-                if (r < len) out[r] = acc[v][r];
-        }
-    }
-}
-
-// S[pidx[m]] = w[m] * sum_blk Sp[blk][m]: workgroup = 32 modes x 8 partial-sum lanes.
-__global__ __launch_bounds__(256) void k_ff_reduce(const double2 *__restrict__ Sp, int nblk, const double *__restrict__ w,
-                                                   const int *__restrict__ pidx, int n_modes, double2 *__restrict__ S,
-                                                   long long vs_sp = 0, long long vs_s = 0) {
-    __shared__ double2 part[8][32];
-    Sp += (long long)blockIdx.z * vs_sp;  // vector blockIdx.z of a many-vector launch
-    S += (long long)blockIdx.z * vs_s;
-    const int ml = threadIdx.x & 31, g = threadIdx.x >> 5;
-    const int m = blockIdx.x * 32 + ml;
-    double sr = 0, si = 0;
-    if (m < n_modes)
-        for (int b = g; b < nblk; b += 8) {
-            const double2 v = Sp[(size_t)b * n_modes + m];
-            sr += v.x;
-            si += v.y;
-        }
-    part[g][ml] = make_double2(sr, si);
-    __syncthreads();
-    if (g == 0 && m < n_modes) {
-        double tr = 0, ti = 0;
-        for (int k = 0; k < 8; ++k) {
-            tr += part[k][ml].x;
-            ti += part[k][ml].y;
-        }
-        S[pidx[m]] = make_double2(tr * w[m], ti * w[m]);
-    }
-}
-
-// e *= z^d for a wave-uniform exponent d by square-and-multiply (|z| = 1, z^-1 = conj z).
-__device__ __forceinline__ void ff_advance(double2 &e, int d, double2 z) {
-    if (d < 0) {
-        z.y = -z.y;
-        d = -d;
-    }
-    while (d) {
-        if (d & 1) e = cmul(e, z);
-        d >>= 1;
-        if (d) z = cmul(z, z);
-    }
-}
-
-// far[u] = sum_m Re( S[m] e^{+i(i th1 + j th2 + k th3)} ), one point per lane.  Line L =
-// (j, k, ilo, nq) holds its weighted S at S[base[L] ..], padded to nq * FF_QUAD entries; its
-// sum over i is a Horner polynomial in z1 = e^{i th1} with wave-uniform coefficients (read
-// FF_QUAD at a time), multiplied by z1^ilo z2^j z3^k, which is advanced from the previous
-// line by (small) exponent steps.  Workgroup z of a many-vector launch evaluates vectors
-// V z .. V z + V - 1 (< nv; S at S + v vs_s, output at far + v vs_far) with one set of
-// phases; each vector's sums are those of a one-vector launch, bit for bit.
-template <int V>
-__global__ __launch_bounds__(256) void k_ff_eval(const double *__restrict__ theta, int n, const int4 *__restrict__ lines,
-                                                 const int *__restrict__ base, int n_lines, const double2 *__restrict__ S,
-                                                 double *__restrict__ far, long long vs_s = 0, long long vs_far = 0,
-                                                 int nv = 1) {
-    const int v0 = blockIdx.z * V;
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    const int uc = u < n ? u : n - 1;
-    double2 z1, z2, z3;
-    {
-        double s, c;
-        sincos(theta[3 * (size_t)uc], &s, &c);
-        z1 = make_double2(c, s);
-        sincos(theta[3 * (size_t)uc + 1], &s, &c);
-        z2 = make_double2(c, s);
-        sincos(theta[3 * (size_t)uc + 2], &s, &c);
-        z3 = make_double2(c, s);
-    }
-    // vectors past nv read vector v0's sums (in bounds) and store nothing
-    const double2 *Sv[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) Sv[v] = S + (long long)(v0 + (v0 + v < nv ? v : 0)) * vs_s;
-    double2 e1 = make_double2(1, 0), e2 = make_double2(1, 0), e3 = make_double2(1, 0);
-    int ic = 0, jc = 0, kc = 0;
-    double acc[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] = 0;
-    for (int L = 0; L < n_lines; ++L) {
-        const int4 d = lines[L];
-        const int bL = base[L];
-        ff_advance(e1, d.z - ic, z1);
-        ff_advance(e2, d.x - jc, z2);
-        ff_advance(e3, d.y - kc, z3);
-        ic = d.z;
-        jc = d.x;
-        kc = d.y;
-        double2 h[V];
-#pragma unroll
-        for (int v = 0; v < V; ++v) h[v] = make_double2(0, 0);
-        for (int qd = d.w - 1; qd >= 0; --qd) {
+        for (int e = 0; e < 4; ++e) {
+            const int line = un.x * 16 + kk + 4 * e;
+            const int4 ln = lines[line];
+            const bool mode = i >= ln.z && i <= ln.w && !((c & 1) && i == 0);
+            double2 *out = Sp + (size_t)blockIdx.x * n_modes + line_m0[line] + i - ln.z;
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                double2 sv[FF_QUAD];
-#pragma unroll
-                for (int r = 0; r < FF_QUAD; ++r) sv[r] = Sv[v][bL + FF_QUAD * qd + r];
-#pragma unroll
-                for (int r = FF_QUAD - 1; r >= 0; --r)
-                    h[v] = make_double2(fma(h[v].x, z1.x, fma(-h[v].y, z1.y, sv[r].x)),
-                                        fma(h[v].x, z1.y, fma(h[v].y, z1.x, sv[r].y)));
+                const double mr = are[v][u][e], mi = aim[v][u][e], pr = __shfl_xor(mr, 1), pi = __shfl_xor(mi, 1);
+                // S(+i) = C - i D, S(-i) = C + i D (C the cos, D the sin column)
+                if (mode && v0 + v < nv)
+                    out[(long long)(v0 + v) * vs_sp] = (c & 1) ? make_double2(pr - mi, pi + mr) : make_double2(mr + pi, mi - pr);
             }
         }
-        const double2 bs = cmul(cmul(e1, e2), e3);
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc[v] = fma(h[v].x, bs.x, fma(-h[v].y, bs.y, acc[v]));
     }
-    if (u < n) {
+}
+
+// Column sums of the partial structure factors, weighted, as the evaluation's operands:
+// with T(+-i) = w S(+-i), line (j, k) contributes Re(e^{i(j th2 + k th3)} sum_i (Gc cos i th1 +
+// Gs sin i th1)), Gc = T(i) + T(-i), Gs = i (T(i) - T(-i)).  Tile t's G starts at info[t].y:
+// [ks][re, im][64], column 4 ks + l / 16 of line l % 16 at lane l.  One workgroup per line, its
+// modes contiguous: 32 modes x 16 groups of columns at a time, the groups added in order, the
+// weighted sums of the line kept in LDS for the (+i, -i) pairs.  (32 modes x 8 groups per
+// workgroup, one thread per 64 columns, left 44 workgroups to read all partial sums: 21 us at
+// N = 1e4, 110 us at 2.5e5 beside the near field.)
+__global__ __launch_bounds__(512) void k_ff_reduce(const double2 *__restrict__ Sp, int nblk, const double *__restrict__ w,
+                                                   const int4 *__restrict__ lines, const int *__restrict__ line_m0,
+                                                   const int2 *__restrict__ info, int n_modes, double *__restrict__ G,
+                                                   long long vs_sp = 0, long long vs_g = 0) {
+    extern __shared__ double2 ff_lds[];
+    double2 *part = ff_lds, *T = ff_lds + 512;  // T[mode of the line]
+    const int4 ln = lines[blockIdx.x];
+    const int len = ln.w - ln.z + 1, m0 = line_m0[blockIdx.x];
+    if (len <= 0) return;  // padding line: its G stays zero
+    Sp += (long long)blockIdx.z * vs_sp + m0;
+    const int l = threadIdx.x & 31, g = threadIdx.x >> 5;
+    for (int c = 0; c < len; c += 32) {
+        double2 a = make_double2(0, 0);
+        if (c + l < len) {
+#pragma unroll 4
+            for (int k = g; k < nblk; k += 16) {
+                const double2 x = Sp[(size_t)k * n_modes + c + l];
+                a.x += x.x;
+                a.y += x.y;
+            }
+        }
+        part[threadIdx.x] = a;
+        __syncthreads();
+        if (g == 0 && c + l < len) {
+            double2 t = make_double2(0, 0);
 #pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (v0 + v < nv) far[(long long)(v0 + v) * vs_far + u] = acc[v];
+            for (int k = 0; k < 16; ++k) {
+                t.x += part[32 * k + l].x;
+                t.y += part[32 * k + l].y;
+            }
+            const double wm = w[m0 + c + l];
+            T[c + l] = make_double2(t.x * wm, t.y * wm);
+        }
+        __syncthreads();
+    }
+    const int2 inf = info[blockIdx.x >> 4];
+    G += (long long)blockIdx.z * vs_g + inf.y;
+    for (int i = threadIdx.x; i <= inf.x; i += 512) {
+        double2 u = make_double2(0, 0), v = make_double2(0, 0);
+        if (i >= ln.z && i <= ln.w) u = T[i - ln.z];
+        if (i > 0 && -i >= ln.z && -i <= ln.w) v = T[-i - ln.z];
+        double *o = G + (size_t)(i >> 1) * 128 + (i & 1) * 32 + (blockIdx.x & 15);  // columns 2 i, 2 i + 1
+        o[0] = u.x + v.x;
+        o[64] = u.y + v.y;
+        o[16] = v.y - u.y;
+        o[64 + 16] = u.x - v.x;
+    }
+}
+
+// far[u] = sum_m Re( S[m] e^{+i(i th1 + j th2 + k th3)} ).  Per line tile the products
+// D = trig x G (points by lines, real and imaginary part) on the matrix cores, then
+// Re(e^{i(j th2 + k th3)} D) added up per point.  A workgroup takes 16 RT points; its 4 waves
+// share the line tiles, so that also a few hundred points fill several CUs, and their sums
+// are added in wave order.  Workgroup z of a many-vector launch evaluates vectors V z .. (< nv;
+// G + v vs_g, output at far + v vs_far) on one set of tables and phases, each as a one-vector
+// launch does, bit for bit.
+template <int RT, int V>
+__global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ theta, int n, FfDims d,
+                                                 const int4 *__restrict__ lines, const int2 *__restrict__ info, int n_lt,
+                                                 const double *__restrict__ G, double *__restrict__ far,
+                                                 long long vs_g = 0, long long vs_far = 0, int nv = 1) {
+    extern __shared__ double2 ff_lds[];
+    constexpr int TP = 16 * RT;
+    __shared__ double red[V][4][TP];
+    const int v0 = blockIdx.z * V;
+    double *trig = reinterpret_cast<double *>(ff_lds);
+    const int ts = d.ts();
+    double2 *E2 = reinterpret_cast<double2 *>(trig + (size_t)TP * ts), *E3 = E2 + (size_t)TP * (d.J + 1);
+    const int p0 = blockIdx.x * TP;
+    ff_tables(trig, E2, E3, theta, n, p0, TP, d, 1.0);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, kk = lane >> 4, jj = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double acc[V][RT][4];
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[v][rt][e] = 0;
+    for (int lt = w; lt < n_lt; lt += 4) {
+        const int2 inf = info[lt];
+        const int nks = (inf.x + 2) >> 1;  // 4 columns each: 2 (imax + 1), rounded up
+        const int4 ln = lines[lt * 16 + jj];
+        c2p_d4 dr[V][RT], di[V][RT];
+        const double *tr = trig + (size_t)jj * ts + kk;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            // (a vector past nv repeats vector v0 and stores nothing)
+            const double *g = G + (long long)(v0 + (v0 + v < nv ? v : 0)) * vs_g + inf.y + lane;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) dr[v][rt] = di[v][rt] = c2p_d4{0, 0, 0, 0};
+            double br = g[0], bi = g[64];
+            for (int ks = 0; ks < nks; ++ks) {
+                // the next step's operands (the last step reads the table's padding)
+                const double nr = g[(size_t)(ks + 1) * 128], ni = g[(size_t)(ks + 1) * 128 + 64];
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const double a = tr[(size_t)rt * 16 * ts + 4 * ks];
+                    dr[v][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, br, dr[v][rt], 0, 0, 0);
+                    di[v][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bi, di[v][rt], 0, 0, 0);
+                }
+                br = nr;
+                bi = ni;
+            }
+        }
+        const int o2 = abs(ln.x), o3 = abs(ln.y);
+        const double s2 = ln.x < 0 ? -1.0 : 1.0, s3 = ln.y < 0 ? -1.0 : 1.0;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = 16 * rt + kk + 4 * e;
+                const double2 x = E2[(size_t)p * (d.J + 1) + o2], y = E3[(size_t)p * (d.K + 1) + o3];
+                const double xi = s2 * x.y, yi = s3 * y.y;
+                const double ar = fma(x.x, y.x, -xi * yi), ai = fma(x.x, yi, xi * y.x);
+#pragma unroll
+                for (int v = 0; v < V; ++v)
+                    acc[v][rt][e] = fma(ar, dr[v][rt][e], fma(-ai, di[v][rt][e], acc[v][rt][e]));
+            }
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                double t = acc[v][rt][e];
+#pragma unroll
+                for (int m = 8; m >= 1; m >>= 1) t += __shfl_xor(t, m, 16);
+                if (jj == 0) red[v][w][16 * rt + kk + 4 * e] = t;
+            }
+    __syncthreads();
+    for (int t = threadIdx.x; t < TP * V; t += blockDim.x) {
+        const int v = t / TP, p = t % TP;
+        if (p0 + p < n && v0 + v < nv)
+            far[(long long)(v0 + v) * vs_far + p0 + p] = red[v][0][p] + red[v][1][p] + red[v][2][p] + red[v][3][p];
     }
 }
 

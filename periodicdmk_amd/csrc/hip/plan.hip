@@ -902,9 +902,9 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             nf.setup(th, n, ms, mt, mu, T.mode_ijk, T.mode_w, std::max(4, std::min(14, n_digits + 2)));
             for (int i = 0; i < n; ++i) fidx[i] = nf.position[tu[i]];
         } else {
-            // at most 512 point blocks: each writes a partial sum per mode that the reduction
-            // reads back (2048 blocks at N = 2e5, 6 digits, made 95 MB of partial sums per call)
-            ff.setup(th, n, ms, mt, mu, T.mode_ijk, T.mode_w, nullptr, 512);
+            // at most 1024 point blocks (N = 2.5e5, 6 digits, kernel alone: 512 108 us, 1024 93 us;
+            // the reduction 6 and 9 us)
+            ff.setup(th, n, T.mode_ijk, T.mode_w, nullptr, 1024);
         }
         far_idx.upload(fidx);
         if (qp) {
@@ -1485,7 +1485,7 @@ bool Plan<Real>::many_ensure() {
     many_vc_far = far_nufft ? 0 : (int)std::max<size_t>(1, std::min<size_t>(VC, (size_t(128) << 20) / std::max<size_t>(1, sp_v)));
     const size_t pass = 2 * ((size_t)nsall * VC * sizeof(float) + (size_t)n * VC * (sizeof(float) + sizeof(double)));
     const size_t total = pass + chain_v * many_vc_chain + (size_t)n * VC * sizeof(Real) +
-                         (far_nufft ? 0 : sp_v * many_vc_far + sizeof(double2) * ff.s_elems() * VC);
+                         (far_nufft ? 0 : sp_v * many_vc_far + sizeof(double) * ff.s_elems() * VC);
     size_t free_b = 0, total_b = 0;
     check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     if (pw_by_level || total > free_b / 4) {
@@ -1507,7 +1507,7 @@ bool Plan<Real>::many_ensure() {
     many_pot.alloc((size_t)n * VC * sizeof(Real));
     if (!far_nufft) {
         many_sp.alloc(sp_v * many_vc_far);
-        many_s.alloc(sizeof(double2) * ff.s_elems() * VC);
+        many_s.alloc(sizeof(double) * ff.s_elems() * VC);
         check(hipMemset(many_s.p, 0, many_s.bytes), "hipMemset");  // padding of the weighted sums stays zero
     }
     for (auto &e : many_ev) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -1574,7 +1574,7 @@ void Plan<Real>::evaluate_many(int n_vec, const double *d_Q, Real *d_P, hipStrea
             if (far_nufft) {
                 for (int c = 0; c < vc; ++c) nf.run(Q0 + (size_t)c * n, far0 + (size_t)c * n, s_far);
             } else {
-                ff.run_many(Q0, n, vc, far0, n, many_sp.as<double2>(), many_vc_far, many_s.as<double2>(), s_far);
+                ff.run_many(Q0, n, vc, far0, n, many_sp.as<double2>(), many_vc_far, many_s.as<double>(), s_far);
             }
             check(hipEventRecord(e_fr[b], s_far), "hipEventRecord");
             // the chain on s, many_vc_chain vectors per launch, charges from the gathered copy
@@ -1792,12 +1792,9 @@ void Plan<Real>::evaluate_complex_host(const double *q, Real *out) {
     check(hipStreamSynchronize(stream), "hipStreamSynchronize");
 }
 
-void FourierSum::setup(const std::vector<double> &theta_host, int n_points, int ms_, int mt_, int mu_,
-                       const std::vector<int> &M, const std::vector<double> &mode_w, Arena *arena, int max_blocks) {
+void FourierSum::setup(const std::vector<double> &theta_host, int n_points, const std::vector<int> &M,
+                       const std::vector<double> &mode_w, Arena *arena, int max_blocks) {
     n = n_points;
-    ms = ms_;
-    mt = mt_;
-    mu = mu_;
     n_modes = (int)mode_w.size();
     // an array in its owned buffer, or in a slice of the arena
     auto put = [&](DevBuf &own, const auto &v) {
@@ -1808,59 +1805,65 @@ void FourierSum::setup(const std::vector<double> &theta_host, int n_points, int 
     };
     theta_d = put(theta, theta_host);
     w_d = put(w, mode_w);
-    // lines of constant (j, k) and consecutive i, cut into chunks of FF_CHUNK modes
-    std::vector<int> cijk, cm0, clen, ljk, li, lptr;
+    // lines of constant (j, k) and consecutive i, sorted by their largest |i| (descending, so
+    // that the 16 lines of a tile need about the same number of columns)
+    struct Line { int j, k, lo, hi, m0, imax; };
+    std::vector<Line> ls;
+    dim_i = dim_j = dim_k = 0;
     for (int m = 0; m < n_modes;) {
         int e = m + 1;
         while (e < n_modes && M[3 * e + 1] == M[3 * m + 1] && M[3 * e + 2] == M[3 * m + 2] && M[3 * e] == M[3 * (e - 1)] + 1)
             ++e;
-        ljk.push_back(M[3 * m + 1]);
-        ljk.push_back(M[3 * m + 2]);
-        li.push_back(M[3 * m]);
-        li.push_back(M[3 * (e - 1)]);
-        lptr.push_back(m);
-        for (int c = m; c < e; c += FF_CHUNK) {
-            cijk.push_back(M[3 * c]);
-            cijk.push_back(M[3 * c + 1]);
-            cijk.push_back(M[3 * c + 2]);
-            cm0.push_back(c);
-            clen.push_back(std::min(FF_CHUNK, e - c));
-        }
+        const int lo = M[3 * m], hi = M[3 * (e - 1)];
+        ls.push_back({M[3 * m + 1], M[3 * m + 2], lo, hi, m, std::max(std::abs(lo), std::abs(hi))});
+        dim_i = std::max(dim_i, ls.back().imax);
+        dim_j = std::max(dim_j, std::abs(ls.back().j));
+        dim_k = std::max(dim_k, std::abs(ls.back().k));
         m = e;
     }
-    n_lines = (int)lptr.size();
-    n_chunks = (int)cm0.size();
-    chunk_ijk_d = put(chunk_ijk, cijk);
-    chunk_m0_d = put(chunk_m0, cm0);
-    chunk_len_d = put(chunk_len, clen);
-    // weighted structure factors per line, padded at the high-i end to a multiple of
-    // FF_QUAD modes (zeros), so the evaluation reads them FF_QUAD at a time
+    std::stable_sort(ls.begin(), ls.end(), [](const Line &a, const Line &b) { return a.imax > b.imax; });
+    while (ls.size() % 16) ls.push_back({0, 0, 1, 0, 0, 0});  // no modes
+    n_lt = (int)ls.size() / 16;
     std::vector<int4> lv;
-    std::vector<int> lbase, pix(n_modes);
-    int npad = 0;
-    for (size_t L = 0; L < lptr.size(); ++L) {
-        const int len = li[2 * L + 1] - li[2 * L] + 1, nq = (len + FF_QUAD - 1) / FF_QUAD;
-        lv.push_back(make_int4(ljk[2 * L], ljk[2 * L + 1], li[2 * L], nq));
-        lbase.push_back(npad);
-        for (int r = 0; r < len; ++r) pix[lptr[L] + r] = npad + r;
-        npad += nq * FF_QUAD;
+    std::vector<int> lm;
+    std::vector<int2> iv, uv;
+    int g_len = 0;
+    for (const Line &l : ls) {
+        lv.push_back(make_int4(l.j, l.k, l.lo, l.hi));
+        lm.push_back(l.m0);
     }
+    for (int t = 0; t < n_lt; ++t) {
+        const int imax = ls[16 * t].imax;
+        iv.push_back(make_int2(imax, g_len));
+        g_len += (imax + 2) / 2 * 128;
+        for (int c = 0; 16 * c < 2 * (imax + 1); ++c) uv.push_back(make_int2(t, c));
+    }
+    n_units = (int)uv.size();
     lines_d = put(lines, lv);
-    line_base_d = put(line_base, lbase);
-    pidx_d = put(pidx, pix);
-    blocks = std::max(1, std::min(std::min(2048, max_blocks), (n + FF_TP - 1) / FF_TP));
-    const size_t sp_n = (size_t)blocks * std::max(1, n_modes), s_n = (size_t)std::max(1, npad);
-    s_len = s_n;
+    line_m0_d = put(line_m0, lm);
+    info_d = put(info, iv);
+    units_d = put(units, uv);
+    // points per LDS tile: 32, or 16 where many modes per axis make the tables large
+    const FfDims dims{dim_i, dim_j, dim_k};
+    tp = dims.lds_bytes(32) <= 65536 ? 32 : 16;
+    // workgroup columns: each writes a partial sum per mode that the reduction reads back.  A
+    // quarter of the tiles (at least 256) keeps that traffic down where a launch is small or has
+    // many vectors (N = 2e4, one column per tile: 0.5 GB of partial sums per 32 vectors), and
+    // no more than about 2048 workgroups in all (at least 64 columns) are of use
+    const int gy = std::max(1, (n_units + FF_UNITS - 1) / FF_UNITS), tiles = (n + tp - 1) / tp;
+    blocks = std::max(1, std::min({max_blocks, tiles, std::max(256, tiles / 4), std::max(64, 2048 / gy)}));
+    const size_t sp_n = (size_t)blocks * std::max(1, n_modes);
+    s_len = (size_t)g_len + 128;  // the evaluation loads one step ahead
     if (arena) {
         Sp_d = arena->take_n<double2>(sp_n);
-        S_d = arena->take_n<double2>(s_n);
+        S_d = arena->take_n<double>(s_len);
     } else {
         Sp.alloc(sizeof(double2) * sp_n);
-        S.alloc(sizeof(double2) * s_n);
+        S.alloc(sizeof(double) * s_len);
         Sp_d = Sp.as<double2>();
-        S_d = S.as<double2>();
+        S_d = S.as<double>();
     }
-    if (S_d) check(hipMemset(S_d, 0, sizeof(double2) * s_n), "hipMemset");  // padding stays zero
+    if (S_d) check(hipMemset(S_d, 0, sizeof(double) * s_len), "hipMemset");  // padding columns stay zero
 }
 
 void FourierSum::run(const double *d_q, double *d_out, hipStream_t s) const {
@@ -1874,44 +1877,68 @@ void FourierSum::run_at(const double *d_q, const double *d_theta_eval, int n_eva
         check(hipGetLastError(), "k_fill far");
         return;
     }
-    const size_t lds = sizeof(double2) * FF_TP * (ms + mt + mu + 1) + sizeof(double) * FF_TP;
-    dim3 grid(blocks, (n_chunks + 255) / 256);
-    hipLaunchKernelGGL(k_ff_structure<1>, grid, dim3(256), lds, s, theta_d, d_q, n, ms, mt, mu, chunk_ijk_d, chunk_m0_d,
-                       chunk_len_d, n_chunks, n_modes, Sp_d, 0ll, 0ll, 1);
-    check(hipGetLastError(), "k_ff_structure");
-    hipLaunchKernelGGL(k_ff_reduce, dim3((n_modes + 31) / 32), dim3(256), 0, s, Sp_d, blocks, w_d, pidx_d, n_modes, S_d);
+    structure(d_q, 0, 1, Sp_d, S_d, s);
+    eval(d_theta_eval, n_eval, 1, S_d, d_out, 0, s);
+}
+
+// nv vectors along z: partial sums into sp, the weighted sums into g
+void FourierSum::structure(const double *d_q, long long ldq, int nv, double2 *sp, double *g, hipStream_t s) const {
+    const FfDims dims{dim_i, dim_j, dim_k};
+    const long long vs_sp = nv > 1 ? (long long)sp_elems() : 0, vs_g = nv > 1 ? (long long)s_len : 0;
+    // every wave the same count of units: the fewest workgroup rows of at most FF_UNITS, evenly
+    const int gy = (n_units + FF_UNITS - 1) / FF_UNITS;
+    auto go = [&](auto uu) {
+        constexpr int U = decltype(uu)::value;
+        auto launch = [&](auto vv) {
+            constexpr int V = decltype(vv)::value;
+            hipLaunchKernelGGL((k_ff_structure<U, V>), dim3(blocks, (n_units + 4 * U - 1) / (4 * U), (nv + V - 1) / V),
+                               dim3(256), dims.lds_bytes(tp), s, theta_d, d_q, n, tp, dims, lines_d, line_m0_d, units_d,
+                               n_units, n_modes, sp, ldq, vs_sp, nv);
+        };
+        if (nv == 1) launch(std::integral_constant<int, 1>{});
+        else launch(std::integral_constant<int, FF_MANY>{});
+        check(hipGetLastError(), "k_ff_structure");
+    };
+    switch ((n_units + 4 * gy - 1) / (4 * gy)) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    default: go(std::integral_constant<int, 4>{}); break;
+    }
+    hipLaunchKernelGGL(k_ff_reduce, dim3(16 * n_lt, 1, nv), dim3(512), sizeof(double2) * (512 + 2 * dim_i + 1), s, sp, blocks,
+                       w_d, lines_d, line_m0_d, info_d, n_modes, g, vs_sp, vs_g);
     check(hipGetLastError(), "k_ff_reduce");
-    hipLaunchKernelGGL(k_ff_eval<1>, dim3((n_eval + 255) / 256), dim3(256), 0, s, d_theta_eval, n_eval, lines_d,
-                       line_base_d, n_lines, S_d, d_out, 0ll, 0ll, 1);
+}
+
+void FourierSum::eval(const double *d_theta_eval, int n_eval, int nv, const double *g, double *d_out, long long ldo,
+                      hipStream_t s) const {
+    const FfDims dims{dim_i, dim_j, dim_k};
+    auto go = [&](auto rt, auto vv) {
+        constexpr int RT = decltype(rt)::value, V = decltype(vv)::value;
+        hipLaunchKernelGGL((k_ff_eval<RT, V>), dim3((n_eval + 16 * RT - 1) / (16 * RT), 1, (nv + V - 1) / V), dim3(256),
+                           dims.lds_bytes(16 * RT), s, d_theta_eval, n_eval, dims, lines_d, info_d, n_lt, g, d_out,
+                           (long long)s_len, ldo, nv);
+    };
+    auto by_rt = [&](auto vv) {
+        if (tp == 32) go(std::integral_constant<int, 2>{}, vv);
+        else go(std::integral_constant<int, 1>{}, vv);
+    };
+    if (nv == 1) by_rt(std::integral_constant<int, 1>{});
+    else by_rt(std::integral_constant<int, FF_MANY>{});
     check(hipGetLastError(), "k_ff_eval");
 }
 
 void FourierSum::run_many(const double *d_Q, long long ldq, int nv, double *d_out, long long ldo, double2 *Sp_many,
-                          int vc, double2 *S_many, hipStream_t s) const {
+                          int vc, double *S_many, hipStream_t s) const {
     if (nv <= 0 || n <= 0) return;
     if (n_modes == 0) {
         for (int v = 0; v < nv; ++v) run(d_Q + v * ldq, d_out + v * ldo, s);
         return;
     }
     if (vc < 1 || vc > 65535 || nv > 65535) throw std::invalid_argument("FourierSum::run_many: vector count");
-    constexpr int VS = FF_MANY_S, VE = FF_MANY_E;
-    const size_t lds = sizeof(double2) * FF_TP * (ms + mt + mu + 1) + sizeof(double) * FF_TP * VS;
-    const long long spv = (long long)sp_elems(), sv = (long long)s_len;
-    // the sums of run() per vector, VS (VE) vectors per workgroup of the structure factors
-    // (evaluation) along z
-    for (int v0 = 0; v0 < nv; v0 += vc) {
-        const int c = std::min(vc, nv - v0);
-        hipLaunchKernelGGL(k_ff_structure<VS>, dim3(blocks, (n_chunks + 255) / 256, (c + VS - 1) / VS), dim3(256), lds,
-                           s, theta_d, d_Q + v0 * ldq, n, ms, mt, mu, chunk_ijk_d, chunk_m0_d, chunk_len_d, n_chunks,
-                           n_modes, Sp_many, (long long)ldq, spv, c);
-        check(hipGetLastError(), "k_ff_structure");
-        hipLaunchKernelGGL(k_ff_reduce, dim3((n_modes + 31) / 32, 1, c), dim3(256), 0, s, Sp_many, blocks, w_d, pidx_d,
-                           n_modes, S_many + v0 * sv, spv, sv);
-        check(hipGetLastError(), "k_ff_reduce");
-    }
-    hipLaunchKernelGGL(k_ff_eval<VE>, dim3((n + 255) / 256, 1, (nv + VE - 1) / VE), dim3(256), 0, s, theta_d, n,
-                       lines_d, line_base_d, n_lines, S_many, d_out, sv, (long long)ldo, nv);
-    check(hipGetLastError(), "k_ff_eval");
+    for (int v0 = 0; v0 < nv; v0 += vc)
+        structure(d_Q + v0 * ldq, ldq, std::min(vc, nv - v0), Sp_many, S_many + (size_t)v0 * s_len, s);
+    eval(theta_d, n, nv, S_many, d_out, ldo, s);
 }
 
 void NufftFarField::setup(const std::vector<double> &theta_host, int n_points, int ms_, int mt_, int mu_,

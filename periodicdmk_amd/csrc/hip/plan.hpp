@@ -70,33 +70,39 @@ struct Work {
 // Truncated lattice Fourier sum in FP64:
 //   out[u] = sum_{m in the half space} Re( w_m S(m) e^{+i m.theta_u} ),  S(m) = sum_u q_u e^{-i m.theta_u},
 // theta = 2 pi x (fractional coordinates, wrapped to [0, 1)).  Modes (i, j, k) come in lines
-// of constant (j, k) with consecutive i; index ranges are [-m/2, (m-1)/2] for m = ms, mt, mu.
+// of constant (j, k) with consecutive i, taken 16 lines at a time (k_ff_structure).
 // Its arrays are owned buffers, or slices of an Arena when setup() is given one.  The
 // structure factors are summed in `blocks` partial sums of point tiles (at most max_blocks),
 // then added in block order.
 struct FourierSum {
-    int n = 0, ms = 0, mt = 0, mu = 0, n_modes = 0, n_chunks = 0, n_lines = 0, blocks = 0;
-    DevBuf theta, w, chunk_ijk, chunk_m0, chunk_len, lines, line_base, pidx, Sp, S;
+    int n = 0, n_modes = 0, n_lt = 0, n_units = 0, blocks = 0, tp = 32;
+    int dim_i = 0, dim_j = 0, dim_k = 0;  // largest |i|, |j|, |k|
+    DevBuf theta, w, lines, line_m0, info, units, Sp, S;
     const double *theta_d = nullptr, *w_d = nullptr;
-    const int *chunk_ijk_d = nullptr, *chunk_m0_d = nullptr, *chunk_len_d = nullptr, *line_base_d = nullptr,
-              *pidx_d = nullptr;
     const int4 *lines_d = nullptr;
-    double2 *Sp_d = nullptr, *S_d = nullptr;
-    void setup(const std::vector<double> &theta_host, int n_points, int ms_, int mt_, int mu_,
-               const std::vector<int> &mode_ijk, const std::vector<double> &mode_w, Arena *arena = nullptr,
-               int max_blocks = 2048);
+    const int *line_m0_d = nullptr;
+    const int2 *info_d = nullptr, *units_d = nullptr;
+    double2 *Sp_d = nullptr;
+    double *S_d = nullptr;
+    void setup(const std::vector<double> &theta_host, int n_points, const std::vector<int> &mode_ijk,
+               const std::vector<double> &mode_w, Arena *arena = nullptr, int max_blocks = 2048);
     void run(const double *d_q, double *d_out, hipStream_t s) const;  // enqueue only
     // S(m) from the setup points, then out[t] at n_eval other points (theta_eval[3t + d],
     // device, same convention); enqueue only
     void run_at(const double *d_q, const double *d_theta_eval, int n_eval, double *d_out, hipStream_t s) const;
     // run() for nv vectors (charges d_Q + v ldq, output d_out + v ldo), each equal to run() on
     // it: partial sums of vc vectors per launch in Sp_many (vc * sp_elems()), the weighted
-    // sums of all nv in S_many (nv * s_elems(), padding zero), one evaluation launch
+    // sums of all nv in S_many (nv * s_elems() doubles, padding zero), one evaluation launch
     void run_many(const double *d_Q, long long ldq, int nv, double *d_out, long long ldo, double2 *Sp_many, int vc,
-                  double2 *S_many, hipStream_t s) const;
+                  double *S_many, hipStream_t s) const;
     size_t sp_elems() const { return (size_t)blocks * (size_t)std::max(1, n_modes); }
     size_t s_elems() const { return s_len; }
     size_t s_len = 1;
+
+private:
+    void structure(const double *d_q, long long ldq, int nv, double2 *sp, double *g, hipStream_t s) const;
+    void eval(const double *d_theta_eval, int n_eval, int nv, const double *g, double *d_out, long long ldo,
+              hipStream_t s) const;
 };
 
 // The same Fourier sum by a non-uniform FFT (spreading with an exponential-of-semicircle
