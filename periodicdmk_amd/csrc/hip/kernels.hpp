@@ -1871,26 +1871,30 @@ __device__ __forceinline__ T nf_load_u32(const B *base, unsigned off) {
 
 // PASS 0: steps of row g in the k-th entry of item i -> cnt[(ie_base[i] + k) * 16 + g], and the
 // in-support pairs added to *pairs.  PASS 1: the source indices into the row blocks from
-// steps + wave_base[i] (the item's K, as built on the host, in items[i].w).
+// steps + wave_base[i] (the item's K, as built on the host, in items[i].w).  With parts
+// (PASS 1) items come in n_parts parts each: wavefront p of item i writes the lists of entries
+// parts[p' ].x .. parts[p'].y - 1, p' = i n_parts + p, from wave_base[p'].
 template <class R, int PASS>
 __global__ __launch_bounds__(256) void k_near_rows_build(
     const P4<R> *__restrict__ src, const P4<R> *__restrict__ trg, const int4 *__restrict__ items,
     const P4<R> *__restrict__ wbox, const int *__restrict__ l1_ptr, const NfEntry *__restrict__ l1,
     const P4<R> *__restrict__ geom, const P4<R> *__restrict__ cbox, const int *__restrict__ ie_base,
     int *__restrict__ cnt, const long long *__restrict__ wave_base, int *__restrict__ steps,
-    unsigned long long *__restrict__ pairs, int n_items) {
-    const int item = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (item >= n_items) return;  // whole wavefront
+    unsigned long long *__restrict__ pairs, int n_items, const int2 *__restrict__ parts = nullptr, int n_parts = 1) {
+    const int wave = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wave >= n_items * n_parts) return;  // whole wavefront
+    const int item = wave / n_parts;
     const int lane = threadIdx.x & 63;
     const int4 it = items[item];
     const bool active = lane < it.y;
     const P4<R> me = active ? trg[it.x + lane] : P4<R>{R(1e18), R(1e18), R(1e18), R(0)};
     const P4<R> blo = wbox[2 * item], bhi = wbox[2 * item + 1];
     const int eb = l1_ptr[it.z], base = ie_base[item];
-    int *out = PASS == 1 ? steps + wave_base[item] + lane : nullptr;
+    int *out = PASS == 1 ? steps + wave_base[wave] + lane : nullptr;
     unsigned long long np = 0;
     int k_row = 0;  // steps of this lane's row so far (the same in the row's 4 lanes)
-    for (int e = eb; e < l1_ptr[it.z + 1]; ++e) {
+    const int e_first = parts ? eb + parts[wave].x : eb, e_last = parts ? eb + parts[wave].y : l1_ptr[it.z + 1];
+    for (int e = e_first; e < e_last; ++e) {
         const NfEntry E = l1[e];
         const P4<R> gm = geom[e];
         const R bs = gm.w, d2max = bs * bs;
@@ -1944,7 +1948,12 @@ __global__ __launch_bounds__(256) void k_near_rows_build(
 // (end step << 16) | byte offset of the entry's geometry from the LDS base (end steps below
 // 2^16, and the workgroup's LDS below 64 KiB, both checked on the host; the terminator's end
 // is clamped to 2^16 - 1, past every step).
-template <int NC>
+// S > 1: trees with few items (N = 1e4: 192 wavefronts for 1024 SIMDs, each a serial walk of
+// 1300 steps, 174 us).  A workgroup of S waves takes one item, each wave the row lists of its
+// share of the list1 entries (items[item S + wave]); the entries' sums meet in LDS and are
+// added in entry order, so the potentials are those of S = 1 bit for bit (73 us with S = 8;
+// near_parts() has the other sizes).
+template <int NC, int S>
 __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict__ src, const P4<float> *__restrict__ trg,
                                                    const int4 *__restrict__ items, const int *__restrict__ l1_ptr,
                                                    const P4<float> *__restrict__ geom, const int *__restrict__ rs_base,
@@ -1953,14 +1962,21 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
                                                    float *__restrict__ pot_sorted, int item0, int item1, int ne_max) {
     extern __shared__ float4 nf_lds[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
-    if (item >= item1) return;  // whole wavefront (no workgroup barrier below)
+    const int item = S > 1 ? (int)blockIdx.x * S + w
+                           : item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
+    if (S == 1 && item >= item1) return;  // whole wavefront (no workgroup barrier below)
     const int lane = threadIdx.x & 63, g = lane >> 2;
     const int4 it = items[item];  // (first target, count, target-leaf list index, K)
     // this wavefront's LDS: ne_max + 1 entries x (offset+bs, consts), then (ne_max + 1) x 16 slots
     float4 *geo = nf_lds + (size_t)w * (ne_max + 1) * 6;
     int *slots = reinterpret_cast<int *>(geo + 2 * (ne_max + 1));
     const int eb = l1_ptr[it.z], ne = l1_ptr[it.z + 1] - eb;
+    // S > 1: the entries' sums [ne + 1][64]
+    float *sums = reinterpret_cast<float *>(nf_lds + (size_t)S * (ne_max + 1) * 6);
+    if (S > 1) {
+        for (int k = threadIdx.x; k < ne * 64; k += 64 * S) sums[k] = 0;
+        __syncthreads();
+    }
     for (int e = lane; e <= ne; e += 64) {
         const P4<float> gm = e < ne ? geom[eb + e] : P4<float>{0.0f, 0.0f, 0.0f, 0.0f};
         const float bs = gm.w;
@@ -1968,8 +1984,9 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
         geo[2 * e + 1] = make_float4(e < ne ? 2.0f / bs : 0.0f, -bs / 2.0f, 0.0f, 0.0f);
     }
     const int *rs = rslot + (size_t)rs_base[item] * NF_ROWS;
+    const int n_slots = S > 1 ? rs_base[item + 1] - rs_base[item] : ne + 1;
     const unsigned geo_off = (unsigned)((const char *)geo - (const char *)nf_lds);
-    for (int k = lane; k < (ne + 1) * NF_ROWS; k += 64) {
+    for (int k = lane; k < n_slots * NF_ROWS; k += 64) {
         const int v = rs[k];
         slots[k] = (int)(((unsigned)min(v >> 8, 0xffff) << 16) | (geo_off + 32u * (unsigned)(v & 255)));
     }
@@ -1991,12 +2008,15 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     const int *slot = slots + g;  // the row's next slot
     double acc = 0;
     float ea = 0;
+    float *sum = sums + (size_t)ne * 64 + lane;  // the current entry's (row ne: none)
     auto enter = [&]() {  // the row's next non-empty entry (or the terminator)
-        acc += (double)ea;
+        if (S > 1) *sum = ea;
+        else acc += (double)ea;
         ea = 0;
         const unsigned v = (unsigned)*slot;
         slot += NF_ROWS;
         end = (int)(v >> 16);
+        if (S > 1) sum = sums + ((v & 0xffffu) - geo_off) * 2 + lane;  // 32 bytes of geometry, 64 sums
         const float4 *ge = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(nf_lds) + (v & 0xffffu));
         const float4 a = ge[0], b = ge[1];
         tx = me.x + a.x;
@@ -2071,7 +2091,14 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
         block(pb, mb, 4 * b + 4);
     }
     if (b < nb) block(pa, ma, 4 * b);
-    acc += (double)ea;
+    if (S > 1) {
+        *sum = ea;
+        __syncthreads();
+        if (w > 0) return;
+        for (int e = 0; e < ne; ++e) acc += (double)sums[e * 64 + lane];
+    } else {
+        acc += (double)ea;
+    }
     if (active) pot_sorted[it.x + lane] += (float)acc;
 }
 
@@ -2254,7 +2281,7 @@ __host__ __device__ inline size_t near_rows64_lds_per_wave(int ne_max) {
     return 64 * 2 * sizeof(double2) + (size_t)(ne_max + 1) * 3 * sizeof(double2) + (size_t)(ne_max + 1) * NF_ROWS * 4;
 }
 
-template <int NC>
+template <int NC, int S>
 __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restrict__ src,
                                                       const P4<double> *__restrict__ trg,
                                                       const int4 *__restrict__ items, const int *__restrict__ l1_ptr,
@@ -2265,14 +2292,21 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
                                                       double *__restrict__ pot_sorted, int item0, int item1, int ne_max) {
     extern __shared__ double2 nf_lds64[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
-    if (item >= item1) return;  // whole wavefront (no workgroup barrier below)
+    const int item = S > 1 ? (int)blockIdx.x * S + w
+                           : item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
+    if (S == 1 && item >= item1) return;  // whole wavefront (no workgroup barrier below)
     const int lane = threadIdx.x & 63, g = lane >> 2;
     const int4 it = items[item];  // (first target, count, target-leaf list index, K)
     double2 *pts = reinterpret_cast<double2 *>(reinterpret_cast<char *>(nf_lds64) + (size_t)w * near_rows64_lds_per_wave(ne_max));
     double2 *geo = pts + 128;
     int *slots = reinterpret_cast<int *>(geo + 3 * (ne_max + 1));
     const int eb = l1_ptr[it.z], ne = l1_ptr[it.z + 1] - eb;
+    // S > 1: the entries' sums [ne + 1][64]
+    double *sums = reinterpret_cast<double *>(reinterpret_cast<char *>(nf_lds64) + (size_t)S * near_rows64_lds_per_wave(ne_max));
+    if (S > 1) {
+        for (int k = threadIdx.x; k < ne * 64; k += 64 * S) sums[k] = 0;
+        __syncthreads();
+    }
     for (int e = lane; e <= ne; e += 64) {
         const P4<double> gm = e < ne ? geom[eb + e] : P4<double>{0.0, 0.0, 0.0, 0.0};
         const double bs = gm.w;
@@ -2282,7 +2316,8 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
     }
     const int *rs = rslot + (size_t)rs_base[item] * NF_ROWS;
     const unsigned geo_off = (unsigned)((const char *)geo - (const char *)nf_lds64);
-    for (int k = lane; k < (ne + 1) * NF_ROWS; k += 64) {
+    const int n_slots = S > 1 ? rs_base[item + 1] - rs_base[item] : ne + 1;
+    for (int k = lane; k < n_slots * NF_ROWS; k += 64) {
         const int v = rs[k];
         slots[k] = (int)(((unsigned)min(v >> 8, 0xffff) << 16) | (geo_off + 48u * (unsigned)(v & 255)));
     }
@@ -2299,12 +2334,15 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
     int end = 0;
     const int *slot = slots + g;  // the row's next slot
     double acc = 0, ea = 0;
+    double *sum = sums + (size_t)ne * 64 + lane;  // the current entry's (row ne: none)
     auto enter = [&]() {  // the row's next non-empty entry (or the terminator)
-        acc += ea;
+        if (S > 1) *sum = ea;
+        else acc += ea;
         ea = 0;
         const unsigned v = (unsigned)*slot;
         slot += NF_ROWS;
         end = (int)(v >> 16);
+        if (S > 1) sum = sums + ((v & 0xffffu) - geo_off) / 48u * 64u + lane;
         const double2 *ge = reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(nf_lds64) + (v & 0xffffu));
         const double2 a = ge[0], b = ge[1], cc = ge[2];
         tx = me.x + a.x;
@@ -2368,7 +2406,14 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
         block(pb, mb, 4 * b + 4);
     }
     if (b < nb) block(pa, ma, 4 * b);
-    acc += ea;
+    if (S > 1) {
+        *sum = ea;
+        __syncthreads();
+        if (w > 0) return;
+        for (int e = 0; e < ne; ++e) acc += sums[e * 64 + lane];
+    } else {
+        acc += ea;
+    }
     if (active) pot_sorted[it.x + lane] += acc;
 }
 

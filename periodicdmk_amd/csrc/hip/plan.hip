@@ -107,6 +107,29 @@ int log2_bucket(long long v) {
     return b;
 }
 
+// LDS of a row near-field workgroup of S waves that share one item (k_near_rows, k_near_rows64)
+template <class Real> size_t near_parts_lds(int S, int ne_max) {
+    const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(ne_max + 1) * 6 * 16
+                                                             : near_rows64_lds_per_wave(ne_max);
+    return S * per_wave + (size_t)(ne_max + 1) * 64 * sizeof(Real);
+}
+
+// Waves per item of the row near field.  Alone, 6 digits FP32 / FP64, one wave per item against
+// 4 and 8: 64 items (N = 1e3) 50 / 59 us, 40 / 43, 36 / 39; 192 items (1e4) 174 / 242 us,
+// 86 / 117, 73 / 96; 512 items (3e4) 152 / 212, 82 / 111, 75 / 110; 2048 items (1.2e5) 329 / 511,
+// 247 / 413, 258 / 453; 4096 items (2.5e5) 206 / 331, 224 / 500, -: one wave from 2560 items on,
+// 8 up to 256, within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or 8 forces a count).
+template <class Real> int near_parts(int n_items, int ne_max) {
+    int S = n_items <= 256 ? 8 : (n_items < 2560 ? 4 : 1);
+    if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
+        const int v = std::atoi(e);
+        S = v >= 8 ? 8 : (v >= 4 ? 4 : 1);
+    }
+    if (S == 8 && near_parts_lds<Real>(S, ne_max) > 65536) S = 4;
+    if (S == 4 && near_parts_lds<Real>(S, ne_max) > 65536) S = 1;
+    return S;
+}
+
 int nc_for_digits(int d) {
     static const int nc[] = {5, 5, 5, 6, 9, 11, 12, 15, 17, 18, 22, 23, 25};
     return nc[std::min(12, std::max(0, d))];
@@ -813,6 +836,10 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             size_t mem_free = 0, mem_total = 0;
             check(hipMemGetInfo(&mem_free, &mem_total), "hipMemGetInfo");
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
+            if (nf_rows) {
+                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max);
+                if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c);
+            }
         }
         if (n_nf_items > 0 && nf_rows) {
             nf_items.upload(itv);
@@ -833,6 +860,18 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                                nf_wave_base.as<long long>(), nf_row_steps.as<int>(), (unsigned long long *)nullptr,
                                n_nf_items);
             check(hipGetLastError(), "k_near_rows_build write");
+            if (nf_parts > 1) {
+                const int n_sub = n_nf_items * nf_parts;
+                hipLaunchKernelGGL(k_fill<int>, dim3((unsigned)((np_total + NF_ROW_PAD + 255) / 256)), dim3(256), 0, stream,
+                                   np_steps.as<int>(), sentinel, (int)(np_total + NF_ROW_PAD));
+                check(hipGetLastError(), "k_fill part steps");
+                hipLaunchKernelGGL((k_near_rows_build<Real, 1>), dim3((n_sub + 3) / 4), dim3(256), 0, stream,
+                                   src.as<P4<Real>>(), trg.as<P4<Real>>(), nf_items.as<int4>(), nf_wbox.as<P4<Real>>(),
+                                   nf_ptr.as<int>(), nf_l1.as<NfEntry>(), nf_geom.as<P4<Real>>(), nf_cbox.as<P4<Real>>(),
+                                   nf_ie_base.as<int>(), (int *)nullptr, np_wave_base.as<long long>(), np_steps.as<int>(),
+                                   (unsigned long long *)nullptr, n_nf_items, np_range.as<int2>(), nf_parts);
+                check(hipGetLastError(), "k_near_rows_build parts");
+            }
             work.nf_pairs_support = (double)np;
         }
         if (n_nf_items > 0 && !nf_rows) {
@@ -1043,6 +1082,75 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     }
     build_ms[0] = ms_since(t_start);
     guard.armed = false;
+}
+
+// Row lists of the items in nf_parts parts each: list1 entries in order, cut where the parts
+// hold about the same steps (rows summed); per part the rows' steps and slots as in the
+// undivided lists.  c: steps per (item, entry, row).
+template <typename Real>
+void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vector<int> &ptr, const std::vector<int> &ieb,
+                                  const std::vector<int> &c) {
+    const int S = nf_parts, n_sub = n_nf_items * S;
+    std::vector<int4> items(n_sub);
+    std::vector<int2> range(n_sub);
+    std::vector<int> rsb(n_sub + 1, 0);
+    std::vector<long long> wb(n_sub, 0);
+    host_parallel(n_nf_items, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            const int ne = ptr[itv[i].z + 1] - ptr[itv[i].z];
+            const int *ci = &c[(size_t)ieb[i] * NF_ROWS];
+            std::vector<long> cum(ne + 1, 0);
+            for (int e = 0; e < ne; ++e) {
+                long t = 0;
+                for (int g = 0; g < NF_ROWS; ++g) t += ci[(size_t)e * NF_ROWS + g];
+                cum[e + 1] = cum[e] + t;
+            }
+            for (int p = 0, e = 0; p < S; ++p) {
+                const int e0 = e;
+                const double stop = (double)cum[ne] * (p + 1) / S;
+                // the boundary nearest to an even share
+                while (e < ne && (p == S - 1 || 0.5 * ((double)cum[e] + (double)cum[e + 1]) <= stop)) ++e;
+                range[(size_t)i * S + p] = make_int2(e0, e);
+                int kmax = 0;
+                for (int g = 0; g < NF_ROWS; ++g) {
+                    int k = 0;
+                    for (int x = e0; x < e; ++x) k += ci[(size_t)x * NF_ROWS + g];
+                    kmax = std::max(kmax, k);
+                }
+                items[(size_t)i * S + p] = make_int4(itv[i].x, itv[i].y, itv[i].z, (kmax + 3) & ~3);
+            }
+        }
+    });
+    np_total = 0;
+    for (int k = 0; k < n_sub; ++k) {
+        rsb[k + 1] = rsb[k] + range[k].y - range[k].x + 1;
+        wb[k] = np_total;
+        np_total += (long long)items[k].w * NF_ROWS;
+    }
+    std::vector<int> slot((size_t)rsb[n_sub] * NF_ROWS);
+    host_parallel(n_nf_items, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            const int ne = ptr[itv[i].z + 1] - ptr[itv[i].z];
+            for (int k = i * S; k < (i + 1) * S; ++k) {
+                std::fill(slot.begin() + (size_t)rsb[k] * NF_ROWS, slot.begin() + (size_t)rsb[k + 1] * NF_ROWS,
+                          (0x7fffff << 8) | ne);
+                for (int g = 0; g < NF_ROWS; ++g)
+                    for (int e = range[k].x, sl = 0, n_st = 0; e < range[k].y; ++e) {
+                        const int ce = c[(size_t)(ieb[i] + e) * NF_ROWS + g];
+                        if (ce == 0) continue;
+                        n_st += ce;
+                        slot[(size_t)(rsb[k] + sl) * NF_ROWS + g] = (n_st << 8) | e;
+                        ++sl;
+                    }
+            }
+        }
+    });
+    np_items.upload(items);
+    np_range.upload(range);
+    np_rs_base.upload(rsb);
+    np_rslot.upload(slot);
+    np_wave_base.upload(wb);
+    np_steps.alloc(sizeof(int) * (size_t)(np_total + NF_ROW_PAD));
 }
 
 template <typename Real>
@@ -1308,45 +1416,61 @@ void launch_near(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1) {
     check(hipGetLastError(), "k_near_field");
 }
 
-// quad-row near field (FP32 plans built with row step lists)
+// row near field (plans built with row step lists): wpb items per workgroup, or nf_parts waves
+// per item
 template <class Real>
 void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1) {
-    if constexpr (std::is_same<Real, float>::value) {
-        if (i1 <= i0) return;
-        // (the LDS tables of a workgroup's wavefronts stay within 64 KiB)
-        const size_t per_wave = (size_t)(pl.nf_ne_max + 1) * 6 * sizeof(float4);
-        while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
-        const size_t lds = (size_t)wpb * per_wave;
-        hipLaunchKernelGGL((k_near_rows<12>), dim3((i1 - i0 + wpb - 1) / wpb), dim3(64 * wpb), lds, s,
-                           pl.src.template as<P4<float>>(), pl.trg.template as<P4<float>>(),
-                           pl.nf_items.template as<int4>(), pl.nf_ptr.template as<int>(),
-                           pl.nf_geom.template as<P4<float>>(), pl.nf_rs_base.template as<int>(),
-                           pl.nf_rslot.template as<int>(), pl.nf_wave_base.template as<long long>(),
-                           pl.nf_row_steps.template as<int>(), pl.coeffs.template as<float>(),
-                           pl.pot_near.template as<float>(), i0, i1, pl.nf_ne_max);
-        check(hipGetLastError(), "k_near_rows");
-    } else {
-        if (i1 <= i0) return;
-        const size_t per_wave = near_rows64_lds_per_wave(pl.nf_ne_max);
-        while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
-        const size_t lds = (size_t)wpb * per_wave;
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((i1 - i0 + wpb - 1) / wpb), dim3(64 * wpb), lds, s,
-                               pl.src.template as<P4<double>>(), pl.trg.template as<P4<double>>(),
+    if (i1 <= i0) return;
+    const int S = pl.nf_parts;
+    const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(pl.nf_ne_max + 1) * 6 * sizeof(float4)
+                                                             : near_rows64_lds_per_wave(pl.nf_ne_max);
+    // (the LDS tables of a workgroup's wavefronts stay within 64 KiB)
+    while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
+    auto go = [&](auto kern) {
+        if (S > 1)
+            hipLaunchKernelGGL(kern, dim3(i1 - i0), dim3(64 * S), near_parts_lds<Real>(S, pl.nf_ne_max), s,
+                               pl.src.template as<P4<Real>>(), pl.trg.template as<P4<Real>>(),
+                               pl.np_items.template as<int4>(), pl.nf_ptr.template as<int>(),
+                               pl.nf_geom.template as<P4<Real>>(), pl.np_rs_base.template as<int>(),
+                               pl.np_rslot.template as<int>(), pl.np_wave_base.template as<long long>(),
+                               pl.np_steps.template as<int>(), pl.coeffs.template as<Real>(),
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max);
+        else
+            hipLaunchKernelGGL(kern, dim3((i1 - i0 + wpb - 1) / wpb), dim3(64 * wpb), wpb * per_wave, s,
+                               pl.src.template as<P4<Real>>(), pl.trg.template as<P4<Real>>(),
                                pl.nf_items.template as<int4>(), pl.nf_ptr.template as<int>(),
-                               pl.nf_geom.template as<P4<double>>(), pl.nf_rs_base.template as<int>(),
+                               pl.nf_geom.template as<P4<Real>>(), pl.nf_rs_base.template as<int>(),
                                pl.nf_rslot.template as<int>(), pl.nf_wave_base.template as<long long>(),
-                               pl.nf_row_steps.template as<int>(), pl.coeffs.template as<double>(),
-                               pl.pot_near.template as<double>(), i0, i1, pl.nf_ne_max);
-        };
-        switch (pl.nc) {
-        case 12: go(k_near_rows64<12>); break;
-        case 18: go(k_near_rows64<18>); break;
-        case 25: go(k_near_rows64<25>); break;
-        default: throw std::logic_error("row near field: unsupported coefficient count");
+                               pl.nf_row_steps.template as<int>(), pl.coeffs.template as<Real>(),
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max);
+        check(hipGetLastError(), "k_near_rows");
+    };
+    auto by_parts = [&](auto nc) {
+        constexpr int NC = decltype(nc)::value;
+        if constexpr (std::is_same<Real, float>::value) {
+            switch (S) {
+            case 8: go(k_near_rows<NC, 8>); break;
+            case 4: go(k_near_rows<NC, 4>); break;
+            default: go(k_near_rows<NC, 1>); break;
+            }
+        } else {
+            switch (S) {
+            case 8: go(k_near_rows64<NC, 8>); break;
+            case 4: go(k_near_rows64<NC, 4>); break;
+            default: go(k_near_rows64<NC, 1>); break;
+            }
         }
-        check(hipGetLastError(), "k_near_rows64");
+    };
+    switch (pl.nc) {
+    case 12: by_parts(std::integral_constant<int, 12>{}); return;
+    case 18:
+        if constexpr (std::is_same<Real, double>::value) { by_parts(std::integral_constant<int, 18>{}); return; }
+        break;
+    case 25:
+        if constexpr (std::is_same<Real, double>::value) { by_parts(std::integral_constant<int, 25>{}); return; }
+        break;
     }
+    throw std::logic_error("row near field: unsupported coefficient count");
 }
 
 }  // namespace

@@ -211,6 +211,13 @@ struct Plan {
     bool nf_rows = false;
     int nf_ne_max = 0;  // most list1 entries of a target leaf
     DevBuf nf_rs_base, nf_rslot, nf_wave_base, nf_row_steps;
+    // few items: nf_parts > 1 waves per item, part p of item i at i nf_parts + p with its range
+    // of list1 entries (np_range), K (np_items[].w), slots and blocks as above
+    int nf_parts = 1;
+    long long np_total = 0;
+    DevBuf np_items, np_range, np_rs_base, np_rslot, np_wave_base, np_steps;
+    void build_near_parts(const std::vector<int4> &itv, const std::vector<int> &ptr, const std::vector<int> &ieb,
+                          const std::vector<int> &c);
     // far field: exact Fourier sum, or the NUFFT for large N x modes
     int far_nufft = 0;
     FourierSum ff;
