@@ -64,32 +64,63 @@ template <> __device__ __forceinline__ double rsqrt_full<double>(double x) {
 }
 
 // ------------------------------------------------------------------ O(N) stages
-// Charges of the sorted sources.  Quasi-periodic passes multiply each by the real (comp 0)
-// or imaginary (comp 1) part of its image phase e^{i b.R} (originals: phase 1).
+// Charges of the sorted sources.
 template <class R>
 __global__ void k_gather_charges(const double *__restrict__ q, const int *__restrict__ src_user, P4<R> *__restrict__ src,
-                                 int nsall, R *__restrict__ pot_sorted, R *__restrict__ pot_near, int n,
-                                 const double2 *__restrict__ phase, int comp) {
+                                 int nsall, R *__restrict__ pot_sorted, R *__restrict__ pot_near, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nsall) {
-        double v = q[src_user[i]];
-        if (phase) v *= comp == 0 ? phase[i].x : phase[i].y;
-        src[i].w = (R)v;
-    }
+    if (i < nsall) src[i].w = (R)q[src_user[i]];
     if (i < n) {
         pot_sorted[i] = R(0);
         pot_near[i] = R(0);
     }
 }
 
-// pot[stride u] = pot_sorted[i] - w0_i q_u + far[u], u = trg_user[i] (stride 2: one component
-// of an interleaved complex output).  Vector v = blockIdx.z of a many-vector launch uses the
+// Quasi-periodic trees: the charges times the real and the imaginary part of their image phase
+// e^{i b.R} (originals: phase 1), each in a copy of the sources (ld apart), and both
+// components' potentials cleared.
+template <class R>
+__global__ void k_gather_qp(const double *__restrict__ q, const int *__restrict__ src_user,
+                            const double2 *__restrict__ phase, P4<R> *__restrict__ src, long long ld, int nsall,
+                            R *__restrict__ pot_sorted, R *__restrict__ pot_near, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nsall) {
+        const double v = q[src_user[i]];
+        const double2 ph = phase[i];
+        src[i].w = (R)(v * ph.x);
+        src[ld + i].w = (R)(v * ph.y);
+    }
+    if (i < 2 * n) {
+        pot_sorted[i] = R(0);
+        pot_near[i] = R(0);
+    }
+}
+
+// out[2 u], out[2 u + 1] = Re, Im: the two components' chain and near-field potentials, the self
+// correction on the real one (the originals' charges are real), rounded to R, and the complex
+// far field added to that.
+template <class R>
+__global__ void k_finalize_qp(const R *__restrict__ pot_sorted, const R *__restrict__ pot_near, const double *__restrict__ w0,
+                              const int *__restrict__ trg_user, const double *__restrict__ q,
+                              const double2 *__restrict__ far, R *__restrict__ out, int n, int use_self, int use_far) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int u = trg_user[i];
+    double re = (double)pot_sorted[i] + (double)pot_near[i], im = (double)pot_sorted[n + i] + (double)pot_near[n + i];
+    if (use_self) re -= w0[i] * q[u];
+    double2 f = make_double2(0, 0);
+    if (use_far) f = far[u];
+    out[2 * (size_t)u] = (R)((double)(R)re + f.x);
+    out[2 * (size_t)u + 1] = (R)((double)(R)im + f.y);
+}
+
+// pot[u] = pot_sorted[i] - w0_i q_u + far[u], u = trg_user[i].  Vector v = blockIdx.z of a many-vector launch uses the
 // arrays offset by v times the vs_* element strides (all zero for one vector).
 template <class R>
 __global__ void k_finalize(const R *__restrict__ pot_sorted, const R *__restrict__ pot_near, const double *__restrict__ w0,
                            const int *__restrict__ trg_user, const double *__restrict__ q, const double *__restrict__ far,
                            const int *__restrict__ far_idx, R *__restrict__ pot, int n, int use_self, int use_far,
-                           int stride, long long vs_sorted = 0, long long vs_near = 0, long long vs_q = 0,
+                           long long vs_sorted = 0, long long vs_near = 0, long long vs_q = 0,
                            long long vs_far = 0, long long vs_pot = 0) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -103,7 +134,7 @@ __global__ void k_finalize(const R *__restrict__ pot_sorted, const R *__restrict
     double v = (double)pot_sorted[i] + (double)pot_near[i];
     if (use_self) v -= w0[i] * q[u];
     if (use_far) v += far[far_idx[i]];
-    pot[(size_t)stride * u] = (R)v;
+    pot[u] = (R)v;
 }
 
 // ------------------------------------------------------------------ upward pass
@@ -132,8 +163,9 @@ __global__ __launch_bounds__(C2pCfg<P>::threads) void k_charge2proxy(
     const P4<R> *__restrict__ src, const int *__restrict__ grp_slot, const R *__restrict__ grp_geom,
     const int *__restrict__ grp_rng, const int *__restrict__ rng_begin, const int *__restrict__ rng_count,
     const R *__restrict__ rng_off, R *__restrict__ proxy, const R *__restrict__ qv = nullptr, int qv_ld = 0,
-    long long vs_out = 0) {
+    long long vs_out = 0, long long vs_src = 0) {
     chain_priority();
+    src += (long long)blockIdx.z * vs_src;  // (vectors with copies of the sources of their own)
     constexpr int RB = C2pCfg<P>::RB, NB = C2pCfg<P>::NB, NT = C2pCfg<P>::threads;
     // many-vector launch: vector blockIdx.z takes its charges from qv[source * qv_ld + v]
     // (src[].w otherwise) and writes its own proxy array, vs_out elements further on
@@ -1719,7 +1751,10 @@ __global__ __launch_bounds__(1024) void k_near_field(const P4<R> *__restrict__ s
                                                      const NfEntry *__restrict__ l1, const P4<R> *__restrict__ geom,
                                                      const int *__restrict__ ie_base, const long long *__restrict__ ie_ptr,
                                                      const int *__restrict__ step_src, const R *__restrict__ coeffs,
-                                                     R *__restrict__ pot_sorted, int item0, int item1) {
+                                                     R *__restrict__ pot_sorted, int item0, int item1, long long vs_src = 0,
+                                                     long long vs_pot = 0) {
+    src += (long long)blockIdx.z * vs_src;  // component blockIdx.z of a quasi-periodic pass
+    pot_sorted += (long long)blockIdx.z * vs_pot;
     // wave index made wave-uniform explicitly, so everything derived from it lives in SGPRs
     const int item = item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) +
                      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1953,13 +1988,17 @@ __global__ __launch_bounds__(256) void k_near_rows_build(
 // share of the list1 entries (items[item S + wave]); the entries' sums meet in LDS and are
 // added in entry order, so the potentials are those of S = 1 bit for bit (73 us with S = 8;
 // near_parts() has the other sizes).
-template <int NC, int S>
+// V = 2 (quasi-periodic): the residual formed once for two charges, the second from the copy of
+// the sources vs_src further on (potentials vs_pot further on); each component's sums are those
+// of V = 1.  (N = 1e5, beside the chain: 404 us against 504 for the two components along z.)
+template <int NC, int S, int V>
 __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict__ src, const P4<float> *__restrict__ trg,
                                                    const int4 *__restrict__ items, const int *__restrict__ l1_ptr,
                                                    const P4<float> *__restrict__ geom, const int *__restrict__ rs_base,
                                                    const int *__restrict__ rslot, const long long *__restrict__ wave_base,
                                                    const int *__restrict__ steps, const float *__restrict__ coeffs,
-                                                   float *__restrict__ pot_sorted, int item0, int item1, int ne_max) {
+                                                   float *__restrict__ pot_sorted, int item0, int item1, int ne_max,
+                                                   long long vs_src = 0, long long vs_pot = 0) {
     extern __shared__ float4 nf_lds[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int item = S > 1 ? (int)blockIdx.x * S + w
@@ -1971,10 +2010,10 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     float4 *geo = nf_lds + (size_t)w * (ne_max + 1) * 6;
     int *slots = reinterpret_cast<int *>(geo + 2 * (ne_max + 1));
     const int eb = l1_ptr[it.z], ne = l1_ptr[it.z + 1] - eb;
-    // S > 1: the entries' sums [ne + 1][64]
+    // S > 1: the entries' sums [V][ne + 1][64]
     float *sums = reinterpret_cast<float *>(nf_lds + (size_t)S * (ne_max + 1) * 6);
     if (S > 1) {
-        for (int k = threadIdx.x; k < ne * 64; k += 64 * S) sums[k] = 0;
+        for (int k = threadIdx.x; k < V * (ne + 1) * 64; k += 64 * S) sums[k] = 0;
         __syncthreads();
     }
     for (int e = lane; e <= ne; e += 64) {
@@ -2006,13 +2045,21 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     float tx = 0, ty = 0, tz = 0, d2max = 0, rsc = 0, cen = 0;
     int end = 0;
     const int *slot = slots + g;  // the row's next slot
-    double acc = 0;
-    float ea = 0;
+    double acc[V];
+    float ea[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        acc[v] = 0;
+        ea[v] = 0;
+    }
     float *sum = sums + (size_t)ne * 64 + lane;  // the current entry's (row ne: none)
     auto enter = [&]() {  // the row's next non-empty entry (or the terminator)
-        if (S > 1) *sum = ea;
-        else acc += (double)ea;
-        ea = 0;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if (S > 1) sum[v * (ne + 1) * 64] = ea[v];
+            else acc[v] += (double)ea[v];
+            ea[v] = 0;
+        }
         const unsigned v = (unsigned)*slot;
         slot += NF_ROWS;
         end = (int)(v >> 16);
@@ -2033,8 +2080,10 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     const int *sb = steps + wave_base[item];
     auto index = [&](int b) { return nf_load_u32<int>(sb + (size_t)b * 64, (unsigned)lane * 4u); };
     auto point = [&](int id) { return nf_load_u32<P4<float>>(src, (unsigned)id * 16u); };
+    const P4<float> *src1 = src + vs_src;
+    auto charge1 = [&](int id) { return V > 1 ? nf_load_u32<float>(&src1->w, (unsigned)id * 16u) : 0.0f; };
     // m: ballot of the block's entry flags, bit 4 g + s = row g switches entries at step s
-    auto block = [&](const P4<float> &pc, unsigned long long m, int k) {
+    auto block = [&](const P4<float> &pc, float q1, unsigned long long m, int k) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             // rows reach their entries' ends at different steps; the wave-wide test is scalar
@@ -2063,12 +2112,16 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
                 for (int i = NC - 3; i >= 0; --i) p = fmaf(p, x, c[i]);
                 u = p * rinv;
             }
-            switch (s) {
-            case 0: fmac_quad1<0>(ea, pc.w, u); break;
-            case 1: fmac_quad1<1>(ea, pc.w, u); break;
-            case 2: fmac_quad1<2>(ea, pc.w, u); break;
-            default: fmac_quad1<3>(ea, pc.w, u); break;
-            }
+            auto add = [&](float &e, float q) {
+                switch (s) {
+                case 0: fmac_quad1<0>(e, q, u); break;
+                case 1: fmac_quad1<1>(e, q, u); break;
+                case 2: fmac_quad1<2>(e, q, u); break;
+                default: fmac_quad1<3>(e, q, u); break;
+                }
+            };
+            add(ea[0], pc.w);
+            if (V > 1) add(ea[V - 1], q1);
         }
     };
     // two blocks per iteration, each block's point loaded one block ahead and its index two
@@ -2078,28 +2131,35 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     int id = index(0);
     unsigned long long ma = __ballot(id < 0), mb;
     P4<float> pa = point(id), pb;
+    float qa = charge1(id), qb = 0;
     id = index(1);
     int b = 0;
     for (; b + 2 <= nb; b += 2) {
         mb = __ballot(id < 0);
         pb = point(id);
+        qb = charge1(id);
         id = index(b + 2);
-        block(pa, ma, 4 * b);
+        block(pa, qa, ma, 4 * b);
         ma = __ballot(id < 0);
         pa = point(id);
+        qa = charge1(id);
         id = index(b + 3);
-        block(pb, mb, 4 * b + 4);
+        block(pb, qb, mb, 4 * b + 4);
     }
-    if (b < nb) block(pa, ma, 4 * b);
+    if (b < nb) block(pa, qa, ma, 4 * b);
     if (S > 1) {
-        *sum = ea;
+#pragma unroll
+        for (int v = 0; v < V; ++v) sum[v * (ne + 1) * 64] = ea[v];
         __syncthreads();
-        if (w > 0) return;
-        for (int e = 0; e < ne; ++e) acc += (double)sums[e * 64 + lane];
-    } else {
-        acc += (double)ea;
+        if (w >= V) return;  // wave v adds component v
+        double t = 0;
+        for (int e = 0; e < ne; ++e) t += (double)sums[(w * (ne + 1) + e) * 64 + lane];
+        if (active) pot_sorted[w * vs_pot + it.x + lane] += (float)t;
+        return;
     }
-    if (active) pot_sorted[it.x + lane] += (float)acc;
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        if (active) pot_sorted[v * vs_pot + it.x + lane] += (float)(acc[v] + (double)ea[v]);
 }
 
 // ------------------------------------------------ near field of many charge vectors (FP32)
@@ -2289,7 +2349,10 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
                                                       const int *__restrict__ rs_base, const int *__restrict__ rslot,
                                                       const long long *__restrict__ wave_base,
                                                       const int *__restrict__ steps, const double *__restrict__ coeffs,
-                                                      double *__restrict__ pot_sorted, int item0, int item1, int ne_max) {
+                                                      double *__restrict__ pot_sorted, int item0, int item1, int ne_max,
+                                                   long long vs_src = 0, long long vs_pot = 0) {
+    src += (long long)blockIdx.z * vs_src;  // component blockIdx.z of a quasi-periodic pass
+    pot_sorted += (long long)blockIdx.z * vs_pot;
     extern __shared__ double2 nf_lds64[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int item = S > 1 ? (int)blockIdx.x * S + w
@@ -2495,14 +2558,18 @@ __device__ __forceinline__ void ff_tables(double *trig, double2 *E2, double2 *E3
 // launch takes vectors V z .. V z + V - 1 (< nv; vector v's charges at q + v vs_q, its sums at
 // Sp + v vs_sp) on one set of tables and phases; each vector's sums are those of a one-vector
 // launch, bit for bit.
-template <int U, int V>
-__global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restrict__ theta, const double *__restrict__ q, int n,
+//
+// CPLX (quasi-periodic, V = 1): charges q e^{-i bx} and lines over the whole mode box.
+template <int U, int V, bool CPLX>
+__global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restrict__ theta, const double *__restrict__ q,
+                                                       const double *__restrict__ bx, int n,
                                                        int tp, FfDims d, const int4 *__restrict__ lines,
                                                        const int *__restrict__ line_m0, const int2 *__restrict__ units,
                                                        int n_units, int n_modes, double2 *__restrict__ Sp,
                                                        long long vs_q = 0, long long vs_sp = 0, int nv = 1) {
     extern __shared__ double2 ff_lds[];
-    __shared__ double Qs[V][32];
+    static_assert(!CPLX || V == 1, "complex charges: one vector");
+    __shared__ double Qs[CPLX ? 2 : V][32];
     const int v0 = blockIdx.z * V;
     double *trig = reinterpret_cast<double *>(ff_lds);
     const int ts = d.ts();
@@ -2531,6 +2598,14 @@ __global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restric
         // (from the last threads down: the first ones are busy with the tables)
         for (int t = 255 - (int)threadIdx.x; t < tp * V; t += 256) {
             const int pp = t % tp, v = t / tp;
+            if constexpr (CPLX) {
+                double sn = 0, cs = 0;
+                if (p0 + pp < n) sincos(bx[p0 + pp], &sn, &cs);
+                const double qp = p0 + pp < n ? q[p0 + pp] : 0.0;
+                Qs[0][pp] = qp * cs;
+                Qs[1][pp] = -qp * sn;
+                continue;
+            }
             Qs[v][pp] = p0 + pp < n && v0 + v < nv ? q[(long long)(v0 + v) * vs_q + p0 + pp] : 0.0;
         }
         __syncthreads();
@@ -2543,6 +2618,7 @@ __global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restric
             double qq[V];
 #pragma unroll
             for (int v = 0; v < V; ++v) qq[v] = Qs[v][p];
+            const double qi = CPLX ? Qs[1][p] : 0.0;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 b[u] = tr[oc[u]];
@@ -2553,6 +2629,11 @@ __global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restric
             for (int u = 0; u < U; ++u) {
                 const double xi = s2[u] * x[u].y, yi = s3[u] * y[u].y;
                 const double ar = fma(x[u].x, y[u].x, -xi * yi), ai = fma(x[u].x, yi, xi * y[u].x);
+                if constexpr (CPLX) {
+                    are[0][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(fma(qq[0], ar, -qi * ai), b[u], are[0][u], 0, 0, 0);
+                    aim[0][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(fma(qq[0], ai, qi * ar), b[u], aim[0][u], 0, 0, 0);
+                    continue;
+                }
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
                     const double qb = qq[v] * b[u];
@@ -2648,14 +2729,18 @@ __global__ __launch_bounds__(512) void k_ff_reduce(const double2 *__restrict__ S
 // are added in wave order.  Workgroup z of a many-vector launch evaluates vectors V z .. (< nv;
 // G + v vs_g, output at far + v vs_far) on one set of tables and phases, each as a one-vector
 // launch does, bit for bit.
-template <int RT, int V>
-__global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ theta, int n, FfDims d,
+// CPLX: far holds complex values, e^{i bx} sum_m S[m] e^{i m.th}.
+template <int RT, int V, bool CPLX>
+__global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ theta, const double *__restrict__ bx, int n,
+                                                 FfDims d,
                                                  const int4 *__restrict__ lines, const int2 *__restrict__ info, int n_lt,
                                                  const double *__restrict__ G, double *__restrict__ far,
                                                  long long vs_g = 0, long long vs_far = 0, int nv = 1) {
     extern __shared__ double2 ff_lds[];
     constexpr int TP = 16 * RT;
-    __shared__ double red[V][4][TP];
+    static_assert(!CPLX || V == 1, "complex charges: one vector");
+    constexpr int VO = CPLX ? 2 : V;  // sums per point
+    __shared__ double red[VO][4][TP];
     const int v0 = blockIdx.z * V;
     double *trig = reinterpret_cast<double *>(ff_lds);
     const int ts = d.ts();
@@ -2665,9 +2750,9 @@ __global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ t
     __syncthreads();
     const int lane = threadIdx.x & 63, kk = lane >> 4, jj = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    double acc[V][RT][4];
+    double acc[VO][RT][4];
 #pragma unroll
-    for (int v = 0; v < V; ++v)
+    for (int v = 0; v < VO; ++v)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -2711,10 +2796,11 @@ __global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ t
 #pragma unroll
                 for (int v = 0; v < V; ++v)
                     acc[v][rt][e] = fma(ar, dr[v][rt][e], fma(-ai, di[v][rt][e], acc[v][rt][e]));
+                if constexpr (CPLX) acc[1][rt][e] = fma(ar, di[0][rt][e], fma(ai, dr[0][rt][e], acc[1][rt][e]));
             }
     }
 #pragma unroll
-    for (int v = 0; v < V; ++v)
+    for (int v = 0; v < VO; ++v)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -2727,6 +2813,16 @@ __global__ __launch_bounds__(256, 2) void k_ff_eval(const double *__restrict__ t
     __syncthreads();
     for (int t = threadIdx.x; t < TP * V; t += blockDim.x) {
         const int v = t / TP, p = t % TP;
+        if constexpr (CPLX) {
+            if (p0 + p >= n) continue;
+            double sn, cs;
+            sincos(bx[p0 + p], &sn, &cs);
+            reinterpret_cast<double2 *>(far)[p0 + p] =
+                cmul(make_double2(red[0][0][p] + red[0][1][p] + red[0][2][p] + red[0][3][p],
+                                  red[1][0][p] + red[1][1][p] + red[1][2][p] + red[1][3][p]),
+                     make_double2(cs, sn));
+            continue;
+        }
         if (p0 + p < n && v0 + v < nv)
             far[(long long)(v0 + v) * vs_far + p0 + p] = red[v][0][p] + red[v][1][p] + red[v][2][p] + red[v][3][p];
     }
@@ -3134,154 +3230,6 @@ __global__ __launch_bounds__(64) void k_nufft_interp(const double *__restrict__ 
         }
     }
     reduce(nb);
-}
-
-
-// ------------------------------------------------------------------ quasi-periodic far field
-// psi(x_u) = e^{i b.x_u} sum_m w_m S(m) e^{i m.theta_u},  S(m) = sum_l q_l e^{-i b.x_l}
-// e^{-i m.theta_l}, over the full mode box m = (i, j, k) - (ms/2, mt/2, mu/2), index
-// i + ms (j + mt k); w_m = 0 outside the window (cpp/src/dmk/pbc.cpp:249-355).  FP64.
-// Sp[y][m]: partial structure factors of the points of workgroup column y.  Per tile of tp
-// points the per-axis factors e^{-i m_d theta_d} are tabulated in LDS by recurrence
-// (tp (ms + mt + mu + 2) complex values); a thread owns QP_CHUNK consecutive i of one (j, k)
-// line and walks them by multiplying with e^{-i theta_1}, so a (point, mode) pair costs one
-// complex multiply-add.
-constexpr int QP_CHUNK = 8;
-__global__ __launch_bounds__(256) void k_qp_structure(const double *__restrict__ theta, const double *__restrict__ bx,
-                                                       const double *__restrict__ q, int n, int ms, int mt, int mu, int tp,
-                                                       double2 *__restrict__ Sp) {
-    extern __shared__ double2 qp_lds[];
-    double2 *E1 = qp_lds, *E2 = E1 + tp * ms, *E3 = E2 + tp * mt, *Q = E3 + tp * mu, *Est = Q + tp;
-    const int M = ms * mt * mu, nci = (ms + QP_CHUNK - 1) / QP_CHUNK;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = c < nci * mt * mu;
-    const int i0 = active ? QP_CHUNK * (c % nci) : 0, j = active ? (c / nci) % mt : 0, k = active ? c / (nci * mt) : 0;
-    double2 acc[QP_CHUNK];
-#pragma unroll
-    for (int r = 0; r < QP_CHUNK; ++r) acc[r] = make_double2(0, 0);
-    for (int p0 = blockIdx.y * tp; p0 < n; p0 += gridDim.y * tp) {
-        __syncthreads();
-        for (int t = threadIdx.x; t < tp * 4; t += blockDim.x) {
-            const int pp = t % tp, ax = t / tp, gp = p0 + pp;
-            if (ax == 3) {  // q e^{-i b.x}
-                double sn = 0, cs = 0;
-                if (gp < n) {
-                    sincos(-bx[gp], &sn, &cs);
-                    sn *= q[gp];
-                    cs *= q[gp];
-                }
-                Q[pp] = make_double2(cs, sn);
-                continue;
-            }
-            const int cnt = ax == 0 ? ms : (ax == 1 ? mt : mu);
-            double2 *row = (ax == 0 ? E1 : (ax == 1 ? E2 : E3)) + pp * cnt;
-            const double th = gp < n ? theta[3 * (size_t)gp + ax] : 0.0;
-            double s1, c1, sl, cl;
-            sincos(th, &s1, &c1);
-            sincos(th * (cnt / 2), &sl, &cl);
-            const double2 step = make_double2(c1, -s1);  // e^{-i th}
-            if (ax == 0) Est[pp] = step;
-            double2 cur = make_double2(cl, sl);  // e^{-i (-(cnt/2)) th}
-            for (int mm = 0; mm < cnt; ++mm) {
-                row[mm] = cur;
-                cur = cmul(cur, step);
-            }
-        }
-        __syncthreads();
-        if (active) {
-            const int np = min(tp, n - p0);
-            for (int pp = 0; pp < np; ++pp) {
-                const double2 st = Est[pp];
-                double2 cur = cmul(cmul(cmul(E1[pp * ms + i0], E2[pp * mt + j]), E3[pp * mu + k]), Q[pp]);
-#pragma unroll
-                for (int r = 0; r < QP_CHUNK; ++r) {
-                    acc[r].x += cur.x;
-                    acc[r].y += cur.y;
-                    cur = cmul(cur, st);
-                }
-            }
-        }
-    }
-    if (active) {
-        const int m0 = i0 + ms * (j + mt * k);
-#pragma unroll
-        for (int r = 0; r < QP_CHUNK; ++r)
-            if (i0 + r < ms) Sp[(size_t)blockIdx.y * M + m0 + r] = acc[r];
-    }
-}
-
-// S[m] = w[m] sum_y Sp[y][m], partials added in column order (deterministic).
-__global__ __launch_bounds__(256) void k_qp_reduce(const double2 *__restrict__ Sp, int nblk, const double *__restrict__ w,
-                                                    int M, double2 *__restrict__ S) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M) return;
-    double2 a = make_double2(0, 0);
-    for (int b = 0; b < nblk; ++b) {
-        const double2 v = Sp[(size_t)b * M + m];
-        a.x += v.x;
-        a.y += v.y;
-    }
-    S[m] = make_double2(a.x * w[m], a.y * w[m]);
-}
-
-// out[2u], out[2u + 1] += Re, Im psi(x_u).  The i axis is taken in chunks of QP_CHUNK: the
-// chunk's factors e^{i m_1 theta_1} sit in registers and serve every (j, k) line, whose
-// factors follow recurrences in e^{i theta_2}, e^{i theta_3}; the weighted structure factors
-// are read at wave-uniform addresses.
-template <class R>
-__global__ __launch_bounds__(256) void k_qp_eval(const double *__restrict__ theta, const double *__restrict__ bx, int n,
-                                                  int ms, int mt, int mu, const double2 *__restrict__ S, R *__restrict__ out) {
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= n) return;
-    double2 st[3], e[3];
-    const int cnt[3] = {ms, mt, mu};
-    for (int d = 0; d < 3; ++d) {
-        const double th = theta[3 * (size_t)u + d];
-        double sn, cs;
-        sincos(th, &sn, &cs);
-        e[d] = make_double2(cs, sn);  // e^{i th}
-        sincos(-th * (cnt[d] / 2), &sn, &cs);
-        st[d] = make_double2(cs, sn);  // e^{i (-(cnt/2)) th}
-    }
-    double2 acc = make_double2(0, 0), c1next = st[0];
-    for (int i0 = 0; i0 < ms; i0 += QP_CHUNK) {
-        double2 c1[QP_CHUNK];
-#pragma unroll
-        for (int r = 0; r < QP_CHUNK; ++r) {
-            c1[r] = c1next;
-            c1next = cmul(c1next, e[0]);
-        }
-        const int nr = min(QP_CHUNK, ms - i0);
-        double2 c3 = st[2];
-        for (int k = 0; k < mu; ++k) {
-            double2 acc2 = make_double2(0, 0), c2 = st[1];
-            for (int j = 0; j < mt; ++j) {
-                const double2 *row = S + ((size_t)k * mt + j) * ms + i0;
-                double2 l = make_double2(0, 0);
-#pragma unroll
-                for (int r = 0; r < QP_CHUNK; ++r) {
-                    if (r < nr) {
-                        const double2 v = row[r];
-                        l.x = fma(v.x, c1[r].x, fma(-v.y, c1[r].y, l.x));
-                        l.y = fma(v.x, c1[r].y, fma(v.y, c1[r].x, l.y));
-                    }
-                }
-                const double2 t2 = cmul(l, c2);
-                acc2.x += t2.x;
-                acc2.y += t2.y;
-                c2 = cmul(c2, e[1]);
-            }
-            const double2 t3 = cmul(acc2, c3);
-            acc.x += t3.x;
-            acc.y += t3.y;
-            c3 = cmul(c3, e[2]);
-        }
-    }
-    double sn, cs;
-    sincos(bx[u], &sn, &cs);
-    const double2 psi = cmul(acc, make_double2(cs, sn));
-    out[2 * (size_t)u] = (R)((double)out[2 * (size_t)u] + psi.x);
-    out[2 * (size_t)u + 1] = (R)((double)out[2 * (size_t)u + 1] + psi.y);
 }
 
 }  // namespace pdmk::gpu

@@ -108,10 +108,11 @@ int log2_bucket(long long v) {
 }
 
 // LDS of a row near-field workgroup of S waves that share one item (k_near_rows, k_near_rows64)
-template <class Real> size_t near_parts_lds(int S, int ne_max) {
+// (pair 2: sums of both components of a quasi-periodic tree)
+template <class Real> size_t near_parts_lds(int S, int ne_max, int pair = 1) {
     const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(ne_max + 1) * 6 * 16
                                                              : near_rows64_lds_per_wave(ne_max);
-    return S * per_wave + (size_t)(ne_max + 1) * 64 * sizeof(Real);
+    return S * per_wave + (size_t)(ne_max + 1) * 64 * sizeof(Real) * pair;
 }
 
 // Waves per item of the row near field.  Alone, 6 digits FP32 / FP64, one wave per item against
@@ -119,14 +120,14 @@ template <class Real> size_t near_parts_lds(int S, int ne_max) {
 // 86 / 117, 73 / 96; 512 items (3e4) 152 / 212, 82 / 111, 75 / 110; 2048 items (1.2e5) 329 / 511,
 // 247 / 413, 258 / 453; 4096 items (2.5e5) 206 / 331, 224 / 500, -: one wave from 2560 items on,
 // 8 up to 256, within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or 8 forces a count).
-template <class Real> int near_parts(int n_items, int ne_max) {
+template <class Real> int near_parts(int n_items, int ne_max, int pair) {
     int S = n_items <= 256 ? 8 : (n_items < 2560 ? 4 : 1);
     if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
         const int v = std::atoi(e);
         S = v >= 8 ? 8 : (v >= 4 ? 4 : 1);
     }
-    if (S == 8 && near_parts_lds<Real>(S, ne_max) > 65536) S = 4;
-    if (S == 4 && near_parts_lds<Real>(S, ne_max) > 65536) S = 1;
+    if (S == 8 && near_parts_lds<Real>(S, ne_max, pair) > 65536) S = 4;
+    if (S == 4 && near_parts_lds<Real>(S, ne_max, pair) > 65536) S = 1;
     return S;
 }
 
@@ -282,8 +283,14 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     trg.upload(trgv);
     trg_user.upload(tu);
     trg_w0.upload(tw0);
-    pot_sorted.alloc(sizeof(Real) * (size_t)n);
-    pot_near.alloc(sizeof(Real) * (size_t)n);
+    pot_sorted.alloc(sizeof(Real) * (size_t)n * (qp ? 2 : 1));
+    pot_near.alloc(sizeof(Real) * (size_t)n * (qp ? 2 : 1));
+    if (qp) {
+        const size_t ld = sizeof(P4<Real>) * (size_t)(nsall + NF_CHUNK + 1);
+        qp_src.alloc(2 * ld);
+        for (int c = 0; c < 2; ++c)
+            check(hipMemcpy(qp_src.as<char>() + c * ld, src.p, ld, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
+    }
     q_dev.alloc(sizeof(double) * (size_t)n);
     pot_dev.alloc(sizeof(Real) * (size_t)n);
     far.alloc(sizeof(double) * (size_t)n);
@@ -404,8 +411,18 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     for (int b = 0; b < nboxes; ++b) up_src[b] = fold[b] < 0 ? up_of[b] : up_of[fold[b]];
     const size_t P3 = (size_t)p * p * p;
     const int H = (n_pw + 1) / 2, NM = n_pw * n_pw * H;
-    proxy_up.alloc(sizeof(Real) * P3 * std::max(1, n_up));
-    proxy_down.alloc(sizeof(Real) * P3 * std::max(1, n_down));
+    st_up = (long long)P3 * std::max(1, n_up);
+    st_down = (long long)P3 * std::max(1, n_down);
+    if (qp && p < 28) {
+        // both components of a quasi-periodic call per chain launch when their buffers take less
+        // than half of the free device memory
+        size_t free_b = 0, total_b = 0;
+        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        const double one = sizeof(Real) * ((double)st_up * 2 + (double)st_down + 2.0 * NM * std::max(1, n_up)) + kPinBytes;
+        if (2 * one < 0.5 * (double)free_b) qp_nv = 2;
+    }
+    proxy_up.alloc(sizeof(Real) * st_up * qp_nv);
+    proxy_down.alloc(sizeof(Real) * st_down * qp_nv);
 
     // ---------------- upward: one charge->proxy group per proxy slot (possibly without sources)
     {
@@ -837,7 +854,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             check(hipMemGetInfo(&mem_free, &mem_total), "hipMemGetInfo");
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
             if (nf_rows) {
-                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max);
+                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, qp && std::is_same<Real, float>::value ? 2 : 1);
                 if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c);
             }
         }
@@ -960,7 +977,8 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             const double *a = T.ainv;  // a11, a21, a22, a31, a32, a33
             const double dfac = 4 * M_PI / (T.psi0 * U[0] * U[4] * U[8]);
             const host::Pswf pf(T.beta);
-            std::vector<double> wq((size_t)qs * qt * qu, 0.0), bx(n);
+            std::vector<int> qm;
+            std::vector<double> wq, bx(n);
             for (int k = 0; k < qu; ++k)
                 for (int j = 0; j < qt; ++j)
                     for (int i = 0; i < qs; ++i) {
@@ -970,12 +988,16 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                         const double kk = k1 * k1 + k2 * k2 + k3 * k3;
                         if (kk < 1e-30) continue;
                         const double x = std::sqrt(kk) * rc / T.beta;
-                        if (x <= 1) wq[i + (size_t)qs * (j + (size_t)qt * k)] = dfac * pf(x) / kk;
+                        if (x > 1) continue;
+                        for (int v : {mi, mj, mk}) qm.push_back(v);
+                        wq.push_back(dfac * pf(x) / kk);
                     }
             for (int u = 0; u < n; ++u)
                 bx[u] = bloch[0] * g.r_src[3 * (size_t)u] + bloch[1] * g.r_src[3 * (size_t)u + 1] +
                         bloch[2] * g.r_src[3 * (size_t)u + 2];
-            qpf.setup(th, bx, n, qs, qt, qu, wq);
+            qpf.bx.upload(bx);
+            qpf.setup(th, n, qm, wq, nullptr, 1024);
+            qp_far.alloc(sizeof(double2) * (size_t)n);
             pot_dev2.alloc(2 * sizeof(Real) * (size_t)n);
         }
         build_ms[2] = ms_since(t_far);
@@ -998,7 +1020,8 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         for (auto &E : eval_levels) items = std::max(items, E.n_items);
         pin_batch = std::max(1, std::min(items, (int)(kPinBytes / ((size_t)NM * 2 * sizeof(Real)))));
         if (pin_batch < items) pin_batch = std::max(kShiftGroup, pin_batch / kShiftGroup * kShiftGroup);
-        pin.alloc((size_t)pin_batch * NM * 2 * sizeof(Real));
+        st_pin = (long long)pin_batch * NM;
+        pin.alloc((size_t)st_pin * 2 * sizeof(Real) * qp_nv);
         // two-pass proxy <-> plane-wave transforms (FP64 at p >= 28, whose slices re-read a
         // box's input kTwoPassSlices times or more): the first contraction of a chunk of boxes
         // (PDMK_TWO_PASS=0 turns them off, PDMK_TWO_PASS=<MiB> caps the chunk scratch)
@@ -1026,7 +1049,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         for (auto &E : eval_levels) lvl_cnt = std::max(lvl_cnt, E.pw_cnt);
         size_t free_b = 0, total_b = 0;
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        const size_t all_bytes = pw_slot * (size_t)std::max(1, n_up) + c2p_bytes;
+        const size_t all_bytes = (pw_slot * (size_t)std::max(1, n_up) + c2p_bytes) * qp_nv;
         pw_by_level = all_bytes + (size_t(1) << 30) > free_b;
         if (const char *e = std::getenv("PDMK_PW_LEVELS")) pw_by_level = e[0] == '1';
         if (const char *e = std::getenv("PDMK_T3_MFMA")) t3_mfma = e[0] != '0';
@@ -1042,10 +1065,15 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         shift_groups = p >= 28;
         if (const char *e = std::getenv("PDMK_SHIFT_GROUPS")) shift_groups = e[0] != '0';
         if (pw_by_level) {
-            pw_out.alloc(std::max(pw_slot * (size_t)lvl_cnt, c2p_bytes));
+            // (in whole plane-wave elements: the child -> parent scratch starts at the same places)
+            st_pw = (long long)((std::max(pw_slot * (size_t)lvl_cnt, c2p_bytes) + 2 * sizeof(Real) - 1) / (2 * sizeof(Real)));
+            st_c2p = 2 * st_pw;
+            pw_out.alloc((size_t)st_pw * 2 * sizeof(Real) * qp_nv);
         } else {
-            pw_out.alloc(pw_slot * (size_t)std::max(1, n_up));
-            c2p_scratch.alloc(c2p_bytes);
+            st_pw = (long long)NM * std::max(1, n_up);
+            st_c2p = (long long)(c2p_bytes / sizeof(Real));
+            pw_out.alloc((size_t)st_pw * 2 * sizeof(Real) * qp_nv);
+            c2p_scratch.alloc(c2p_bytes * qp_nv);
         }
     }
 
@@ -1186,17 +1214,20 @@ namespace {
 
 // The arrays one pass of the proxy / plane-wave chain works on: the plan's own (one vector,
 // charges in src[].w), or nv vectors' copies, vector v at v times the element strides, with
-// charges qv[source * qv_ld + v] (the kernels take v from blockIdx.z).
+// charges qv[source * qv_ld + v], or src[v s_src + source].w without qv (the kernels take v from
+// blockIdx.z).
 template <class Real> struct ChainBufs {
     Real *up, *c2p, *down, *pot;
     Cx<Real> *pw, *pin;
+    const P4<Real> *src;
     const Real *qv = nullptr;
     int qv_ld = 0, nv = 1;
-    long long s_up = 0, s_c2p = 0, s_pw = 0, s_pin = 0, s_down = 0, s_pot = 0;
+    long long s_src = 0, s_up = 0, s_c2p = 0, s_pw = 0, s_pin = 0, s_down = 0, s_pot = 0;
 };
 
 template <class Real> ChainBufs<Real> own_chain(Plan<Real> &pl) {
     ChainBufs<Real> b;
+    b.src = pl.src.template as<P4<Real>>();
     b.up = pl.proxy_up.template as<Real>();
     b.c2p = pl.c2p_buffer();
     b.down = pl.proxy_down.template as<Real>();
@@ -1256,7 +1287,7 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
             auto c2p = [&](auto wide) {
                 constexpr bool W = decltype(wide)::value;
                 hipLaunchKernelGGL((k_charge2proxy_mfma<Real, P, W>), dim3(pl.n_up * C2pMfmaCfg<P, W>::RS),
-                                   dim3(64 * C2pMfmaCfg<P, W>::NW), 0, s, pl.src.template as<P4<Real>>(),
+                                   dim3(64 * C2pMfmaCfg<P, W>::NW), 0, s, B.src,
                                    pl.up_slot.template as<int>(), pl.up_geom.template as<Real>(),
                                    pl.up_rng.template as<int>(), pl.rng_begin.template as<int>(),
                                    pl.rng_count.template as<int>(), pl.rng_off.template as<Real>(), B.up);
@@ -1268,9 +1299,9 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
                 c2p(std::false_type{});
         } else {
             hipLaunchKernelGGL((k_charge2proxy<Real, P>), dim3(pl.n_up, 1, nv), dim3(C2pCfg<P>::threads), 0, s,
-                               pl.src.template as<P4<Real>>(), pl.up_slot.template as<int>(), pl.up_geom.template as<Real>(),
+                               B.src, pl.up_slot.template as<int>(), pl.up_geom.template as<Real>(),
                                pl.up_rng.template as<int>(), pl.rng_begin.template as<int>(), pl.rng_count.template as<int>(),
-                               pl.rng_off.template as<Real>(), B.up, B.qv, B.qv_ld, B.s_up);
+                               pl.rng_off.template as<Real>(), B.up, B.qv, B.qv_ld, B.s_up, B.s_src);
             check(hipGetLastError(), "k_charge2proxy");
         }
     }
@@ -1402,56 +1433,84 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
     }
 }
 
+// the near field's sources: the plan's, or both components' of a quasi-periodic tree (grid z)
+template <class Real> struct NearSrc {
+    const P4<Real> *src;
+    int nz = 1;
+    long long vs_src = 0, vs_pot = 0;
+    NearSrc(Plan<Real> &pl, bool pair) : src(pl.src.template as<P4<Real>>()) {
+        if (!pair) return;
+        src = pl.qp_src.template as<P4<Real>>();
+        nz = 2;
+        vs_src = pl.nsall + NF_CHUNK + 1;
+        vs_pot = pl.n;
+    }
+};
+
 // wpb = wavefronts (items) per workgroup: 4 when the near field runs beside the whole
 // transform chain; 16 when it starts late beside the long FP64 downward pass, where whole
 // 16-wave workgroups retiring at once leave room for the chain's large workgroups.
 template <class Real, int NC, bool SPLIT>
-void launch_near(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1) {
+void launch_near(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1, bool pair) {
     if (i1 <= i0) return;
-    hipLaunchKernelGGL((k_near_field<Real, NC, SPLIT>), dim3((i1 - i0 + wpb - 1) / wpb), dim3(64 * wpb), 0, s,
-                       pl.src.template as<P4<Real>>(), pl.trg.template as<P4<Real>>(), pl.nf_items.template as<int4>(),
+    const NearSrc<Real> N(pl, pair);
+    hipLaunchKernelGGL((k_near_field<Real, NC, SPLIT>), dim3((i1 - i0 + wpb - 1) / wpb, 1, N.nz), dim3(64 * wpb), 0, s,
+                       N.src, pl.trg.template as<P4<Real>>(), pl.nf_items.template as<int4>(),
                        pl.nf_ptr.template as<int>(), pl.nf_l1.template as<NfEntry>(), pl.nf_geom.template as<P4<Real>>(),
                        pl.nf_ie_base.template as<int>(), pl.nf_ie_ptr.template as<long long>(), pl.nf_steps.template as<int>(),
-                       pl.coeffs.template as<Real>(), pl.pot_near.template as<Real>(), i0, i1);
+                       pl.coeffs.template as<Real>(), pl.pot_near.template as<Real>(), i0, i1, N.vs_src, N.vs_pot);
     check(hipGetLastError(), "k_near_field");
 }
 
 // row near field (plans built with row step lists): wpb items per workgroup, or nf_parts waves
 // per item
 template <class Real>
-void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1) {
+void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1, bool pair) {
     if (i1 <= i0) return;
     const int S = pl.nf_parts;
     const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(pl.nf_ne_max + 1) * 6 * sizeof(float4)
                                                              : near_rows64_lds_per_wave(pl.nf_ne_max);
     // (the LDS tables of a workgroup's wavefronts stay within 64 KiB)
     while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
+    const NearSrc<Real> N(pl, pair);
+    // FP32: one launch forms both components of a pair (V = 2); FP64: components along z
+    constexpr bool F32 = std::is_same<Real, float>::value;
+    const int nz = F32 ? 1 : N.nz;
     auto go = [&](auto kern) {
         if (S > 1)
-            hipLaunchKernelGGL(kern, dim3(i1 - i0), dim3(64 * S), near_parts_lds<Real>(S, pl.nf_ne_max), s,
-                               pl.src.template as<P4<Real>>(), pl.trg.template as<P4<Real>>(),
+            hipLaunchKernelGGL(kern, dim3(i1 - i0, 1, nz), dim3(64 * S),
+                               near_parts_lds<Real>(S, pl.nf_ne_max, F32 ? N.nz : 1), s,
+                               N.src, pl.trg.template as<P4<Real>>(),
                                pl.np_items.template as<int4>(), pl.nf_ptr.template as<int>(),
                                pl.nf_geom.template as<P4<Real>>(), pl.np_rs_base.template as<int>(),
                                pl.np_rslot.template as<int>(), pl.np_wave_base.template as<long long>(),
                                pl.np_steps.template as<int>(), pl.coeffs.template as<Real>(),
-                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max);
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot);
         else
-            hipLaunchKernelGGL(kern, dim3((i1 - i0 + wpb - 1) / wpb), dim3(64 * wpb), wpb * per_wave, s,
-                               pl.src.template as<P4<Real>>(), pl.trg.template as<P4<Real>>(),
+            hipLaunchKernelGGL(kern, dim3((i1 - i0 + wpb - 1) / wpb, 1, nz), dim3(64 * wpb), wpb * per_wave, s,
+                               N.src, pl.trg.template as<P4<Real>>(),
                                pl.nf_items.template as<int4>(), pl.nf_ptr.template as<int>(),
                                pl.nf_geom.template as<P4<Real>>(), pl.nf_rs_base.template as<int>(),
                                pl.nf_rslot.template as<int>(), pl.nf_wave_base.template as<long long>(),
                                pl.nf_row_steps.template as<int>(), pl.coeffs.template as<Real>(),
-                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max);
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot);
         check(hipGetLastError(), "k_near_rows");
     };
     auto by_parts = [&](auto nc) {
         constexpr int NC = decltype(nc)::value;
-        if constexpr (std::is_same<Real, float>::value) {
+        if constexpr (F32) {
+            if (pair) {
+                switch (S) {
+                case 8: go(k_near_rows<NC, 8, 2>); break;
+                case 4: go(k_near_rows<NC, 4, 2>); break;
+                default: go(k_near_rows<NC, 1, 2>); break;
+                }
+                return;
+            }
             switch (S) {
-            case 8: go(k_near_rows<NC, 8>); break;
-            case 4: go(k_near_rows<NC, 4>); break;
-            default: go(k_near_rows<NC, 1>); break;
+            case 8: go(k_near_rows<NC, 8, 1>); break;
+            case 4: go(k_near_rows<NC, 4, 1>); break;
+            default: go(k_near_rows<NC, 1, 1>); break;
             }
         } else {
             switch (S) {
@@ -1473,7 +1532,40 @@ void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1) {
     throw std::logic_error("row near field: unsupported coefficient count");
 }
 
+template <class Real> void run_chain(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) {
+    switch (pl.p) {
+    case 9: launch_transforms<Real, 9, 13>(pl, s, B); break;
+    case 18: launch_transforms<Real, 18, 27>(pl, s, B); break;
+    case 28: launch_transforms<Real, 28, 39>(pl, s, B); break;
+    case 38: launch_transforms<Real, 38, 55>(pl, s, B); break;
+    default: throw std::logic_error("unsupported proxy order");
+    }
+}
+
 }  // namespace
+
+template <typename Real>
+void Plan<Real>::near_field(hipStream_t s, int wpb, bool pair) {
+    const int i0 = 0, i1 = n_nf_items;
+    if (nf_rows) {
+        launch_near_rows<Real>(*this, s, wpb, i0, i1, pair);
+        return;
+    }
+    switch (n_digits) {
+    case 1: case 2: launch_near<Real, 5, true>(*this, s, wpb, i0, i1, pair); break;
+    case 3: launch_near<Real, 6, true>(*this, s, wpb, i0, i1, pair); break;
+    case 4: launch_near<Real, 9, true>(*this, s, wpb, i0, i1, pair); break;
+    case 5: launch_near<Real, 11, true>(*this, s, wpb, i0, i1, pair); break;
+    case 6: launch_near<Real, 12, false>(*this, s, wpb, i0, i1, pair); break;
+    case 7: launch_near<Real, 15, false>(*this, s, wpb, i0, i1, pair); break;
+    case 8: launch_near<Real, 17, false>(*this, s, wpb, i0, i1, pair); break;
+    case 9: launch_near<Real, 18, false>(*this, s, wpb, i0, i1, pair); break;
+    case 10: launch_near<Real, 22, false>(*this, s, wpb, i0, i1, pair); break;
+    case 11: launch_near<Real, 23, false>(*this, s, wpb, i0, i1, pair); break;
+    case 12: launch_near<Real, 25, false>(*this, s, wpb, i0, i1, pair); break;
+    default: throw std::logic_error("unsupported digit count");
+    }
+}
 
 template <typename Real>
 void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int stages, double *times_ms) {
@@ -1506,8 +1598,7 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     {
         const int m = std::max(nsall, n);
         hipLaunchKernelGGL(k_gather_charges<Real>, dim3((m + 255) / 256), dim3(256), 0, s, d_q, src_user.as<int>(),
-                           src.as<P4<Real>>(), nsall, pot_sorted.as<Real>(), pot_near.as<Real>(), n,
-                           qp_comp >= 0 ? src_phase.as<double2>() : (const double2 *)nullptr, qp_comp < 0 ? 0 : qp_comp);
+                           src.as<P4<Real>>(), nsall, pot_sorted.as<Real>(), pot_near.as<Real>(), n);
         check(hipGetLastError(), "k_gather_charges");
     }
     mark(1, 1, s);
@@ -1517,33 +1608,9 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     }
     const bool near_late = !serial && (knobs.near_late >= 0 ? knobs.near_late == 1 : p >= 28);
     const int wpb = knobs.near_wpb > 0 ? knobs.near_wpb : (near_late ? 16 : 4);
-    auto near_field = [&](int i0, int i1) {
+    auto near = [&]() {
         mark(3, 0, sn);
-        if (stages & 2) {
-            switch (n_digits) {
-            case 1: case 2: launch_near<Real, 5, true>(*this, sn, wpb, i0, i1); break;
-            case 3: launch_near<Real, 6, true>(*this, sn, wpb, i0, i1); break;
-            case 4: launch_near<Real, 9, true>(*this, sn, wpb, i0, i1); break;
-            case 5: launch_near<Real, 11, true>(*this, sn, wpb, i0, i1); break;
-            case 6:
-                if (nf_rows) launch_near_rows<Real>(*this, sn, wpb, i0, i1);
-                else launch_near<Real, 12, false>(*this, sn, wpb, i0, i1);
-                break;
-            case 7: launch_near<Real, 15, false>(*this, sn, wpb, i0, i1); break;
-            case 8: launch_near<Real, 17, false>(*this, sn, wpb, i0, i1); break;
-            case 9:
-                if (nf_rows) launch_near_rows<Real>(*this, sn, wpb, i0, i1);
-                else launch_near<Real, 18, false>(*this, sn, wpb, i0, i1);
-                break;
-            case 10: launch_near<Real, 22, false>(*this, sn, wpb, i0, i1); break;
-            case 11: launch_near<Real, 23, false>(*this, sn, wpb, i0, i1); break;
-            case 12:
-                if (nf_rows) launch_near_rows<Real>(*this, sn, wpb, i0, i1);
-                else launch_near<Real, 25, false>(*this, sn, wpb, i0, i1);
-                break;
-            default: throw std::logic_error("unsupported digit count");
-            }
-        }
+        if (stages & 2) near_field(sn, wpb);
         mark(3, 1, sn);
     };
     // Start of the near field: at once when its cost is comparable to the transform chain's
@@ -1553,23 +1620,17 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     // field cut into two launches, is slower at 6 digits; the late start is faster at 9; a
     // start after the whole chain was slower at 6 and 9 digits, FP32 and FP64.)
     e_upward = near_late ? e_up : nullptr;
-    if (!serial && !near_late) near_field(0, n_nf_items);
+    if (!serial && !near_late) near();
     mark(2, 0, s);
     if (stages & 1) {
-        switch (p) {
-        case 9: launch_transforms<Real, 9, 13>(*this, s, own_chain(*this)); break;
-        case 18: launch_transforms<Real, 18, 27>(*this, s, own_chain(*this)); break;
-        case 28: launch_transforms<Real, 28, 39>(*this, s, own_chain(*this)); break;
-        case 38: launch_transforms<Real, 38, 55>(*this, s, own_chain(*this)); break;
-        default: throw std::logic_error("unsupported proxy order");
-        }
+        run_chain(*this, s, own_chain(*this));
     }
     mark(2, 1, s);
     if (times_ms) check(hipEventRecord(ev[2], s), "hipEventRecord");
-    if (serial) near_field(0, n_nf_items);
+    if (serial) near();
     if (near_late) {
         check(hipStreamWaitEvent(sn, e_up, 0), "hipStreamWaitEvent");
-        near_field(0, n_nf_items);
+        near();
     }
     if (!serial) {
         check(hipEventRecord(e_near, sn), "hipEventRecord");
@@ -1579,7 +1640,7 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     mark(4, 0, s);
     hipLaunchKernelGGL(k_finalize<Real>, dim3((n + 255) / 256), dim3(256), 0, s, pot_sorted.as<Real>(), pot_near.as<Real>(),
                        trg_w0.as<double>(), trg_user.as<int>(), d_q, far.as<double>(), far_idx.as<int>(), d_pot, n,
-                       (stages & 4) ? 1 : 0, (stages & 8) ? 1 : 0, qp_comp >= 0 ? 2 : 1);
+                       (stages & 4) ? 1 : 0, (stages & 8) ? 1 : 0);
     check(hipGetLastError(), "k_finalize");
     mark(4, 1, s);
     if (times_ms) {
@@ -1655,6 +1716,7 @@ void Plan<Real>::evaluate_many(int n_vec, const double *d_Q, Real *d_P, hipStrea
         while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
         // the chain copies: vector c of a chain launch at c times these element strides
         ChainBufs<float> cb;
+        cb.src = src.as<P4<float>>();
         cb.up = many_up.as<float>();
         cb.c2p = many_c2p.as<float>();
         cb.down = many_down.as<float>();
@@ -1718,7 +1780,7 @@ void Plan<Real>::evaluate_many(int n_vec, const double *d_Q, Real *d_P, hipStrea
             check(hipStreamWaitEvent(s, e_fr[b], 0), "hipStreamWaitEvent");
             hipLaunchKernelGGL(k_finalize<float>, dim3((n + 255) / 256, 1, vc), dim3(256), 0, s, many_pot.as<float>(),
                                many_near[b].as<float>(), trg_w0.as<double>(), trg_user.as<int>(), Q0, far0,
-                               far_idx.as<int>(), d_P + (size_t)v0 * n, n, 1, 1, 1, (long long)n, (long long)n,
+                               far_idx.as<int>(), d_P + (size_t)v0 * n, n, 1, 1, (long long)n, (long long)n,
                                (long long)n, (long long)n, (long long)n);
             check(hipGetLastError(), "k_finalize");
             check(hipEventRecord(e_fin[b], s), "hipEventRecord");
@@ -1851,60 +1913,76 @@ int Plan<Real>::kernel_times(double *avg_ms, int *n_calls) {
     return nc;
 }
 
-void QpFarField::setup(const std::vector<double> &theta_host, const std::vector<double> &bx_host, int n_points,
-                       int ms_, int mt_, int mu_, const std::vector<double> &w_full) {
-    n = n_points;
-    ms = ms_;
-    mt = mt_;
-    mu = mu_;
-    M = ms * mt * mu;
-    theta.upload(theta_host);
-    bx.upload(bx_host);
-    w.upload(w_full);
-    // points per LDS tile: up to 16 within 48 KB of tables; point columns: enough workgroups
-    // to fill the GPU, partials M complex each
-    tp = std::max(1, std::min(16, (int)((48 << 10) / (sizeof(double2) * (size_t)(ms + mt + mu + 2)))));
-    const int cblk = (((ms + QP_CHUNK - 1) / QP_CHUNK) * mt * mu + 255) / 256;
-    nblk = std::max(1, std::min((n + tp - 1) / tp, std::max(1, 4096 / cblk)));
-    Sp.alloc(sizeof(double2) * (size_t)nblk * M);
-    S.alloc(sizeof(double2) * (size_t)M);
-}
-
-template <class R>
-void QpFarField::run(const double *d_q, R *d_out, hipStream_t s) const {
-    if (n == 0) return;
-    const size_t lds = sizeof(double2) * (size_t)tp * (ms + mt + mu + 2);
-    const int nch = ((ms + QP_CHUNK - 1) / QP_CHUNK) * mt * mu;
-    hipLaunchKernelGGL(k_qp_structure, dim3((nch + 255) / 256, nblk), dim3(256), lds, s, theta.as<double>(), bx.as<double>(),
-                       d_q, n, ms, mt, mu, tp, Sp.as<double2>());
-    check(hipGetLastError(), "k_qp_structure");
-    hipLaunchKernelGGL(k_qp_reduce, dim3((M + 255) / 256), dim3(256), 0, s, Sp.as<double2>(), nblk, w.as<double>(), M,
-                       S.as<double2>());
-    check(hipGetLastError(), "k_qp_reduce");
-    hipLaunchKernelGGL(k_qp_eval<R>, dim3((n + 255) / 256), dim3(256), 0, s, theta.as<double>(), bx.as<double>(), n, ms, mt,
-                       mu, S.as<double2>(), d_out);
-    check(hipGetLastError(), "k_qp_eval");
-}
-template void QpFarField::run<float>(const double *, float *, hipStream_t) const;
-template void QpFarField::run<double>(const double *, double *, hipStream_t) const;
-
 template <typename Real>
 void Plan<Real>::evaluate_complex(const double *d_q, Real *d_out, hipStream_t s, int stages) {
     if (!qp) throw std::logic_error("evaluate_complex: bloch not set at construction");
     if (!s) s = stream;
-    // real part: proxy / plane waves, near field and self correction on Re(charges x phase);
-    // imaginary part: the same without the self correction (the originals' charges are real)
-    qp_comp = 0;
-    try {
-        evaluate(d_q, d_out, s, stages & 7, nullptr);
-        qp_comp = 1;
-        evaluate(d_q, d_out + 1, s, stages & 3, nullptr);
-    } catch (...) {
-        qp_comp = -1;
-        throw;
+    hipEvent_t *K = nullptr;
+    if (kslots > 0) K = &kev[(size_t)(kcall++ % kslots) * 2 * kGroups];
+    auto mark = [&](int g, int end, hipStream_t st) {
+        if (K) check(hipEventRecord(K[2 * g + end], st), "hipEventRecord");
+    };
+    const hipStream_t sf = single_stream ? s : s_far, sn = single_stream ? s : s_near;
+    check(hipEventRecord(e_in, s), "hipEventRecord");
+    if (!single_stream) check(hipStreamWaitEvent(sf, e_in, 0), "hipStreamWaitEvent");
+    mark(0, 0, sf);
+    if (stages & 8) qpf.run(d_q, qp_far.as<double>(), sf);
+    mark(0, 1, sf);
+    check(hipEventRecord(e_far, sf), "hipEventRecord");
+    mark(1, 0, s);
+    const long long ld = nsall + NF_CHUNK + 1;
+    const int m = std::max(nsall, 2 * n);
+    hipLaunchKernelGGL(k_gather_qp<Real>, dim3((m + 255) / 256), dim3(256), 0, s, d_q, src_user.as<int>(),
+                       src_phase.as<double2>(), qp_src.as<P4<Real>>(), ld, nsall, pot_sorted.as<Real>(),
+                       pot_near.as<Real>(), n);
+    check(hipGetLastError(), "k_gather_qp");
+    mark(1, 1, s);
+    check(hipEventRecord(e_gather, s), "hipEventRecord");
+    if (!single_stream) check(hipStreamWaitEvent(sn, e_gather, 0), "hipStreamWaitEvent");
+    // near field at once at p < 28, after the first upward pass above, as in evaluate()
+    const bool late = !single_stream && (stages & 1) && (knobs.near_late >= 0 ? knobs.near_late == 1 : p >= 28);
+    const int wpb = knobs.near_wpb > 0 ? knobs.near_wpb : (late ? 16 : 4);
+    auto near = [&]() {
+        mark(3, 0, sn);
+        if (stages & 2) near_field(sn, wpb, true);
+        mark(3, 1, sn);
+        check(hipEventRecord(e_near, sn), "hipEventRecord");
+    };
+    if (!late) near();
+    mark(2, 0, s);
+    if (stages & 1) {
+        ChainBufs<Real> B = own_chain(*this);
+        B.nv = qp_nv;
+        if (qp_nv > 1) {
+            B.s_src = ld;
+            B.s_up = st_up;
+            B.s_down = st_down;
+            B.s_pw = st_pw;
+            B.s_pin = st_pin;
+            B.s_c2p = st_c2p;
+            B.s_pot = n;
+        }
+        for (int c = 0; c < 2; c += qp_nv) {
+            B.src = qp_src.as<P4<Real>>() + c * ld;
+            B.pot = pot_sorted.as<Real>() + (size_t)c * n;
+            e_upward = late && c == 0 ? e_up : nullptr;
+            run_chain(*this, s, B);
+        }
+        e_upward = nullptr;
     }
-    qp_comp = -1;
-    if (stages & 8) qpf.run(d_q, d_out, s);
+    mark(2, 1, s);
+    if (late) {
+        check(hipStreamWaitEvent(sn, e_up, 0), "hipStreamWaitEvent");
+        near();
+    }
+    check(hipStreamWaitEvent(s, e_near, 0), "hipStreamWaitEvent");
+    check(hipStreamWaitEvent(s, e_far, 0), "hipStreamWaitEvent");
+    mark(4, 0, s);
+    hipLaunchKernelGGL(k_finalize_qp<Real>, dim3((n + 255) / 256), dim3(256), 0, s, pot_sorted.as<Real>(),
+                       pot_near.as<Real>(), trg_w0.as<double>(), trg_user.as<int>(), d_q, qp_far.as<double2>(), d_out, n,
+                       (stages & 4) ? 1 : 0, (stages & 8) ? 1 : 0);
+    check(hipGetLastError(), "k_finalize_qp");
+    mark(4, 1, s);
 }
 
 template <typename Real>
@@ -1975,7 +2053,7 @@ void FourierSum::setup(const std::vector<double> &theta_host, int n_points, cons
     // many vectors (N = 2e4, one column per tile: 0.5 GB of partial sums per 32 vectors), and
     // no more than about 2048 workgroups in all (at least 64 columns) are of use
     const int gy = std::max(1, (n_units + FF_UNITS - 1) / FF_UNITS), tiles = (n + tp - 1) / tp;
-    blocks = std::max(1, std::min({max_blocks, tiles, std::max(256, tiles / 4), std::max(64, 2048 / gy)}));
+    blocks = std::max(1, std::min({max_blocks, tiles, std::max(256, tiles / (4 * gy)), std::max(64, 2048 / gy)}));
     const size_t sp_n = (size_t)blocks * std::max(1, n_modes);
     s_len = (size_t)g_len + 128;  // the evaluation loads one step ahead
     if (arena) {
@@ -1997,7 +2075,8 @@ void FourierSum::run(const double *d_q, double *d_out, hipStream_t s) const {
 void FourierSum::run_at(const double *d_q, const double *d_theta_eval, int n_eval, double *d_out, hipStream_t s) const {
     if (n_eval <= 0) return;
     if (n == 0 || n_modes == 0) {
-        hipLaunchKernelGGL(k_fill<double>, dim3((n_eval + 255) / 256), dim3(256), 0, s, d_out, 0.0, n_eval);
+        const int m = bx.p ? 2 * n_eval : n_eval;
+        hipLaunchKernelGGL(k_fill<double>, dim3((m + 255) / 256), dim3(256), 0, s, d_out, 0.0, m);
         check(hipGetLastError(), "k_fill far");
         return;
     }
@@ -2014,12 +2093,15 @@ void FourierSum::structure(const double *d_q, long long ldq, int nv, double2 *sp
     auto go = [&](auto uu) {
         constexpr int U = decltype(uu)::value;
         auto launch = [&](auto vv) {
-            constexpr int V = decltype(vv)::value;
-            hipLaunchKernelGGL((k_ff_structure<U, V>), dim3(blocks, (n_units + 4 * U - 1) / (4 * U), (nv + V - 1) / V),
-                               dim3(256), dims.lds_bytes(tp), s, theta_d, d_q, n, tp, dims, lines_d, line_m0_d, units_d,
+            // (V = 0: complex charges)
+            constexpr int V = std::max(1, (int)decltype(vv)::value);
+            hipLaunchKernelGGL((k_ff_structure<U, V, decltype(vv)::value == 0>),
+                               dim3(blocks, (n_units + 4 * U - 1) / (4 * U), (nv + V - 1) / V),
+                               dim3(256), dims.lds_bytes(tp), s, theta_d, d_q, bx.as<double>(), n, tp, dims, lines_d, line_m0_d, units_d,
                                n_units, n_modes, sp, ldq, vs_sp, nv);
         };
-        if (nv == 1) launch(std::integral_constant<int, 1>{});
+        if (bx.p) launch(std::integral_constant<int, 0>{});
+        else if (nv == 1) launch(std::integral_constant<int, 1>{});
         else launch(std::integral_constant<int, FF_MANY>{});
         check(hipGetLastError(), "k_ff_structure");
     };
@@ -2038,16 +2120,17 @@ void FourierSum::eval(const double *d_theta_eval, int n_eval, int nv, const doub
                       hipStream_t s) const {
     const FfDims dims{dim_i, dim_j, dim_k};
     auto go = [&](auto rt, auto vv) {
-        constexpr int RT = decltype(rt)::value, V = decltype(vv)::value;
-        hipLaunchKernelGGL((k_ff_eval<RT, V>), dim3((n_eval + 16 * RT - 1) / (16 * RT), 1, (nv + V - 1) / V), dim3(256),
-                           dims.lds_bytes(16 * RT), s, d_theta_eval, n_eval, dims, lines_d, info_d, n_lt, g, d_out,
+        constexpr int RT = decltype(rt)::value, V = std::max(1, (int)decltype(vv)::value);
+        hipLaunchKernelGGL((k_ff_eval<RT, V, decltype(vv)::value == 0>), dim3((n_eval + 16 * RT - 1) / (16 * RT), 1, (nv + V - 1) / V), dim3(256),
+                           dims.lds_bytes(16 * RT), s, d_theta_eval, bx.as<double>(), n_eval, dims, lines_d, info_d, n_lt, g, d_out,
                            (long long)s_len, ldo, nv);
     };
     auto by_rt = [&](auto vv) {
         if (tp == 32) go(std::integral_constant<int, 2>{}, vv);
         else go(std::integral_constant<int, 1>{}, vv);
     };
-    if (nv == 1) by_rt(std::integral_constant<int, 1>{});
+    if (bx.p) by_rt(std::integral_constant<int, 0>{});
+    else if (nv == 1) by_rt(std::integral_constant<int, 1>{});
     else by_rt(std::integral_constant<int, FF_MANY>{});
     check(hipGetLastError(), "k_ff_eval");
 }

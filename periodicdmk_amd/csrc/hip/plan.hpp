@@ -74,10 +74,14 @@ struct Work {
 // Its arrays are owned buffers, or slices of an Arena when setup() is given one.  The
 // structure factors are summed in `blocks` partial sums of point tiles (at most max_blocks),
 // then added in block order.
+//
+// With bx (quasi-periodic): S(m) = sum_u q_u e^{-i bx_u} e^{-i m.theta_u} over the listed modes of
+// the whole box, and out[2u], out[2u + 1] = e^{i bx_u} sum_m w_m S(m) e^{i m.theta_u}; run() only.
 struct FourierSum {
     int n = 0, n_modes = 0, n_lt = 0, n_units = 0, blocks = 0, tp = 32;
     int dim_i = 0, dim_j = 0, dim_k = 0;  // largest |i|, |j|, |k|
     DevBuf theta, w, lines, line_m0, info, units, Sp, S;
+    DevBuf bx;
     const double *theta_d = nullptr, *w_d = nullptr;
     const int4 *lines_d = nullptr;
     const int *line_m0_d = nullptr;
@@ -117,16 +121,6 @@ struct NufftFarField {
     void setup(const std::vector<double> &theta_host, int n_points, int ms_, int mt_, int mu_,
                const std::vector<int> &mode_ijk, const std::vector<double> &mode_w, int width);
     void run(const double *d_q, double *d_out, hipStream_t s) const;  // enqueue only
-};
-
-// Quasi-periodic far field, exact (all N x modes products): wave vectors 2 pi U^{-T} m + b
-// over the full mode box, complex output added to an interleaved (Re, Im) array.
-struct QpFarField {
-    int n = 0, ms = 0, mt = 0, mu = 0, M = 0, nblk = 0, tp = 0;
-    DevBuf theta, bx, w, Sp, S;
-    void setup(const std::vector<double> &theta_host, const std::vector<double> &bx_host, int n_points, int ms_,
-               int mt_, int mu_, const std::vector<double> &w_full);
-    template <class R> void run(const double *d_q, R *d_out, hipStream_t s) const;  // enqueue only
 };
 
 // Launch shapes of evaluate() the autotuner chooses among (0 / -1 = the built-in rule).
@@ -182,6 +176,8 @@ struct Plan {
     // evaluate() on the caller's stream only (the stages one after another): for callers that
     // run many trees side by side, where the trees, not the stages, fill the GPU
     bool single_stream = false;
+    // elements of one vector's proxies, plane waves and child -> parent scratch
+    long long st_up = 0, st_down = 0, st_pw = 0, st_pin = 0, st_c2p = 0;
     Real *c2p_buffer() { return pw_by_level ? pw_out.template as<Real>() : c2p_scratch.template as<Real>(); }
     DevBuf mats_rm;                         // parent <-> child matrices: [transposed][minus / plus][p][p]
     // plane waves
@@ -280,17 +276,23 @@ struct Plan {
     void autotune(int repeats, double *ms_default, double *ms_tuned);
 
     // Quasi-periodic evaluate (bloch given at construction): d_out holds 2N Real, (Re, Im)
-    // per point in user order.  Two passes of the proxy / plane-wave chain and the near field
-    // (charges times the real, then the imaginary part of each image's phase), the self
-    // correction on the real part, then the quasi-periodic far field.
+    // per point in user order.  The charges times the real and the imaginary part of each image's
+    // phase are two real vectors: one near-field launch for both, the proxy / plane-wave chain
+    // for qp_nv vectors per launch (2 below p = 28 when a second set of chain buffers fits, else
+    // one after the other), beside the quasi-periodic far field on s_far; the self correction
+    // goes to the real part.
     bool qp = false;
     double bloch[3] = {0, 0, 0};
+    int qp_nv = 1;
     DevBuf src_phase;   // (cos, sin) of b.R per sorted source (R: the image's lattice translation)
-    QpFarField qpf;
-    int qp_comp = -1;   // component of the pass in progress (-1: not quasi-periodic)
+    DevBuf qp_src;      // the sources twice (nsall + NF_CHUNK + 1 apart), one copy per component
+    FourierSum qpf;
+    DevBuf qp_far;      // complex far field, user order
     DevBuf pot_dev2;    // 2N Real for the host-buffer path
     void evaluate_complex(const double *d_q, Real *d_out, hipStream_t s, int stages = 15);
     void evaluate_complex_host(const double *q, Real *out);
+    // near-field launch (pair: both components of a quasi-periodic tree, from qp_src)
+    void near_field(hipStream_t s, int wpb, bool pair = false);
 
     // Per-kernel-group timing with HIP events on the stream each group runs on (start and
     // end event per group).  Groups: 0 far field, 1 charge gather, 2 proxy/plane-wave
