@@ -1509,137 +1509,159 @@ __global__ __launch_bounds__(EV_THREADS) void k_eval_targets(const R *__restrict
     }
 }
 
-// The same evaluation on the FP64 matrix cores, for p >= 28.  Per leaf and stage of
-// targets
-//   R[t, (c, b)] = sum_a T_a(x_t) C[(c, b), a]          (GEMM, a padded to 16s)
+// The same evaluation on the matrix cores, for p >= 18.  Per leaf and stage of targets
+//   R[t, (c, b)] = sum_a T_a(x_t) C[(c, b), a]          (GEMM, a padded to 4s)
 //   pot_t += sum_(c,b) R[t, (c, b)] T_b(y_t) T_c(z_t)
-// with v_mfma_f64_16x16x4f64 (operand layout as in k_charge2proxy_mfma: A[l % 16][l / 16],
-// B[l / 16][l % 16], D[l / 16 + 4 r][l % 16]).  Wave w takes the (c, b) tiles w, w + NW, ...,
-// whose B operands stay in registers for the whole leaf; each stage runs the TT target tiles
-// as independent accumulators.  Lane partials are reduced over each 16-lane row, then over
-// the waves in a fixed order.  (Reloading the B operands per stage of 64 targets read each
-// leaf's proxy 4 times: 1846 us at N=1e6, 9 digits.)  At p = 38 a wave's B operands would not
-// fit its registers: the leaf's (c, b) tiles are taken in RH = 2 halves, each half a pass over
-// the leaf's targets that adds its part of the sum to the potentials.
-template <int P> struct EvMfmaCfg {
+// with 16 x 16 x 4 products (Mfma16).  Wave w takes the (c, b) tiles w, w + NW, ..., whose B
+// operands (the leaf's proxy rows) stay in registers for the whole leaf, so the proxy is read
+// once per leaf, all its loads in flight together; the targets pass by in stages of TT tiles of
+// 16.  Lane partials are reduced over each 16-lane row (halving the values with each exchange),
+// then over the waves in a fixed order.  At p = 38 a wave's B operands would not fit its
+// registers: the leaf's (c, b) tiles are taken in RH = 2 halves, each a pass over the leaf's
+// targets that adds its part of the sum to the potentials.
+// At p = 18 the vector kernel ran 18 dependent plane loads per leaf and took vector issue from
+// the near field beside it.  Alone, FP32 / FP64: N = 1e3 48 / 69 -> 6 / 7 us, 3e4 88 / 131 ->
+// 14 / 22, 2.5e5 164 / 332 -> 63 / 124, 1e6 256 / 492 -> 180 / 382.  What bounds it now: the
+// matrix cores at about half their rate, then the stages' serial parts (tables, reduction).
+template <int CTRL> __device__ __forceinline__ float row_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double row_dpp(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xF, 0xF, true);
+    const unsigned hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+// a = the lane's and its partner's a (upper lanes of each pair: b)
+template <int CTRL, class R> __device__ __forceinline__ void row_fold(R &a, const R &b, int upper) {
+    const R keep = upper ? +b : +a, give = upper ? +a : +b;
+    a = keep + row_dpp<CTRL>(give);
+}
+template <class R, int P> struct EvMfmaCfg {
     static constexpr int RT = (P * P + 15) / 16;
-    static constexpr int NW = 8;
-    static constexpr int RH = P >= 38 ? 2 : 1;              // passes over the leaf's targets
+    // (4 waves and more passes: two workgroups per CU, one's table building and reduction beside
+    // the other's products; N = 1e6: 9 digits 1220 us with 7 waves in one pass, 1094 with 4 in
+    // two; 12 digits 3781 us with 8 waves in two passes, 2994 with 4 in four)
+    static constexpr int NW = 4;
+    static constexpr int RH = P >= 38 ? 4 : (P >= 28 ? 2 : 1);  // passes over the leaf's targets
     static constexpr int MT = (RT + NW * RH - 1) / (NW * RH);  // (c, b) tiles per wave and pass
-    static constexpr int TT = 2;                   // target tiles per stage
+    static constexpr int TT = P < 28 ? 2 : 2;   // target tiles per stage
     static constexpr int NT = 16 * TT;             // targets per stage
-    static constexpr int PA = (P + 15) / 16 * 16;
-    // LDS row strides, in elements: the A reads (16 targets x 2 a per half wavefront) at a
-    // stride of 34 and the T_b / T_c reads (2 targets x 16 (c, b) columns) at 48 fall on
-    // distinct banks; the stride of 32 put the 16 targets of an A read on the same banks
-    // (measured at N=1e6, 9 digits: 3.3x fewer LDS bank-conflict cycles, 20% fewer busy
-    // cycles; an XOR-swizzled layout removed more conflicts but its address arithmetic cost
-    // more than it saved)
-    static constexpr int LX = PA + 2, LY = 48;
+    static constexpr int PA = (P + 3) / 4 * 4;
+    // LDS row strides, in elements, for the A reads (16 targets x 2 a per half wavefront) and
+    // the T_b / T_c reads (2 targets x 16 (c, b) columns): FP64 rows of 34 and 48 measured 3.3x
+    // fewer bank-conflict cycles than 32 (16 targets on the same banks); FP32 rows of odd length
+    static constexpr int LX = sizeof(R) == 8 ? (PA + 15) / 16 * 16 + 2 : PA + 1;
+    static constexpr int LY = sizeof(R) == 8 ? (P > 24 ? 48 : 24) : 19 + (P > 19 ? 32 : 0);
     static_assert(P <= LY, "order above the table stride");
 };
-// One workgroup per leaf.  Wave w owns the (c, b) tiles w, w + NW, ...: their B operands
-// (the leaf's proxy rows) are loaded into registers once per leaf, and the targets pass by
-// in stages of NT, so the proxy is read from memory once per leaf.
-template <int P>
-__global__ __launch_bounds__(64 * EvMfmaCfg<P>::NW) void k_eval_targets_mfma(
-    const double *__restrict__ down_base, const int *__restrict__ leaf_down, const double *__restrict__ leaf_geom,
-    const int *__restrict__ leaf_trg, const P4<double> *__restrict__ trg, double *__restrict__ pot_sorted) {
+template <class R, int P>
+__global__ __launch_bounds__((64 * EvMfmaCfg<R, P>::NW), 2) void k_eval_targets_mfma(
+    const R *__restrict__ down_base, const int *__restrict__ leaf_down, const R *__restrict__ leaf_geom,
+    const int *__restrict__ leaf_trg, const P4<R> *__restrict__ trg, R *__restrict__ pot_sorted, long long vs_in = 0,
+    long long vs_out = 0) {
     chain_priority();
-    using C = EvMfmaCfg<P>;
+    using C = EvMfmaCfg<R, P>;
+    using M = Mfma16<R>;
     constexpr int RT = C::RT, NW = C::NW, RH = C::RH, MT = C::MT, TT = C::TT, NT = C::NT, PA = C::PA, PP = P * P;
     static_assert(P <= PA, "order above the padded a count");
+    static_assert(TT == 2, "the row reduction halves 8 values");
     constexpr int LX = C::LX, LY = C::LY;
-    __shared__ double Tx[NT * LX], Ty[NT * LY], Tz[NT * LY], red[NW * NT];
+    __shared__ R Tx[NT * LX], Ty[NT * LY], Tz[NT * LY], red[NW * NT];
+    down_base += (long long)blockIdx.z * vs_in;  // vector blockIdx.z of a many-vector launch
+    pot_sorted += (long long)blockIdx.z * vs_out;
     const int lf = blockIdx.x, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kk = lane >> 4, jj = lane & 15;
-    const double *Cm = down_base + (size_t)leaf_down[lf] * P * PP;
-    const double cx = leaf_geom[4 * lf], cy = leaf_geom[4 * lf + 1], cz = leaf_geom[4 * lf + 2], sc = leaf_geom[4 * lf + 3];
+    const R *Cm = down_base + (size_t)leaf_down[lf] * P * PP;
+    const R cx = leaf_geom[4 * lf], cy = leaf_geom[4 * lf + 1], cz = leaf_geom[4 * lf + 2], sc = leaf_geom[4 * lf + 3];
     const int beg = leaf_trg[2 * lf], cnt = leaf_trg[2 * lf + 1];
     for (int h = 0; h < RH; ++h) {
         // B operands of tile rt = w + NW (h MT + m): lane (kk, jj) supplies C[rt 16 + jj][4 ks + kk]
-        double B[MT][PA / 4];
+        R B[MT][PA / 4];
+        int ob[MT], oc[MT];  // table offsets of its (c, b)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const int row = (w + NW * (h * MT + m)) * 16 + jj;
+            oc[m] = row < PP ? row / P : 0;
+            ob[m] = row < PP ? row % P : 0;
 #pragma unroll
             for (int ks = 0; ks < PA / 4; ++ks) {
                 const int a = 4 * ks + kk;
-                B[m][ks] = (row < PP && a < P) ? Cm[(size_t)row * P + a] : 0.0;
+                B[m][ks] = (row < PP && a < P) ? Cm[(size_t)row * P + a] : R(0);
             }
         }
         for (int t0 = 0; t0 < cnt; t0 += NT) {
             __syncthreads();
             for (int task = threadIdx.x; task < 3 * NT; task += blockDim.x) {
                 const int t = task % NT, d = task / NT;
-                double *T = d == 0 ? Tx + t * LX : (d == 1 ? Ty + t * LY : Tz + t * LY);
+                R *T = d == 0 ? Tx + t * LX : (d == 1 ? Ty + t * LY : Tz + t * LY);
                 const int len = d == 0 ? PA : P;
                 if (t0 + t < cnt) {
-                    const P4<double> pt = trg[beg + t0 + t];
-                    const double x = sc * (d == 0 ? pt.x - cx : (d == 1 ? pt.y - cy : pt.z - cz));
-                    double ta = 1.0, tb = x;
-                    T[0] = 1.0;
+                    const P4<R> pt = trg[beg + t0 + t];
+                    const R x = sc * (d == 0 ? pt.x - cx : (d == 1 ? pt.y - cy : pt.z - cz));
+                    R ta = R(1), tb = x;
+                    T[0] = R(1);
                     T[1] = x;
                     for (int k = 2; k < P; ++k) {
-                        const double tn = 2.0 * x * tb - ta;
+                        const R tn = R(2) * x * tb - ta;
                         T[k] = tn;
                         ta = tb;
                         tb = tn;
                     }
-                    for (int k = P; k < len; ++k) T[k] = 0.0;
+                    for (int k = P; k < len; ++k) T[k] = R(0);
                 } else {
-                    for (int k = 0; k < len; ++k) T[k] = 0.0;
+                    for (int k = 0; k < len; ++k) T[k] = R(0);
                 }
             }
             __syncthreads();
-            double A[TT][PA / 4];
+            R A[TT][PA / 4];
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                 for (int ks = 0; ks < PA / 4; ++ks) A[tt][ks] = Tx[(tt * 16 + jj) * LX + 4 * ks + kk];
-            double part[TT][4];
+            R part[4 * TT];
 #pragma unroll
-            for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) part[tt][e] = 0.0;
+            for (int e = 0; e < 4 * TT; ++e) part[e] = R(0);
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
                 const int rt = w + NW * (h * MT + m);
                 if (rt >= RT) break;  // wave-uniform
-                const int row = rt * 16 + jj;  // (c, b) of the B column this lane supplies
-                c2p_d4 D[TT];
+                typename M::acc_t D[TT];
 #pragma unroll
-                for (int tt = 0; tt < TT; ++tt) D[tt] = c2p_d4{0.0, 0.0, 0.0, 0.0};
+                for (int tt = 0; tt < TT; ++tt) D[tt] = typename M::acc_t{R(0), R(0), R(0), R(0)};
 #pragma unroll
                 for (int ks = 0; ks < PA / 4; ++ks)
 #pragma unroll
-                    for (int tt = 0; tt < TT; ++tt)
-                        D[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[tt][ks], B[m][ks], D[tt], 0, 0, 0);
-                // D[tt][e] = R[target tt 16 + kk + 4 e, (c, b) = rt 16 + jj]
-                const int cb = row < PP ? row : 0, c = cb / P, b = cb % P;
+                    for (int tt = 0; tt < TT; ++tt) D[tt] = M::mma(A[tt][ks], B[m][ks], D[tt]);
+                // D[tt][e] = R[target tt 16 + M::row(kk, e), (c, b) = rt 16 + jj]
 #pragma unroll
                 for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const int t = tt * 16 + kk + 4 * e;
-                        part[tt][e] = fma(D[tt][e], Ty[t * LY + b] * Tz[t * LY + c], part[tt][e]);
+                        const int t = tt * 16 + M::row(kk, e);
+                        part[4 * tt + e] =
+                            fma(D[tt][e], Ty[t * LY + ob[m]] * Tz[t * LY + oc[m]], part[4 * tt + e]);
                     }
             }
-            // sum over the 16 lanes of each row (the (c, b) columns), then over the waves
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    double v = part[tt][e];
-#pragma unroll
-                    for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 16);
-                    if (jj == 0) red[w * NT + tt * 16 + kk + 4 * e] = v;
-                }
+            // sum over the 16 lanes of each row (the (c, b) columns): 8 values per lane, halved with
+            // each of three exchanges (partners i ^ 15, i ^ 7, i ^ 3, then i ^ 1: DPP moves); lane
+            // jj ends with value 4 tt + e = jj / 2.  (Unary pluses: a conditional between array
+            // elements would select their addresses.)
+            row_fold<0x140>(part[0], part[4], jj & 8);
+            row_fold<0x140>(part[1], part[5], jj & 8);
+            row_fold<0x140>(part[2], part[6], jj & 8);
+            row_fold<0x140>(part[3], part[7], jj & 8);
+            row_fold<0x141>(part[0], part[2], jj & 4);
+            row_fold<0x141>(part[1], part[3], jj & 4);
+            row_fold<0x1B>(part[0], part[1], jj & 2);
+            part[0] += row_dpp<0xB1>(part[0]);
+            if ((jj & 1) == 0) red[w * NT + (jj >> 3) * 16 + M::row(kk, (jj >> 1) & 3)] = part[0];
             __syncthreads();
             for (int t = threadIdx.x; t < NT; t += blockDim.x) {
                 if (t0 + t < cnt) {
-                    double v = 0;
+                    R v = R(0);
+#pragma unroll
                     for (int q = 0; q < NW; ++q) v += red[q * NT + t];
                     pot_sorted[beg + t0 + t] += v;
                 }
@@ -2603,7 +2625,7 @@ __global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restric
                 if (p0 + pp < n) sincos(bx[p0 + pp], &sn, &cs);
                 const double qp = p0 + pp < n ? q[p0 + pp] : 0.0;
                 Qs[0][pp] = qp * cs;
-                Qs[1][pp] = -qp * sn;
+                Qs[CPLX][pp] = -qp * sn;
                 continue;
             }
             Qs[v][pp] = p0 + pp < n && v0 + v < nv ? q[(long long)(v0 + v) * vs_q + p0 + pp] : 0.0;
@@ -2618,7 +2640,7 @@ __global__ __launch_bounds__(256, 2) void k_ff_structure(const double *__restric
             double qq[V];
 #pragma unroll
             for (int v = 0; v < V; ++v) qq[v] = Qs[v][p];
-            const double qi = CPLX ? Qs[1][p] : 0.0;
+            const double qi = CPLX ? Qs[CPLX][p] : 0.0;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 b[u] = tr[oc[u]];

@@ -117,11 +117,16 @@ template <class Real> size_t near_parts_lds(int S, int ne_max, int pair = 1) {
 
 // Waves per item of the row near field.  Alone, 6 digits FP32 / FP64, one wave per item against
 // 4 and 8: 64 items (N = 1e3) 50 / 59 us, 40 / 43, 36 / 39; 192 items (1e4) 174 / 242 us,
-// 86 / 117, 73 / 96; 512 items (3e4) 152 / 212, 82 / 111, 75 / 110; 2048 items (1.2e5) 329 / 511,
-// 247 / 413, 258 / 453; 4096 items (2.5e5) 206 / 331, 224 / 500, -: one wave from 2560 items on,
-// 8 up to 256, within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or 8 forces a count).
-template <class Real> int near_parts(int n_items, int ne_max, int pair) {
-    int S = n_items <= 256 ? 8 : (n_items < 2560 ? 4 : 1);
+// 86 / 117, 73 / 96; 512 items (3e4) 152 / 212, 82 / 111, 75 / 110; 1024 items (6e4) 167 / 243,
+// 118 / 181, 115 / 187; 2048 items (1.2e5) 329 / 511, 247 / 413, 258 / 453; 4096 items (2.5e5)
+// 206 / 331, 224 / 500, -.  Beside the chain the extra waves cost it more than the near field
+// gains from about 2000 items on (2249 items, FP64: near field 793 -> 682 us, evaluate() 810 ->
+// 843): 8 waves up to 256 items, 4 up to 1280 (2560 for quasi-periodic trees, whose near field
+// forms both components: N = 1e5, 1834 items, 1017 -> 867 us per call), within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or
+// 8 forces a count).
+template <class Real> int near_parts(int n_items, int ne_max, bool qp) {
+    const int pair = qp && std::is_same<Real, float>::value ? 2 : 1;
+    int S = n_items <= 256 ? 8 : (n_items <= (qp ? 2560 : 1280) ? 4 : 1);
     if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
         const int v = std::atoi(e);
         S = v >= 8 ? 8 : (v >= 4 ? 4 : 1);
@@ -659,13 +664,19 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     {
         std::vector<int> ld, lt;
         std::vector<Real> lg;
+        // a leaf's targets in pieces of at most 1/1024 of all targets (whole stages of 32), so that
+        // a few large leaves do not set the time (N = 3e4, 6 digits: 9 of 449 leaves hold 440
+        // targets, the others 60: 44 -> 14 us)
+        const int piece = std::max(32, (n / 1024 + 31) / 32 * 32);
         for (int b = 0; b < nboxes; ++b) {
             if (!(t.tpeval[b] && t.trg_count[b] > 0)) continue;
-            ld.push_back(down_of[b]);
-            for (int d = 0; d < 3; ++d) lg.push_back(Real(0));  // targets are relative to this leaf's centre
-            lg.push_back((Real)(2.0 / t.boxsize[t.level[b]]));
-            lt.push_back(t.trg_begin[b]);
-            lt.push_back(t.trg_count[b]);
+            for (int t0 = 0; t0 < t.trg_count[b]; t0 += piece) {
+                ld.push_back(down_of[b]);
+                for (int d = 0; d < 3; ++d) lg.push_back(Real(0));  // targets are relative to this leaf's centre
+                lg.push_back((Real)(2.0 / t.boxsize[t.level[b]]));
+                lt.push_back(t.trg_begin[b] + t0);
+                lt.push_back(std::min(piece, t.trg_count[b] - t0));
+            }
             work.transform_flops += 2.0 * (double)P3 * t.trg_count[b];
         }
         n_leaf_eval = (int)ld.size();
@@ -854,7 +865,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             check(hipMemGetInfo(&mem_free, &mem_total), "hipMemGetInfo");
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
             if (nf_rows) {
-                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, qp && std::is_same<Real, float>::value ? 2 : 1);
+                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, qp);
                 if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c);
             }
         }
@@ -1419,12 +1430,20 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
                                        pl.t3_mfma, nv, B.s_down, B.s_down);
     }
     if (pl.n_leaf_eval > 0) {
-        if constexpr (std::is_same_v<Real, double> && P >= 28) {
-            hipLaunchKernelGGL((k_eval_targets_mfma<P>), dim3(pl.n_leaf_eval), dim3(64 * EvMfmaCfg<P>::NW), 0, s, B.down,
-                               pl.leaf_down.template as<int>(), pl.leaf_geom.template as<Real>(),
-                               pl.leaf_trg.template as<int>(), pl.trg.template as<P4<Real>>(), B.pot);
-            check(hipGetLastError(), "k_eval_targets_mfma");
-        } else {
+        // Quasi-periodic FP32 trees keep the vector kernel: evaluate_complex hands their values out
+        // as FP64 numbers, which stay the same to the last bit.
+        constexpr bool kMfma = P >= 18 && (P <= 18 || std::is_same_v<Real, double>);
+        bool mfma = kMfma;
+        if constexpr (std::is_same_v<Real, float>) mfma = kMfma && !pl.qp;
+        if (mfma) {
+            if constexpr (kMfma) {
+                hipLaunchKernelGGL((k_eval_targets_mfma<Real, P>), dim3(pl.n_leaf_eval, 1, nv),
+                                   dim3(64 * EvMfmaCfg<Real, P>::NW), 0, s, B.down, pl.leaf_down.template as<int>(),
+                                   pl.leaf_geom.template as<Real>(), pl.leaf_trg.template as<int>(),
+                                   pl.trg.template as<P4<Real>>(), B.pot, B.s_down, B.s_pot);
+                check(hipGetLastError(), "k_eval_targets_mfma");
+            }
+        } else if constexpr (!(kMfma && std::is_same_v<Real, double>)) {
             hipLaunchKernelGGL((k_eval_targets<Real, P>), dim3(pl.n_leaf_eval, 1, nv), dim3(EV_THREADS), 0, s, B.down,
                                pl.leaf_down.template as<int>(), pl.leaf_geom.template as<Real>(),
                                pl.leaf_trg.template as<int>(), pl.trg.template as<P4<Real>>(), B.pot, B.s_down, B.s_pot);
