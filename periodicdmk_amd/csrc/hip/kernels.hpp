@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "dpp_fma.hpp"
 
@@ -137,119 +138,6 @@ __global__ void k_finalize(const R *__restrict__ pot_sorted, const R *__restrict
     pot[u] = (R)v;
 }
 
-// ------------------------------------------------------------------ upward pass
-// One workgroup per destination box:
-//   C[c][b][a] = sum_s T_a(x_s) T_b(y_s) T_c(z_s) q_s,  x_s = sc (r_s - centre).
-// Sources hold coordinates relative to their leaf centre; each range lies in one leaf and
-// carries rng_off = leaf centre - box centre, so x_s = sc (local_s + off).  Per tile of
-// C2P_TS sources the Chebyshev values are tabulated in LDS (q folded into T_c); thread
-// (c, bb) then owns the RB x P output block C[c][bb RB .. bb RB + RB - 1][0 .. P-1] in
-// registers, so each source costs RB P FMAs per thread against ceil(P/4) + 2 LDS reads.
-constexpr int C2P_TS = 64;
-
-// register block RB (b values per thread) and workgroup size per order; output blocks beyond
-// one workgroup's threads are processed in further passes over the sources
-template <int P> struct C2pCfg {
-    // (RB 2 at P = 18: 162 columns, 3 wavefronts per box instead of 2 with RB 3; the 6-digit chain
-    // alone at N=1e6 1.21 -> 1.12 ms in FP32, 1.87 -> 1.62 ms in FP64, the sums unchanged)
-    static constexpr int RB = P >= 18 ? 2 : 3;
-    static constexpr int NB = (P + RB - 1) / RB;
-    static constexpr int cols = NB * P;
-    static constexpr int threads = P >= 38 ? 256 : (cols + 63) / 64 * 64;
-};
-
-template <class R, int P>
-__global__ __launch_bounds__(C2pCfg<P>::threads) void k_charge2proxy(
-    const P4<R> *__restrict__ src, const int *__restrict__ grp_slot, const R *__restrict__ grp_geom,
-    const int *__restrict__ grp_rng, const int *__restrict__ rng_begin, const int *__restrict__ rng_count,
-    const R *__restrict__ rng_off, R *__restrict__ proxy, const R *__restrict__ qv = nullptr, int qv_ld = 0,
-    long long vs_out = 0, long long vs_src = 0) {
-    chain_priority();
-    src += (long long)blockIdx.z * vs_src;  // (vectors with copies of the sources of their own)
-    constexpr int RB = C2pCfg<P>::RB, NB = C2pCfg<P>::NB, NT = C2pCfg<P>::threads;
-    // many-vector launch: vector blockIdx.z takes its charges from qv[source * qv_ld + v]
-    // (src[].w otherwise) and writes its own proxy array, vs_out elements further on
-    proxy += (long long)blockIdx.z * vs_out;
-    constexpr int PX = (P + 3) & ~3, PY = NB * RB;  // padded table rows
-    __shared__ R Tx[C2P_TS * PX], Ty[C2P_TS * PY], Tz[C2P_TS * P];
-    const int g = blockIdx.x;
-    const R sc = grp_geom[4 * g + 3];
-    for (int col0 = 0; col0 < NB * P; col0 += NT) {
-        const int col = col0 + (int)threadIdx.x;
-        const int c = col / NB, bb = col - c * NB;
-        const bool active = col < NB * P;
-        R acc[RB][P];
-#pragma unroll
-        for (int j = 0; j < RB; ++j)
-#pragma unroll
-            for (int a = 0; a < P; ++a) acc[j][a] = R(0);
-        for (int r = grp_rng[g]; r < grp_rng[g + 1]; ++r) {
-            const int beg = rng_begin[r], cnt = rng_count[r];
-            for (int s0 = 0; s0 < cnt; s0 += C2P_TS) {
-                const int ns = min(C2P_TS, cnt - s0);
-                __syncthreads();
-                for (int t = threadIdx.x; t < 3 * C2P_TS; t += NT) {
-                    const int s = t % C2P_TS, d = t / C2P_TS;
-                    R *T = d == 0 ? Tx + s * PX : (d == 1 ? Ty + s * PY : Tz + s * P);
-                    const int len = d == 0 ? PX : (d == 1 ? PY : P);
-                    if (s < ns) {
-                        const P4<R> pt = src[beg + s0 + s];
-                        const R x = sc * ((d == 0 ? pt.x : (d == 1 ? pt.y : pt.z)) + rng_off[4 * r + d]);
-                        const R m = (d == 2) ? (qv ? qv[(size_t)(beg + s0 + s) * qv_ld + blockIdx.z] : pt.w) : R(1);
-                        R t0 = m, t1 = x * m;
-                        T[0] = t0;
-                        if (P > 1) T[1] = t1;
-                        for (int k = 2; k < P; ++k) {
-                            const R t2 = R(2) * x * t1 - t0;
-                            T[k] = t2;
-                            t0 = t1;
-                            t1 = t2;
-                        }
-                        for (int k = P; k < len; ++k) T[k] = R(0);
-                    } else {
-                        for (int k = 0; k < len; ++k) T[k] = R(0);
-                    }
-                }
-                __syncthreads();
-                if (active) {
-                    for (int s = 0; s < ns; ++s) {
-                        R tx[P];
-#pragma unroll
-                        for (int a = 0; a < P; ++a) tx[a] = Tx[s * PX + a];
-                        const R z = Tz[s * P + c];
-#pragma unroll
-                        for (int j = 0; j < RB; ++j) {
-                            const R w = Ty[s * PY + bb * RB + j] * z;
-#pragma unroll
-                            for (int a = 0; a < P; ++a) acc[j][a] = fma(tx[a], w, acc[j][a]);
-                        }
-                    }
-                }
-            }
-        }
-        if (active) {
-            R *out = proxy + (size_t)grp_slot[g] * (P * P * P) + (size_t)P * P * c;
-#pragma unroll
-            for (int j = 0; j < RB; ++j) {
-                const int b = bb * RB + j;
-                if (b < P)
-#pragma unroll
-                    for (int a = 0; a < P; ++a) out[a + P * b] = acc[j][a];
-            }
-        }
-    }
-}
-
-// The same proxy charges on the FP64 matrix cores, for p >= 28.  Per destination box
-//   C[(c, b), a] = sum_s A[(c, b), s] B[s, a],  A = q_s T_c(z_s) T_b(y_s),  B = T_a(x_s),
-// is a GEMM of P^2 rows by PA columns (a padded to 16s) over the box's sources, computed with
-// v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and holds
-// D[l / 16 + 4 r][l % 16] in accumulator element r (layout read off gfx950 hardware).  The
-// row tiles of a box are split over RS workgroups; wave w of a workgroup owns its row tiles
-// w, w + NW, ... and every column tile.  Two shapes at p = 28: for trees with many boxes
-// (WIDE) two workgroups of 4 waves per box (7 row tiles per wave, 158 VGPRs: three
-// workgroups share a CU, so one's table building overlaps the others' matrix products);
-// otherwise one workgroup of 16 waves (4 row tiles per wave, 98 VGPRs).
 typedef double c2p_d4 __attribute__((ext_vector_type(4)));
 typedef float c2p_f4 __attribute__((ext_vector_type(4)));
 
@@ -271,107 +159,199 @@ template <> struct Mfma16<float> {
     }
     static __device__ __forceinline__ int row(int kk, int e) { return 4 * kk + e; }
 };
-template <int P, bool WIDE> struct C2pMfmaCfg {
-    static constexpr int RT = (P * P + 15) / 16;                  // row tiles
-    static constexpr int RS = P >= 38 || WIDE ? 2 : 1;            // workgroups per box
-    static constexpr int RTS = (RT + RS - 1) / RS;                // row tiles per workgroup
-    static constexpr int NW = WIDE ? 4 : (P >= 38 ? 8 : 16);      // waves per workgroup
-    static constexpr int TPW = (RTS + NW - 1) / NW;   // row tiles per wave
-    static constexpr int TS = 64;                     // sources per LDS table
-    static constexpr int PA = (P + 15) / 16 * 16;     // a, padded
-    static constexpr int CT = PA / 16;                // column tiles
-    // LDS row strides of the tables (odd numbers of doubles: a thread writing its source's row
-    // and the 4 sources of a fragment read fall on different banks; PA and P put them on one)
-    static constexpr int SX = PA + 1, SY = P % 2 ? P : P + 1;
+// ------------------------------------------------------------------ upward pass
+// One destination box per workgroup (or per `parts` workgroups):
+//   C[c][b][a] = sum_s T_a(x_s) T_b(y_s) T_c(z_s) q_s,  x_s = sc (r_s - centre).
+// Sources hold coordinates relative to their leaf centre; each range lies in one leaf and
+// carries rng_off = leaf centre - box centre, so x_s = sc (local_s + off).
+//
+// Per box this is a GEMM of P^2 columns (c, b) by P values of a over the sources, on the matrix
+// cores with 4-wide blocks, which pad a to a multiple of 4 (18 to 20, 28 and 28): the 16-wide
+// products used before at p = 28 pad it to 32, and at p = 18 that waste kept both precisions on
+// the vector ALUs, in competition with the near field.  Each output is the chain of fused
+// multiply-adds over the sources in order, as on the vector ALUs, bit for bit (checked on
+// gfx950: v_mfma_f32_4x4x1 adds one product per step, v_mfma_f64_4x4x4 four in k order).
+//   FP32, v_mfma_f32_4x4x1 (16 blocks): lane l owns column 64 w + l; its factor q T_b T_c of
+//     a source is the B operand, and T_a comes as an A operand that broadcasts one block of 4
+//     lanes to all (cbsz 4), so one register with the T_a of SPA sources serves SPA G products.
+//   FP64, v_mfma_f64_4x4x4 (4 blocks): a tile of 16 columns by 4 values of a over 4 sources;
+//     lane (k, blk, i) = (l / 16, l / 4 % 4, l % 4) supplies A = q T_b T_c of column 4 blk + i and
+//     B = T_(4 g + i), both at source k, and holds D[column 4 blk + l / 16][a = 4 g + i].
+// Box g's sources are items grp_ptr[g] .. (source, range), its ranges without a break (short leaves
+// fill a tile together, and a tile's loads wait for no walk over the ranges); their Chebyshev values are tabulated in LDS, two buffers in turn: the next tile's
+// points load while the current one's products run.
+//
+// Alone, N = 1e6 (576 boxes): FP32 6 digits 305 -> 223 us, FP64 475 -> 355, 9 digits 975 -> 887
+// (evaluate() 6959 -> 6600); N = 3e4 (64 boxes) 72 -> 34,
+// 81 -> 29, 137 -> 69; clustered, 9 digits N = 1e6 7675 -> 7387, 12 digits N = 1.5e5 2246 -> 1118.
+// Bound by the matrix cores and, with 576 boxes for 256 CUs, by the last round of boxes.
+template <class R, int P> struct C2pCfg {
+    static constexpr bool F32 = sizeof(R) == 4;
+    static constexpr int G = (P + 3) / 4, PX = 4 * G;     // groups of 4 values of a
+    static constexpr int CB = P * P;                      // columns (c, b)
+    static constexpr int CW = F32 ? 64 : 16;              // columns of a tile
+    static constexpr int CT = (CB + CW - 1) / CW;         // column tiles
+    // waves per workgroup.  FP64 at p = 28, 38: 4, one per SIMD, and two workgroups or more per CU
+    // (7 waves of 7 tiles: N = 1e6 9 digits 1012 us, clustered 8942; 5 waves: 1304)
+    static constexpr int NW = F32 ? (CT > 16 ? (CT + 1) / 2 : CT) : (P <= 18 ? 7 : 4);
+    static constexpr int parts(int tpw) { return (CT + NW * tpw - 1) / (NW * tpw); }  // workgroups per box
+    static constexpr int SPA = F32 ? 64 / PX : 4;         // sources per A register / product
+    static constexpr int TS = F32 ? 60 / SPA * SPA : 32;  // sources per table
+    // LDS rows: x values, then y and z (odd, so that the rows of a fragment spread over the banks)
+    static constexpr int SX = F32 ? PX : PX + 1, SY = P | 1;
+    static constexpr int buf = TS * (SX + 2 * SY);        // elements of a buffer
+    static constexpr int NTK = (3 * TS + 64 * NW - 1) / (64 * NW);  // table tasks per thread
 };
 
-template <class R, int P, bool WIDE>
-__global__ __launch_bounds__((64 * C2pMfmaCfg<P, WIDE>::NW)) void k_charge2proxy_mfma(
+// items of the ranges: item[rng_ptr[r] + i] = (rng_begin[r] + i, r), a wavefront per range
+__global__ __launch_bounds__(256) void k_c2p_items(const int *__restrict__ rng_begin, const int *__restrict__ rng_count,
+                                                   const int *__restrict__ rng_ptr, int n_rng, int2 *__restrict__ item) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= n_rng) return;
+    const int beg = rng_begin[r], cnt = rng_count[r], o = rng_ptr[r];
+    for (int i = threadIdx.x & 63; i < cnt; i += 64) item[o + i] = make_int2(beg + i, r);
+}
+
+// SPA G products of one A register, its blocks in turn: sources s, values 4 g .. 4 g + 3
+template <int G, int... I>
+__device__ __forceinline__ void c2p_products(float a, const float *w, c2p_f4 *acc, std::integer_sequence<int, I...>) {
+    ((acc[I % G] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w[I / G], acc[I % G], 4, I, 0)), ...);
+}
+
+// TPW: column tiles per wave (FP32: 1); tile (part NW + w) + parts NW m of wave w
+template <class R, int P, int TPW>
+__global__ __launch_bounds__((64 * C2pCfg<R, P>::NW), 2) void k_charge2proxy(
     const P4<R> *__restrict__ src, const int *__restrict__ grp_slot, const R *__restrict__ grp_geom,
-    const int *__restrict__ grp_rng, const int *__restrict__ rng_begin, const int *__restrict__ rng_count,
-    const R *__restrict__ rng_off, R *__restrict__ proxy) {
+    const int *__restrict__ grp_ptr, const int2 *__restrict__ item, const R *__restrict__ rng_off,
+    R *__restrict__ proxy, const R *__restrict__ qv = nullptr, int qv_ld = 0,
+    long long vs_out = 0, long long vs_src = 0) {
     chain_priority();
-    using C = C2pMfmaCfg<P, WIDE>;
-    using M = Mfma16<R>;
-    constexpr int TS = C::TS, PA = C::PA, RT = C::RT, RS = C::RS, RTS = C::RTS, NW = C::NW, TPW = C::TPW, CT = C::CT,
-                  SX = C::SX, SY = C::SY;
-    static_assert(P <= PA, "order above the padded column count");
-    __shared__ R Tx[TS * SX], Ty[TS * SY], Tz[TS * SY];
-    const int g = blockIdx.x / RS, part = blockIdx.x - g * RS, lane = threadIdx.x & 63;
-    const int rt0 = part * RTS, rt1 = min(RT, rt0 + RTS);  // this workgroup's row tiles
+    using C = C2pCfg<R, P>;
+    constexpr int G = C::G, NW = C::NW, TS = C::TS, SX = C::SX, SY = C::SY, SPA = C::SPA, NTK = C::NTK, CB = C::CB;
+    constexpr int parts = C::parts(TPW);
+    constexpr bool F32 = C::F32;
+    static_assert(!F32 || TPW == 1, "one column per lane");
+    // vector blockIdx.z of a launch for several: its sources at src + z vs_src, or its charges at
+    // qv[source * qv_ld + z] (src[].w otherwise); its proxies vs_out elements further on
+    src += (long long)blockIdx.z * vs_src;
+    proxy += (long long)blockIdx.z * vs_out;
+    __shared__ R lds[2 * C::buf];
+    const int g = blockIdx.x / parts, part = blockIdx.x - g * parts, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int kk = lane >> 4, jj = lane & 15;
     const R sc = grp_geom[4 * g + 3];
-    int ci[TPW], bi[TPW];
-    R rv[TPW];
+    // this lane's columns: table offsets of b and c (columns past the last repeat column 0)
+    int ob[TPW], oc[TPW];
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-        const int row = (rt0 + w + NW * t) * 16 + jj;
-        const bool ok = row < P * P;
-        rv[t] = ok ? R(1) : R(0);
-        ci[t] = ok ? row / P : 0;
-        bi[t] = ok ? row % P : 0;
+    for (int m = 0; m < TPW; ++m) {
+        const int col = ((part * NW + w) + parts * NW * m) * C::CW + (F32 ? lane : (lane & 15));
+        ob[m] = col < CB ? col % P : 0;
+        oc[m] = col < CB ? col / P : 0;
     }
-    typename M::acc_t acc[TPW][CT];
+    static_assert(F32 || C::CT > (TPW - 1) * NW * parts, "every wave has its first TPW - 1 tiles");
+    const int nt = (C::CT - (part * NW + w) + parts * NW - 1) / (parts * NW);  // this wave's tiles
+    c2p_f4 accf[F32 ? G : 1];
+    double accd[F32 ? 1 : TPW][F32 ? 1 : G];
+    if constexpr (F32) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t)
+        for (int i = 0; i < G; ++i) accf[i] = c2p_f4{0, 0, 0, 0};
+    } else {
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[t][ct] = typename M::acc_t{R(0), R(0), R(0), R(0)};
-    for (int r = grp_rng[g]; r < grp_rng[g + 1]; ++r) {
-        const int beg = rng_begin[r], cnt = rng_count[r];
-        for (int s0 = 0; s0 < cnt; s0 += TS) {
-            const int ns = min(TS, cnt - s0);
-            __syncthreads();
-            for (int t = threadIdx.x; t < 3 * TS; t += blockDim.x) {
-                const int s = t % TS, d = t / TS;
-                R *T = d == 0 ? Tx + s * SX : (d == 1 ? Ty + s * SY : Tz + s * SY);
-                const int len = d == 0 ? PA : P;
-                if (s < ns) {
-                    const P4<R> pt = src[beg + s0 + s];
-                    const R x = sc * ((d == 0 ? pt.x : (d == 1 ? pt.y : pt.z)) + rng_off[4 * r + d]);
-                    const R m = (d == 2) ? pt.w : R(1);
-                    R t0 = m, t1 = x * m;
-                    T[0] = t0;
-                    T[1] = t1;
-                    for (int k = 2; k < P; ++k) {
-                        const R t2 = R(2) * x * t1 - t0;
-                        T[k] = t2;
-                        t0 = t1;
-                        t1 = t2;
-                    }
-                    for (int k = P; k < len; ++k) T[k] = R(0);
-                } else {
-                    for (int k = 0; k < len; ++k) T[k] = R(0);
-                }
+        for (int m = 0; m < TPW; ++m)
+#pragma unroll
+            for (int i = 0; i < G; ++i) accd[m][i] = 0;
+    }
+    const int i1 = grp_ptr[g + 1];
+    int i0 = grp_ptr[g];  // the next tile's first source
+    R px[NTK], pq[NTK];
+    // next tile's points into registers (task t: component t / TS of source t % TS; past the end:
+    // charge 0)
+    auto fetch = [&]() {
+#pragma unroll
+        for (int i = 0; i < NTK; ++i) {
+            const int t = (int)threadIdx.x + 64 * NW * i, s = t % TS, d = t / TS;
+            px[i] = R(0);
+            pq[i] = R(0);
+            if (i0 + s < i1 && d < 3) {
+                const int2 e = item[i0 + s];
+                const R *x = reinterpret_cast<const R *>(src + e.x);
+                px[i] = x[d] + rng_off[4 * e.y + d];
+                pq[i] = d == 2 ? (qv ? qv[(size_t)e.x * qv_ld + blockIdx.z] : x[3]) : R(1);
             }
-            __syncthreads();
-            for (int k0 = 0; k0 < ns; k0 += 4) {
-                const int s = k0 + kk;
-                R bv[CT];
+        }
+    };
+    auto tabulate = [&](R *T0) {
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct) bv[ct] = Tx[s * SX + 16 * ct + jj];
+        for (int i = 0; i < NTK; ++i) {
+            const int t = (int)threadIdx.x + 64 * NW * i, s = t % TS, d = t / TS;
+            if (d >= 3) break;
+            R *T = d == 0 ? T0 + s * SX : T0 + TS * SX + ((d - 1) * TS + s) * SY;
+            const R x = sc * px[i], m = pq[i];
+            R t0 = m, t1 = x * m;
+            T[0] = t0;
+            T[1] = t1;
 #pragma unroll
-                for (int t = 0; t < TPW; ++t) {
-                    if (rt0 + w + NW * t < rt1) {
-                        const R a = Tz[s * SY + ci[t]] * Ty[s * SY + bi[t]] * rv[t];
+            for (int k = 2; k < P; ++k) {
+                const R t2 = R(2) * x * t1 - t0;
+                T[k] = t2;
+                t0 = t1;
+                t1 = t2;
+            }
+            if (d == 0)
+                for (int k = P; k < C::PX; ++k) T[k] = R(0);
+        }
+    };
+    fetch();
+    for (int it = 0; i0 < i1; ++it) {
+        R *T0 = lds + (it & 1) * C::buf;
+        tabulate(T0);
+        const int cur = min(TS, i1 - i0);
+        i0 += TS;
+        fetch();
+        // (one barrier per tile: a wave that is a tile ahead writes the other buffer, and a buffer is
+        // written again only after the barrier that follows its last reads)
+        __syncthreads();
+        const R *Tx = T0, *Ty = T0 + TS * SX, *Tz = Ty + TS * SY;
+        if constexpr (F32) {
+            for (int s0 = 0; s0 < cur; s0 += SPA) {
+                const float a = Tx[s0 * SX + lane];  // (lanes past SPA rows: in no product's block)
+                float wv[SPA];
 #pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) acc[t][ct] = M::mma(a, bv[ct], acc[t][ct]);
-                    }
+                for (int i = 0; i < SPA; ++i) wv[i] = Ty[(s0 + i) * SY + ob[0]] * Tz[(s0 + i) * SY + oc[0]];
+                c2p_products<G>(a, wv, accf, std::make_integer_sequence<int, SPA * G>{});
+            }
+        } else {
+            const int kk = lane >> 4, j = lane & 3;
+            for (int s0 = 0; s0 < cur; s0 += 4) {
+                const int s = s0 + kk;
+                double b[G];
+#pragma unroll
+                for (int i = 0; i < G; ++i) b[i] = Tx[s * SX + 4 * i + j];
+#pragma unroll
+                for (int m = 0; m < TPW; ++m) {
+                    // (only the last tile of some waves may be past the end; wave-uniform)
+                    if (C::CT % (NW * parts) != 0 && m == TPW - 1 && m >= nt) break;
+                    const double a = Ty[s * SY + ob[m]] * Tz[s * SY + oc[m]];
+#pragma unroll
+                    for (int i = 0; i < G; ++i) accd[m][i] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b[i], accd[m][i], 0, 0, 0);
                 }
             }
         }
     }
     R *out = proxy + (size_t)grp_slot[g] * (P * P * P);
+    if constexpr (F32) {
+        const int col = (part * NW + w) * 64 + lane;
+        if (col < CB) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-        if (rt0 + w + NW * t >= rt1) continue;
+            for (int a = 0; a < P; ++a) out[(size_t)col * P + a] = accf[a >> 2][a & 3];
+        }
+    } else {
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int a = ct * 16 + jj;
+        for (int m = 0; m < TPW; ++m) {
+            const int col = ((part * NW + w) + parts * NW * m) * 16 + (lane & 12) + (lane >> 4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = (rt0 + w + NW * t) * 16 + M::row(kk, e);
-                if (row < P * P && a < P) out[(size_t)row * P + a] = acc[t][ct][e];
+            for (int i = 0; i < G; ++i) {
+                const int a = 4 * i + (lane & 3);
+                if (col < CB && a < P) out[(size_t)col * P + a] = accd[m][i];
             }
         }
     }
@@ -1548,11 +1528,10 @@ template <class R, int P> struct EvMfmaCfg {
     static constexpr int TT = P < 28 ? 2 : 2;   // target tiles per stage
     static constexpr int NT = 16 * TT;             // targets per stage
     static constexpr int PA = (P + 3) / 4 * 4;
-    // LDS row strides, in elements, for the A reads (16 targets x 2 a per half wavefront) and
-    // the T_b / T_c reads (2 targets x 16 (c, b) columns): FP64 rows of 34 and 48 measured 3.3x
-    // fewer bank-conflict cycles than 32 (16 targets on the same banks); FP32 rows of odd length
-    static constexpr int LX = sizeof(R) == 8 ? (PA + 15) / 16 * 16 + 2 : PA + 1;
-    static constexpr int LY = sizeof(R) == 8 ? (P > 24 ? 48 : 24) : 19 + (P > 19 ? 32 : 0);
+    // LDS row strides, in elements: odd, so that the 32 threads that write their targets' rows in
+    // step and the 16 targets of an A read each fall on distinct banks (FP64 rows of 34 and 48:
+    // 16-way conflicts of the writes, 23% of the kernel's LDS time at N = 1e6, 9 digits)
+    static constexpr int LX = PA | 1, LY = P | 1;
     static_assert(P <= LY, "order above the table stride");
 };
 template <class R, int P>

@@ -59,10 +59,8 @@ constexpr size_t kTwoPassBytes = size_t(512) << 20;  // two-pass transform scrat
 // 4.16 ms with one item per parent)
 constexpr int kC2pFuseParents = 256;
 
-// proxy slots from which the charge -> proxy matrix-core kernel (p = 28) takes its wide
-// workgroup shape: 64 boxes per CU (the N=1e6 uniform tree has about 5e3 slots, the
-// clustered N=4e6 one 1.2e5)
-constexpr int kC2pWideBoxes = 16384;
+// proxy slots below which FP64 charge -> proxy takes several workgroups per box
+constexpr int kC2pSplitBoxes = 256;
 
 // f(i0, i1) over contiguous chunks of [0, n) on up to 16 host threads (construction work
 // whose chunks write disjoint data)
@@ -462,10 +460,24 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         for (int k = 0; k < n_up; ++k) rng[k + 1] += rng[k];
         up_slot.upload(slot);
         up_geom.upload(geom);
-        up_rng.upload(rng);
-        rng_begin.upload(rb);
-        rng_count.upload(rcnt);
         rng_off.upload(roff);
+        // sources of every slot, range after range
+        const int n_rng = (int)rb.size();
+        std::vector<int> rptr(n_rng + 1, 0), uptr(n_up + 1, 0);
+        for (int r = 0; r < n_rng; ++r) rptr[r + 1] = rptr[r] + rcnt[r];
+        for (int k = 0; k <= n_up; ++k) uptr[k] = rptr[rng[k]];
+        up_ptr.upload(uptr);
+        up_item.alloc(sizeof(int2) * (size_t)std::max(1, rptr[n_rng]));
+        if (n_rng > 0) {
+            DevBuf d_beg, d_cnt, d_ptr;
+            d_beg.upload(rb);
+            d_cnt.upload(rcnt);
+            d_ptr.upload(rptr);
+            hipLaunchKernelGGL(k_c2p_items, dim3((n_rng + 3) / 4), dim3(256), 0, stream, d_beg.as<int>(), d_cnt.as<int>(),
+                               d_ptr.as<int>(), n_rng, up_item.as<int2>());
+            check(hipGetLastError(), "k_c2p_items");
+            check(hipStreamSynchronize(stream), "k_c2p_items");
+        }
         double c2p_src = 0;
         for (size_t i = 0; i < rcnt.size(); ++i) c2p_src += rcnt[i];
         work.transform_flops += 2.0 * (double)P3 * c2p_src;
@@ -1064,11 +1076,8 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         pw_by_level = all_bytes + (size_t(1) << 30) > free_b;
         if (const char *e = std::getenv("PDMK_PW_LEVELS")) pw_by_level = e[0] == '1';
         if (const char *e = std::getenv("PDMK_T3_MFMA")) t3_mfma = e[0] != '0';
-        // charge -> proxy workgroup shape at p = 28 (same sums either way): clustered N=4e6,
-        // 124,287 slots, 9-digit evaluate() 130.9 -> 126.2 ms with the wide shape; N=1e6
-        // uniform 7.73 -> 7.53 ms with the 16-wave one
-        c2p_wide = n_up >= kC2pWideBoxes;
-        if (const char *e = std::getenv("PDMK_C2P_WIDE")) c2p_wide = e[0] != '0';
+        c2p_split = n_up < kC2pSplitBoxes;
+        if (const char *e = std::getenv("PDMK_C2P_WIDE")) c2p_split = e[0] != '0';
         // grouped shifts at p >= 28 (N=1e6 9 digits: evaluate() 7.57 -> 7.39 ms; clustered
         // N=4e6 132.5 -> 131.1 ms at 9 digits, 412.5 -> 403.1 ms at 12); at p = 18 one box
         // per workgroup stays faster (6 digits: FP32 2.41 against 2.45 ms, FP64 3.87 against
@@ -1286,35 +1295,21 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
     const int nv = B.nv;
     if (nv < 1 || nv > 65535) throw std::invalid_argument("launch_transforms: vector count");
     if (pl.n_up > 0) {
-        // FP64 at P = 28 (9 digits): matrix cores (a padded to 32 costs 1/8).  At P = 38 (a
-        // padded to 48, each box's row tiles split over two workgroups) the matrix-core kernel
-        // ran slower than the vector ALUs (clustered N = 4e6: 90.5 against 78.7 ms).  FP64 at
-        // P = 18 pads too much.  FP32 at P = 18 on the matrix cores is faster alone (395 -> 307 us at
-        // N=1e6) but slower inside evaluate() (3.02 -> 3.24 ms): its 8-wave workgroups take
-        // wave slots from the near field beside it; it stays on the vector ALUs (and the
-        // many-vector chain with it: the same sums in the same order as one vector's).
-        if constexpr (std::is_same_v<Real, double> && P >= 28 && P <= 32) {
-            if (nv != 1 || B.qv) throw std::logic_error("launch_transforms: one vector on the matrix-core kernels");
-            auto c2p = [&](auto wide) {
-                constexpr bool W = decltype(wide)::value;
-                hipLaunchKernelGGL((k_charge2proxy_mfma<Real, P, W>), dim3(pl.n_up * C2pMfmaCfg<P, W>::RS),
-                                   dim3(64 * C2pMfmaCfg<P, W>::NW), 0, s, B.src,
-                                   pl.up_slot.template as<int>(), pl.up_geom.template as<Real>(),
-                                   pl.up_rng.template as<int>(), pl.rng_begin.template as<int>(),
-                                   pl.rng_count.template as<int>(), pl.rng_off.template as<Real>(), B.up);
-                check(hipGetLastError(), "k_charge2proxy_mfma");
-            };
-            if (pl.c2p_wide)
-                c2p(std::true_type{});
-            else
-                c2p(std::false_type{});
-        } else {
-            hipLaunchKernelGGL((k_charge2proxy<Real, P>), dim3(pl.n_up, 1, nv), dim3(C2pCfg<P>::threads), 0, s,
+        auto c2p = [&](auto tpw) {
+            constexpr int TPW = decltype(tpw)::value;
+            using C = C2pCfg<Real, P>;
+            hipLaunchKernelGGL((k_charge2proxy<Real, P, TPW>), dim3(pl.n_up * C::parts(TPW), 1, nv), dim3(64 * C::NW), 0, s,
                                B.src, pl.up_slot.template as<int>(), pl.up_geom.template as<Real>(),
-                               pl.up_rng.template as<int>(), pl.rng_begin.template as<int>(), pl.rng_count.template as<int>(),
+                               pl.up_ptr.template as<int>(), pl.up_item.template as<int2>(),
                                pl.rng_off.template as<Real>(), B.up, B.qv, B.qv_ld, B.s_up, B.s_src);
             check(hipGetLastError(), "k_charge2proxy");
-        }
+        };
+        // FP64: a box's column tiles in 1, 2 or 4 workgroups (p = 18, 28, 38), or in 3, 5 or 8 where
+        // the boxes alone leave CUs idle (64 boxes, N = 3e4: 6 digits 52 -> 29 us, 9 digits 81 -> 69)
+        constexpr bool F64 = std::is_same_v<Real, double>;
+        constexpr int T_FEW = !F64 || P == 9 ? 1 : (P == 18 ? 3 : (P == 28 ? 7 : 6)), T_MANY = !F64 || P <= 18 ? 1 : 3;
+        if (T_MANY != T_FEW && pl.c2p_split) c2p(std::integral_constant<int, T_MANY>{});
+        else c2p(std::integral_constant<int, T_FEW>{});
     }
     for (auto &C : pl.c2p_levels) {
         if (C.fused) {

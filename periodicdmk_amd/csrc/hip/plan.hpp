@@ -155,7 +155,8 @@ struct Plan {
     // O(N) data
     DevBuf src, src_user, trg, trg_user, trg_w0, pot_sorted, pot_near, q_dev, pot_dev, far, far_idx;
     // upward
-    DevBuf up_slot, up_geom, up_rng, rng_begin, rng_count, rng_off, proxy_up;
+    // sources of slot k: up_item[up_ptr[k] ..], (source, range); rng_off: leaf centre - box centre
+    DevBuf up_slot, up_geom, up_ptr, up_item, rng_off, proxy_up;
     struct Tensor3Launch { int n_items; DevBuf out, add, ptr, in_slot, in_code; };
     // child -> parent per level (deepest first): fused = one item per parent adding its children
     // to the parent's proxy; else per-child transforms into c2p_scratch, then
@@ -170,9 +171,9 @@ struct Plan {
     bool pw_by_level = false;
     bool shift_groups = true;  // k_pw_shift_grp (p >= 28; PDMK_SHIFT_GROUPS=0 / 1 forces either)
     bool t3_mfma = true;  // FP64 tensor transforms at p = 28 on the matrix cores (PDMK_T3_MFMA=0: vector ALUs)
-    // the WIDE shape of k_charge2proxy_mfma (two 4-wave workgroups per box) for trees with at
-    // least kC2pWideBoxes proxy slots, else one 16-wave workgroup (PDMK_C2P_WIDE=0 / 1 forces)
-    bool c2p_wide = false;
+    // several workgroups per box in FP64 charge -> proxy, for trees with fewer than
+    // kC2pSplitBoxes proxy slots (the same sums; PDMK_C2P_WIDE=0 / 1 forces)
+    bool c2p_split = false;
     // evaluate() on the caller's stream only (the stages one after another): for callers that
     // run many trees side by side, where the trees, not the stages, fill the GPU
     bool single_stream = false;
