@@ -411,9 +411,11 @@ template <class R, int P, int NPW, int BK = 0> struct P2pwCfg {
 template <class R, int P, int NPW, int BK = 0> struct Pw2pCfg {
     static constexpr int H = (NPW + 1) / 2;
     // (FP64 at p = 28: 2 slices of a per workgroup, 43 KB, so three workgroups share a CU;
-    // 3 per workgroup at 65 KB fit two: N=1e6 9-digit evaluate() 9.12 -> 9.07 ms)
+    // 3 per workgroup at 65 KB fit two: N=1e6 9-digit evaluate() 9.12 -> 9.07 ms.  p = 18: 32 KB in
+    // FP64, 16 KB in FP32 (3 slices): the FP32 chain alone 81 -> 67 us at N = 1e3, 175 -> 152 at 3e4,
+    // 638 -> 576 at 2.5e5; FP64 at 16 KB 75 -> 84 and 817 -> 896)
     static constexpr int AC = tf_slices(P, (H * NPW + H * OddStride<P>::v) * (int)sizeof(Cx<R>), 0,
-                                        BK ? BK * 1024 : ((P == 28 && sizeof(R) == 8) ? 48 * 1024 : (P == 18 ? 32 * 1024 : kTfLdsBytes)));
+                                        BK ? BK * 1024 : ((P == 28 && sizeof(R) == 8) ? 48 * 1024 : (P == 18 ? (int)sizeof(R) * 4096 : kTfLdsBytes)));
     static constexpr int slices = (P + AC - 1) / AC;
     // the y and z steps have AC H and AC P columns of P outputs for 256 threads; the outputs of
     // a column are split over SGY / SGZ wavefronts when that fills more of them
