@@ -310,7 +310,8 @@ class PDMKSolver:
             rc = lib().pdmk_evaluate_complex_double(self._h, self.n, C.POINTER(C.c_double)(), _d(q), _d(out))
         if rc != 0:
             raise RuntimeError("pdmk_evaluate_complex failed (see stderr)")
-        return out[0::2].astype(np.float64) + 1j * out[1::2].astype(np.float64)
+        pairs = out.view(np.complex64 if self.precision == "float" else np.complex128)  # (Re, Im) per point
+        return pairs.astype(np.complex128, copy=False)
 
     def run_complex_stages(self, charges, stages: int):
         """Quasi-periodic, device path, selected stages only (bits as in STAGE_*)."""
