@@ -1977,6 +1977,9 @@ __global__ __launch_bounds__(256) void k_near_rows_build(
     if (PASS == 0 && lane == 0) atomicAdd(pairs, np);
 }
 
+// float4 of a list entry's geometry in k_near_rows' LDS
+template <int NC, bool SPLIT> __host__ __device__ constexpr int nf_geo_f4() { return SPLIT ? 1 + (NC + 3) / 4 : 2; }
+
 // Residual evaluation over the row step lists (FP32, NC coefficients in the x form).  Row g
 // of item i lists its non-empty entries in slots rslot[(rs_base[i] + s) * 16 + g] =
 // (end step << 8) | ordinal of the entry in the target leaf's list1, followed by a terminator
@@ -1994,14 +1997,18 @@ __global__ __launch_bounds__(256) void k_near_rows_build(
 // V = 2 (quasi-periodic): the residual formed once for two charges, the second from the copy of
 // the sources vs_src further on (potentials vs_pot further on); each component's sums are those
 // of V = 1.  (N = 1e5, beside the chain: 404 us against 504 for the two components along z.)
-template <int NC, int S, int V>
+// SPLIT (fewer than 6 digits): the residual as two polynomials in r^2 (k_near_field), whose
+// coefficients depend on the entry's bs: a row reads its entry's NC coefficients with the entry's
+// geometry.  N = 4e5, 3 digits: 500 us alone with one list per wavefront, 300 with row lists.
+template <int NC, int S, int V, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict__ src, const P4<float> *__restrict__ trg,
                                                    const int4 *__restrict__ items, const int *__restrict__ l1_ptr,
                                                    const P4<float> *__restrict__ geom, const int *__restrict__ rs_base,
                                                    const int *__restrict__ rslot, const long long *__restrict__ wave_base,
                                                    const int *__restrict__ steps, const float *__restrict__ coeffs,
                                                    float *__restrict__ pot_sorted, int item0, int item1, int ne_max,
-                                                   long long vs_src = 0, long long vs_pot = 0) {
+                                                   long long vs_src = 0, long long vs_pot = 0,
+                                                   const NfEntry *__restrict__ l1 = nullptr) {
     extern __shared__ float4 nf_lds[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int item = S > 1 ? (int)blockIdx.x * S + w
@@ -2009,12 +2016,14 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     if (S == 1 && item >= item1) return;  // whole wavefront (no workgroup barrier below)
     const int lane = threadIdx.x & 63, g = lane >> 2;
     const int4 it = items[item];  // (first target, count, target-leaf list index, K)
-    // this wavefront's LDS: ne_max + 1 entries x (offset+bs, consts), then (ne_max + 1) x 16 slots
-    float4 *geo = nf_lds + (size_t)w * (ne_max + 1) * 6;
-    int *slots = reinterpret_cast<int *>(geo + 2 * (ne_max + 1));
+    // this wavefront's LDS: ne_max + 1 entries x GS float4 (offset, bs^2, then 2/bs and -bs/2, or the
+    // coefficients), then (ne_max + 1) x 16 slots
+    constexpr int GS = nf_geo_f4<NC, SPLIT>();
+    float4 *geo = nf_lds + (size_t)w * (ne_max + 1) * (GS + 4);
+    int *slots = reinterpret_cast<int *>(geo + GS * (ne_max + 1));
     const int eb = l1_ptr[it.z], ne = l1_ptr[it.z + 1] - eb;
     // S > 1: the entries' sums [V][ne + 1][64]
-    float *sums = reinterpret_cast<float *>(nf_lds + (size_t)S * (ne_max + 1) * 6);
+    float *sums = reinterpret_cast<float *>(nf_lds + (size_t)S * (ne_max + 1) * (GS + 4));
     if (S > 1) {
         for (int k = threadIdx.x; k < V * (ne + 1) * 64; k += 64 * S) sums[k] = 0;
         __syncthreads();
@@ -2022,15 +2031,22 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     for (int e = lane; e <= ne; e += 64) {
         const P4<float> gm = e < ne ? geom[eb + e] : P4<float>{0.0f, 0.0f, 0.0f, 0.0f};
         const float bs = gm.w;
-        geo[2 * e] = make_float4(gm.x, gm.y, gm.z, bs * bs);
-        geo[2 * e + 1] = make_float4(e < ne ? 2.0f / bs : 0.0f, -bs / 2.0f, 0.0f, 0.0f);
+        geo[GS * e] = make_float4(gm.x, gm.y, gm.z, bs * bs);
+        if constexpr (SPLIT) {
+            const float *ce = coeffs + (e < ne ? l1[eb + e].cfidx : 0) * NF_SPLIT_STRIDE;
+            float *o = reinterpret_cast<float *>(geo + GS * e + 1);
+#pragma unroll
+            for (int i = 0; i < 4 * (GS - 1); ++i) o[i] = i < NC ? ce[i] : 0.0f;
+        } else {
+            geo[GS * e + 1] = make_float4(e < ne ? 2.0f / bs : 0.0f, -bs / 2.0f, 0.0f, 0.0f);
+        }
     }
     const int *rs = rslot + (size_t)rs_base[item] * NF_ROWS;
     const int n_slots = S > 1 ? rs_base[item + 1] - rs_base[item] : ne + 1;
     const unsigned geo_off = (unsigned)((const char *)geo - (const char *)nf_lds);
     for (int k = lane; k < n_slots * NF_ROWS; k += 64) {
         const int v = rs[k];
-        slots[k] = (int)(((unsigned)min(v >> 8, 0xffff) << 16) | (geo_off + 32u * (unsigned)(v & 255)));
+        slots[k] = (int)(((unsigned)min(v >> 8, 0xffff) << 16) | (geo_off + 16u * GS * (unsigned)(v & 255)));
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -2039,12 +2055,12 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
     const P4<float> me = active ? trg[it.x + lane] : P4<float>{1e18f, 1e18f, 1e18f, 0.0f};
     float c[NC];
 #pragma unroll
-    for (int i = 0; i < NC; ++i) c[i] = coeffs[i];
+    for (int i = 0; i < NC; ++i) c[i] = SPLIT ? 0.0f : coeffs[i];
     // the second-highest coefficient in a vector register: the first Horner step then takes
     // the highest from a scalar register and needs no copy per pair (one scalar operand per
     // FMA)
-    float c_next;
-    asm("v_mov_b32 %0, %1" : "=v"(c_next) : "s"(c[NC - 2]));
+    float c_next = 0;
+    if constexpr (!SPLIT) asm("v_mov_b32 %0, %1" : "=v"(c_next) : "s"(c[NC - 2]));
     float tx = 0, ty = 0, tz = 0, d2max = 0, rsc = 0, cen = 0;
     int end = 0;
     const int *slot = slots + g;  // the row's next slot
@@ -2066,15 +2082,21 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
         const unsigned v = (unsigned)*slot;
         slot += NF_ROWS;
         end = (int)(v >> 16);
-        if (S > 1) sum = sums + ((v & 0xffffu) - geo_off) * 2 + lane;  // 32 bytes of geometry, 64 sums
+        if (S > 1) sum = sums + ((v & 0xffffu) - geo_off) / (16u * GS) * 64u + lane;
         const float4 *ge = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(nf_lds) + (v & 0xffffu));
         const float4 a = ge[0], b = ge[1];
         tx = me.x + a.x;
         ty = me.y + a.y;
         tz = me.z + a.z;
         d2max = a.w;
-        rsc = b.x;
-        cen = b.y;
+        if constexpr (SPLIT) {
+            const float *ce = reinterpret_cast<const float *>(ge + 1);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) c[i] = ce[i];
+        } else {
+            rsc = b.x;
+            cen = b.y;
+        }
     };
     enter();
     const int K = it.w;
@@ -2109,11 +2131,21 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
             float u = 0;
             if (r2 < d2max && r2 > 1e-30f) {
                 const float rinv = rsqrt_full<float>(r2);
-                const float x = fmaf(r2, rinv, cen) * rsc;
-                float p = fmaf(c[NC - 1], x, c_next);
+                if constexpr (SPLIT) {
+                    constexpr int SE = (NC - 1) & ~1, SO = ((NC - 2) & ~1) + 1;
+                    float Ev = c[SE], Od = c[SO];
 #pragma unroll
-                for (int i = NC - 3; i >= 0; --i) p = fmaf(p, x, c[i]);
-                u = p * rinv;
+                    for (int i = SE - 2; i >= 0; i -= 2) Ev = fmaf(Ev, r2, c[i]);
+#pragma unroll
+                    for (int i = SO - 2; i >= 0; i -= 2) Od = fmaf(Od, r2, c[i]);
+                    u = fmaf(Ev, rinv, Od);
+                } else {
+                    const float x = fmaf(r2, rinv, cen) * rsc;
+                    float p = fmaf(c[NC - 1], x, c_next);
+#pragma unroll
+                    for (int i = NC - 3; i >= 0; --i) p = fmaf(p, x, c[i]);
+                    u = p * rinv;
+                }
             }
             auto add = [&](float &e, float q) {
                 switch (s) {

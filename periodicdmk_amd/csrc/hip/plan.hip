@@ -105,12 +105,18 @@ int log2_bucket(long long v) {
     return b;
 }
 
+// LDS of a row near-field wavefront (FP32 below 6 digits: an entry's coefficients beside
+// its geometry)
+template <class Real> size_t near_rows_lds(int ne_max, int nc) {
+    if (!std::is_same<Real, float>::value) return near_rows64_lds_per_wave(ne_max);
+    const int geo = nc >= 12 ? nf_geo_f4<12, false>() : 1 + (nc + 3) / 4;
+    return (size_t)(ne_max + 1) * (geo + 4) * 16;
+}
+
 // LDS of a row near-field workgroup of S waves that share one item (k_near_rows, k_near_rows64)
 // (pair 2: sums of both components of a quasi-periodic tree)
-template <class Real> size_t near_parts_lds(int S, int ne_max, int pair = 1) {
-    const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(ne_max + 1) * 6 * 16
-                                                             : near_rows64_lds_per_wave(ne_max);
-    return S * per_wave + (size_t)(ne_max + 1) * 64 * sizeof(Real) * pair;
+template <class Real> size_t near_parts_lds(int S, int ne_max, int nc, int pair = 1) {
+    return S * near_rows_lds<Real>(ne_max, nc) + (size_t)(ne_max + 1) * 64 * sizeof(Real) * pair;
 }
 
 // Waves per item of the row near field.  Alone, 6 digits FP32 / FP64, one wave per item against
@@ -122,15 +128,15 @@ template <class Real> size_t near_parts_lds(int S, int ne_max, int pair = 1) {
 // 843): 8 waves up to 256 items, 4 up to 1280 (2560 for quasi-periodic trees, whose near field
 // forms both components: N = 1e5, 1834 items, 1017 -> 867 us per call), within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or
 // 8 forces a count).
-template <class Real> int near_parts(int n_items, int ne_max, bool qp) {
+template <class Real> int near_parts(int n_items, int ne_max, int nc, bool qp) {
     const int pair = qp && std::is_same<Real, float>::value ? 2 : 1;
     int S = n_items <= 256 ? 8 : (n_items <= (qp ? 2560 : 1280) ? 4 : 1);
     if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
         const int v = std::atoi(e);
         S = v >= 8 ? 8 : (v >= 4 ? 4 : 1);
     }
-    if (S == 8 && near_parts_lds<Real>(S, ne_max, pair) > 65536) S = 4;
-    if (S == 4 && near_parts_lds<Real>(S, ne_max, pair) > 65536) S = 1;
+    if (S == 8 && near_parts_lds<Real>(S, ne_max, nc, pair) > 65536) S = 4;
+    if (S == 4 && near_parts_lds<Real>(S, ne_max, nc, pair) > 65536) S = 1;
     return S;
 }
 
@@ -796,10 +802,10 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             n_ie += ptr[itv[i].z + 1] - ptr[itv[i].z];
         }
         nf_ie_base.upload(ieb);
-        // FP32 at 6 digits: quad-row step lists (k_near_rows); PDMK_NEAR_ROWS=0 keeps the
-        // wavefront-wide lists of k_near_field
+        // FP32 up to 6 digits, FP64 at 6, 9 and 12: quad-row step lists (k_near_rows);
+        // PDMK_NEAR_ROWS=0 keeps the wavefront-wide lists of k_near_field
         const char *rows_env = std::getenv("PDMK_NEAR_ROWS");
-        nf_rows = !split && (nc == 12 || (std::is_same<Real, double>::value && (nc == 18 || nc == 25))) &&
+        nf_rows = (std::is_same<Real, float>::value ? split || nc == 12 : nc == 12 || nc == 18 || nc == 25) &&
                   !(rows_env && rows_env[0] == '0');
         std::vector<long long> wbase;
         std::vector<int> rsb, rend;
@@ -877,7 +883,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             check(hipMemGetInfo(&mem_free, &mem_total), "hipMemGetInfo");
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
             if (nf_rows) {
-                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, qp);
+                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp);
                 if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c);
             }
         }
@@ -1482,24 +1488,23 @@ template <class Real>
 void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1, bool pair) {
     if (i1 <= i0) return;
     const int S = pl.nf_parts;
-    const size_t per_wave = std::is_same<Real, float>::value ? (size_t)(pl.nf_ne_max + 1) * 6 * sizeof(float4)
-                                                             : near_rows64_lds_per_wave(pl.nf_ne_max);
+    const size_t per_wave = near_rows_lds<Real>(pl.nf_ne_max, pl.nc);
     // (the LDS tables of a workgroup's wavefronts stay within 64 KiB)
     while (wpb > 1 && (size_t)wpb * per_wave > 65536) wpb /= 2;
     const NearSrc<Real> N(pl, pair);
     // FP32: one launch forms both components of a pair (V = 2); FP64: components along z
     constexpr bool F32 = std::is_same<Real, float>::value;
     const int nz = F32 ? 1 : N.nz;
-    auto go = [&](auto kern) {
+    auto go = [&](auto kern, auto... l1) {  // l1: the entries' coefficient rows, where the kernel reads them
         if (S > 1)
             hipLaunchKernelGGL(kern, dim3(i1 - i0, 1, nz), dim3(64 * S),
-                               near_parts_lds<Real>(S, pl.nf_ne_max, F32 ? N.nz : 1), s,
+                               near_parts_lds<Real>(S, pl.nf_ne_max, pl.nc, F32 ? N.nz : 1), s,
                                N.src, pl.trg.template as<P4<Real>>(),
                                pl.np_items.template as<int4>(), pl.nf_ptr.template as<int>(),
                                pl.nf_geom.template as<P4<Real>>(), pl.np_rs_base.template as<int>(),
                                pl.np_rslot.template as<int>(), pl.np_wave_base.template as<long long>(),
                                pl.np_steps.template as<int>(), pl.coeffs.template as<Real>(),
-                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot);
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot, l1...);
         else
             hipLaunchKernelGGL(kern, dim3((i1 - i0 + wpb - 1) / wpb, 1, nz), dim3(64 * wpb), wpb * per_wave, s,
                                N.src, pl.trg.template as<P4<Real>>(),
@@ -1507,24 +1512,26 @@ void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1, bo
                                pl.nf_geom.template as<P4<Real>>(), pl.nf_rs_base.template as<int>(),
                                pl.nf_rslot.template as<int>(), pl.nf_wave_base.template as<long long>(),
                                pl.nf_row_steps.template as<int>(), pl.coeffs.template as<Real>(),
-                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot);
+                               pl.pot_near.template as<Real>(), i0, i1, pl.nf_ne_max, N.vs_src, N.vs_pot, l1...);
         check(hipGetLastError(), "k_near_rows");
     };
     auto by_parts = [&](auto nc) {
         constexpr int NC = decltype(nc)::value;
         if constexpr (F32) {
+            constexpr bool SP = NC < 12;
+            const NfEntry *l1 = SP ? pl.nf_l1.template as<NfEntry>() : nullptr;
             if (pair) {
                 switch (S) {
-                case 8: go(k_near_rows<NC, 8, 2>); break;
-                case 4: go(k_near_rows<NC, 4, 2>); break;
-                default: go(k_near_rows<NC, 1, 2>); break;
+                case 8: go(k_near_rows<NC, 8, 2, SP>, l1); break;
+                case 4: go(k_near_rows<NC, 4, 2, SP>, l1); break;
+                default: go(k_near_rows<NC, 1, 2, SP>, l1); break;
                 }
                 return;
             }
             switch (S) {
-            case 8: go(k_near_rows<NC, 8, 1>); break;
-            case 4: go(k_near_rows<NC, 4, 1>); break;
-            default: go(k_near_rows<NC, 1, 1>); break;
+            case 8: go(k_near_rows<NC, 8, 1, SP>, l1); break;
+            case 4: go(k_near_rows<NC, 4, 1, SP>, l1); break;
+            default: go(k_near_rows<NC, 1, 1, SP>, l1); break;
             }
         } else {
             switch (S) {
@@ -1535,6 +1542,18 @@ void launch_near_rows(Plan<Real> &pl, hipStream_t s, int wpb, int i0, int i1, bo
         }
     };
     switch (pl.nc) {
+    case 5:
+        if constexpr (F32) { by_parts(std::integral_constant<int, 5>{}); return; }
+        break;
+    case 6:
+        if constexpr (F32) { by_parts(std::integral_constant<int, 6>{}); return; }
+        break;
+    case 9:
+        if constexpr (F32) { by_parts(std::integral_constant<int, 9>{}); return; }
+        break;
+    case 11:
+        if constexpr (F32) { by_parts(std::integral_constant<int, 11>{}); return; }
+        break;
     case 12: by_parts(std::integral_constant<int, 12>{}); return;
     case 18:
         if constexpr (std::is_same<Real, double>::value) { by_parts(std::integral_constant<int, 18>{}); return; }
@@ -1852,7 +1871,7 @@ void Plan<Real>::autotune(int repeats, double *ms_default, double *ms_tuned) {
     const double base = time_ms();
     double best = base;
     // the rows near field keeps its LDS tables under 64 KiB per workgroup
-    const size_t rows_lds_wave = nf_rows ? (size_t)(nf_ne_max + 1) * 6 * 16 : 0;
+    const size_t rows_lds_wave = nf_rows ? near_rows_lds<Real>(nf_ne_max, nc) : 0;
     auto try_values = [&](int Knobs::*field, std::initializer_list<int> values) {
         int best_v = knobs.*field;
         for (int v : values) {

@@ -1,7 +1,8 @@
 """The row near field with several waves per item (trees with few items: each wave walks the
 lists of its share of an item's list1 entries) against the wavefront-wide lists
 (PDMK_NEAR_ROWS=0): the entries' sums are added in entry order whatever the number of waves, so
-the near-field potentials are bit-identical (tolerance 0).  4 and 8 waves (PDMK_NEAR_PARTS)
+the near-field potentials are bit-identical (tolerance 0).  Below 6 digits (FP32) the rows read
+their entries' coefficients with the geometry.  4 and 8 waves (PDMK_NEAR_PARTS)
 and the built-in choice; a single point, fewer targets than a row, partly filled items, more
 parts than non-empty entries, uneven entries (clusters), 64 targets and one more."""
 import numpy as np
@@ -23,7 +24,8 @@ CASES = {
 
 
 @pytest.mark.parametrize("name", list(CASES))
-@pytest.mark.parametrize("precision,digits", [("float", 6), ("double", 6), ("double", 9), ("double", 12)])
+@pytest.mark.parametrize("precision,digits", [("float", 1), ("float", 3), ("float", 4), ("float", 5), ("float", 6),
+                                              ("double", 6), ("double", 9), ("double", 12)])
 def test_parts_equal_wavefront_lists(pdmk, cuda, monkeypatch, name, precision, digits):
     cell, pos, npl = CASES[name]()
     q = 2.0 * W.uniform01(78, pos.shape[0]) - 1.0
