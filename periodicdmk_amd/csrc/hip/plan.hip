@@ -1611,7 +1611,12 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     // evaluate_timed's split (far field, proxy/plane waves, near field) needs the stages one
     // after the other; otherwise the far field and the near field run on their own streams
     // beside the transform chain and join before the final combination
-    const bool serial = times_ms != nullptr || single_stream;
+    // (small trees too: the eight event calls of the fork and join take the host longer than the
+    // stages beside each other save.  One stream against three, us per call: 3 digits N = 1e3
+    // 51 / 75, 5e3 73 / 104; 6 digits FP32 1e3 72 / 105, 2e3 78 / 76; FP64 1e3 88 / 107, 2e3
+    // 96 / 80; 9 digits never)
+    const bool small = p < 28 && (long)n * (p == 9 ? 1 : (sizeof(Real) == 4 ? 4 : 6)) <= 6000;
+    const bool serial = times_ms != nullptr || single_stream || small;
     hipStream_t sf = serial ? s : s_far, sn = serial ? s : s_near;
     if (!serial) {
         check(hipEventRecord(e_in, s), "hipEventRecord");
