@@ -857,6 +857,120 @@ __global__ __launch_bounds__(256) void k_proxy2pw(const R *__restrict__ proxy, C
     }
 }
 
+// The same transform in FP32 at p = 18 (n = 27) on 4-wide matrix-core blocks (v_mfma_f32_4x4x1, see
+// k_charge2proxy): a lane owns a column and supplies its input as the B operand, the folded
+// matrix F[j][k] (real part of W(k, j) for even j, imaginary part for odd j) comes as the A operand
+// that broadcasts one block of 4 outputs to all lanes; 28 outputs of two j fill one register.
+// The parity of j picks the components as in k_proxy2pw, and every output is the same chain of
+// fused multiply-adds over j, bit for bit.  A workgroup of 6 waves takes 7 k3 planes of a box
+// (half the box): z in 6 column groups, y in 2 groups x 3 parts of the outputs, x in 3 x 2.
+// The vector kernel ran at 29% of the vector rate on its matrix loads; 432 boxes x 4 vectors:
+// 106 -> 54 us, 576 boxes 36 -> 22 us, 64 boxes 11.5 -> 5.4 us alone.
+struct P2pw4Cfg {
+    static constexpr int P = 18, NPW = 27, H = 14, K3 = 7, KG = 7, NW = 6, TS = 19, slices = H / K3;
+};
+template <int B, int G0, int... I>
+__device__ __forceinline__ void p2pw4_step(float a, Cx<float> v, c2p_f4 *re, c2p_f4 *im, std::integer_sequence<int, I...>) {
+    const float xr = (B & 1) ? -v.im : v.re, xi = (B & 1) ? v.re : v.im;
+    constexpr int blk = (B & 1) * P2pw4Cfg::KG + G0;
+    ((re[I] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, xr, re[I], 4, blk + I, 0)), ...);
+    ((im[I] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, xi, im[I], 4, blk + I, 0)), ...);
+}
+// outputs 4 G0 .. 4 (G0 + GN) - 1 of one column over its 18 inputs
+template <int G0, int GN, int... B>
+__device__ __forceinline__ void p2pw4_column(const float *a, const Cx<float> *v, c2p_f4 *re, c2p_f4 *im,
+                                             std::integer_sequence<int, B...>) {
+#pragma unroll
+    for (int g = 0; g < GN; ++g) re[g] = im[g] = c2p_f4{0, 0, 0, 0};
+    (p2pw4_step<B, G0>(a[B / 2], v[B], re, im, std::make_integer_sequence<int, GN>{}), ...);
+}
+template <int... C>
+__device__ __forceinline__ void p2pw4_z(const float *a, const float *x, c2p_f4 *re, c2p_f4 *im, std::integer_sequence<int, C...>) {
+    // even c into re, odd c into im, outputs in 2 groups
+    (((C & 1) ? (im[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[C / 8], x[C], im[0], 4, C % 8 * 2, 0),
+                 im[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[C / 8], x[C], im[1], 4, C % 8 * 2 + 1, 0))
+              : (re[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[C / 8], x[C], re[0], 4, C % 8 * 2, 0),
+                 re[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[C / 8], x[C], re[1], 4, C % 8 * 2 + 1, 0))),
+     ...);
+}
+__global__ __launch_bounds__(64 * P2pw4Cfg::NW, 2) void k_proxy2pw_m4(const float *__restrict__ proxy,
+                                                                      Cx<float> *__restrict__ pw_out,
+                                                                      const float *__restrict__ F, int slot0, int n_boxes,
+                                                                      long long vs_in, long long vs_out) {
+    chain_priority();
+    proxy += (long long)blockIdx.z * vs_in;
+    pw_out += (long long)blockIdx.z * vs_out;
+    constexpr int P = P2pw4Cfg::P, NPW = P2pw4Cfg::NPW, H = P2pw4Cfg::H, K3 = P2pw4Cfg::K3, TS = P2pw4Cfg::TS, PP = P * P,
+                  COL = H * NPW, NS = P2pw4Cfg::slices;
+    __shared__ Cx<float> T1[K3 * PP], T2[K3 * NPW * TS];
+    const int lg = xcd_block(blockIdx.x, gridDim.x), bx = lg / NS, k30 = (lg - bx * NS) * K3;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float *C = proxy + (size_t)(slot0 + bx) * P * PP;
+    using Js = std::make_integer_sequence<int, P>;
+    // A registers: rows 2 r and 2 r + 1 of F, 28 outputs each; for z rows 8 r .. 8 r + 7, this
+    // workgroup's 7 outputs (and one more) each
+    float a[P / 2], az[3];
+#pragma unroll
+    for (int r = 0; r < P / 2; ++r) a[r] = lane < 56 ? F[(2 * r + (lane >= 28)) * 64 + lane - (lane >= 28 ? 28 : 0)] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int j = 8 * r + lane / 8;
+        az[r] = j < P ? F[j * 64 + k30 + lane % 8] : 0.0f;
+    }
+    {
+        const int col = 64 * w + lane, cc = min(col, PP - 1);
+        float x[P];
+#pragma unroll
+        for (int c = 0; c < P; ++c) x[c] = C[c * PP + cc];
+        c2p_f4 re[2], im[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) re[g] = im[g] = c2p_f4{0, 0, 0, 0};
+        p2pw4_z(az, x, re, im, Js{});
+        if (col < PP)
+#pragma unroll
+            for (int k = 0; k < K3; ++k) T1[k * PP + col] = {re[k >> 2][k & 3], im[k >> 2][k & 3]};
+    }
+    __syncthreads();
+    {
+        const int col = 64 * (w / 3) + lane, cc = min(col, K3 * P - 1), k = cc / P, aa = cc - k * P;
+        Cx<float> v[P];
+#pragma unroll
+        for (int b = 0; b < P; ++b) v[b] = T1[k * PP + b * P + aa];
+        auto part = [&](auto g0, auto gn) {
+            constexpr int G0 = decltype(g0)::value, GN = decltype(gn)::value;
+            c2p_f4 re[GN], im[GN];
+            p2pw4_column<G0, GN>(a, v, re, im, Js{});
+            if (col < K3 * P)
+#pragma unroll
+                for (int i = 0; i < 4 * GN; ++i)
+                    if (4 * G0 + i < NPW) T2[(k * NPW + 4 * G0 + i) * TS + aa] = {re[i >> 2][i & 3], im[i >> 2][i & 3]};
+        };
+        const int sub = w % 3;
+        if (sub == 0) part(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+        else if (sub == 1) part(std::integral_constant<int, 3>{}, std::integral_constant<int, 2>{});
+        else part(std::integral_constant<int, 5>{}, std::integral_constant<int, 2>{});
+    }
+    __syncthreads();
+    {
+        const int col = 64 * (w / 2) + lane, cc = min(col, K3 * NPW - 1);
+        Cx<float> v[P];
+#pragma unroll
+        for (int i = 0; i < P; ++i) v[i] = T2[cc * TS + i];
+        Cx<float> *dst = pw_out + (size_t)bx * NPW * COL + (size_t)k30 * NPW + cc;
+        auto part = [&](auto g0, auto gn) {
+            constexpr int G0 = decltype(g0)::value, GN = decltype(gn)::value;
+            c2p_f4 re[GN], im[GN];
+            p2pw4_column<G0, GN>(a, v, re, im, Js{});
+            if (col < K3 * NPW)
+#pragma unroll
+                for (int i = 0; i < 4 * GN; ++i)
+                    if (4 * G0 + i < NPW) dst[(size_t)(4 * G0 + i) * COL] = {re[i >> 2][i & 3], im[i >> 2][i & 3]};
+        };
+        if (w % 2 == 0) part(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+        else part(std::integral_constant<int, 4>{}, std::integral_constant<int, 3>{});
+    }
+}
+
 // Incoming expansion of one level: pin[i][m] = lscale sum_e pw_out[slot_e - slot0][m] shift0[sten_e][m]
 // over box i's CSR range of (neighbour slot, stencil); shift0 holds the level-0 translation
 // times the radial Fourier factor, lscale = 2^level scales the latter to this level.
