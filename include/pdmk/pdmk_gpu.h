@@ -124,8 +124,8 @@ int pdmk_gpu_stats(void* h, long long* out16);
 /// in the handle's precision (N = pdmk_gpu_n_points), enqueued on `stream` (NULL = the
 /// handle's stream).  No reference counterpart (the reference evaluates one vector per call).
 /// FP32 handles at 6 digits (the row near field) form the near field of 16 vectors per pass,
-/// each (target, source) residual once for all 16, beside the far fields, then run the proxy /
-/// plane-wave chain per vector; other handles call evaluate() per vector.  Each vector's
+/// each (target, source) residual once for all 16, beside the far fields and the proxy /
+/// plane-wave chain of several vectors per launch; other handles call evaluate() per vector.  Each vector's
 /// potentials equal pdmk_gpu_evaluate_*'s on it.  The first batched call allocates the
 /// 16-vector buffers (not capture-safe); later calls allocate nothing.  -1 on a NULL handle or
 /// buffer, n_vec < 0, a quasi-periodic handle or a HIP error.
@@ -159,7 +159,8 @@ void pdmk_gpu_tune_cache_clear(void);
 /// ran on the GPU else 0, boxes folded onto a periodic counterpart (their proxies and
 /// outgoing plane waves are not computed), proxy slots computed, 1 if the outgoing plane
 /// waves are held one level at a time (when all of them do not fit in device memory) else 0,
-/// 1 if the near field walks per-row step lists (k_near_rows: FP32 plans at 6 digits) else 0}.
+/// 1 if the near field walks per-row step lists (k_near_rows: FP32 plans up to 6 digits;
+/// k_near_rows64: FP64 plans at 6, 9 and 12) else 0}.
 /// No reference counterpart (measurement hook).
 int pdmk_gpu_build_info(void* h, double* out8);
 

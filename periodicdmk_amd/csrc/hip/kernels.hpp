@@ -576,8 +576,130 @@ __global__ __launch_bounds__((T3Cfg<R, P>::threads)) void k_tensor3(
     }
 }
 
+// The same transform in FP32 at p = 18 on 4-wide matrix-core blocks (v_mfma_f32_4x4x1, see
+// k_charge2proxy): a lane owns a column and supplies its input as the B operand, the matrix rows
+// come as the A operand that broadcasts one block of 4 outputs to all lanes.  A workgroup of 6
+// waves takes 9 of an item's 18 output planes: z in 6 column groups (12 outputs of 5 inputs fill
+// an A register), y and x in 3 column groups x 2 parts of the outputs (20 outputs of 3 inputs).
+// Every output is the chain of fused multiply-adds of k_tensor3 (c, b, a ascending, inputs in
+// order), bit for bit.  The outputs leave through LDS: 12 scalar stores a lane, 72 bytes apart,
+// held the kernel at the vector kernel's time.
+// Alone, N = 1e6: 4096 items 142 -> 77 us (stores as scalars 142), 512 items 27 -> 14; what
+// bounds it now is memory: 95 MB written and the products between the three barriers.
+struct T3m4Cfg {
+    static constexpr int P = 18, K = 9, NW = 6, TS = 19, slices = P / K;
+};
+template <int GPR, int G0, int C, int... I>
+__device__ __forceinline__ void t3m4_step(float a, float x, c2p_f4 *acc, std::integer_sequence<int, I...>) {
+    ((acc[I] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, x, acc[I], 4, C % (16 / GPR) * GPR + G0 + I, 0)), ...);
+}
+// acc += outputs 4 G0 .. 4 (G0 + GN) - 1 of one column over its inputs; GPR groups of 4 outputs
+// per input, 16 / GPR inputs per A register
+template <int GPR, int G0, int GN, int... C>
+__device__ __forceinline__ void t3m4_column(const float *a, const float *x, c2p_f4 *acc, std::integer_sequence<int, C...>) {
+    (t3m4_step<GPR, G0, C>(a[C / (16 / GPR)], x[C], acc, std::make_integer_sequence<int, GN>{}), ...);
+}
+template <bool TRANSPOSE>
+__global__ __launch_bounds__(64 * T3m4Cfg::NW, 2) void k_tensor3_m4(
+    const float *__restrict__ in_base, float *__restrict__ out_base, const int *__restrict__ item_out,
+    const int *__restrict__ item_add, const int *__restrict__ item_ptr, const int *__restrict__ in_slot,
+    const int *__restrict__ in_code, const float *__restrict__ mats_rm, long long vs_in, long long vs_out) {
+    chain_priority();
+    in_base += (long long)blockIdx.z * vs_in;
+    out_base += (long long)blockIdx.z * vs_out;
+    constexpr int P = T3m4Cfg::P, K = T3m4Cfg::K, TS = T3m4Cfg::TS, PP = P * P, NC = K * P;
+    static_assert(NC * P <= K * PP && NC * P % 4 == 0 && K * PP % 4 == 0, "output staging");
+    __shared__ __align__(16) float T1[K * PP], T2[NC * TS];  // T1[k][b][a], T2[k][b'][a]
+    const int lg = xcd_block(blockIdx.x, gridDim.x), it = lg / T3m4Cfg::slices, k0 = (lg % T3m4Cfg::slices) * K;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float *Ubase = mats_rm + (TRANSPOSE ? 2 : 0) * PP;
+    float *out = out_base + (size_t)item_out[it] * P * PP;
+    const bool add = item_add[it] != 0;
+    const int e0 = item_ptr[it], e1 = item_ptr[it + 1];
+    using Cs = std::make_integer_sequence<int, P>;
+    // this wave's column of y and x (clamped to the last one), and its part of the outputs
+    const int col = 64 * (w / 2) + lane, cc = min(col, NC - 1), kk = cc / P, aa = cc - kk * P;
+    const bool low = w % 2 == 0;  // outputs 0 .. 11, else 12 .. 17
+    // A registers of y and x: U(o, c), input c = 3 r + lane / 20, output o = lane % 20; of z: input
+    // c = 5 r + lane / 12, output k0 + lane % 12
+    const int ac = lane / 20, ao = lane % 20, zc = lane / 12, zo = lane % 12;
+    c2p_f4 acc[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) acc[g] = c2p_f4{0, 0, 0, 0};
+    for (int e = e0; e < e1; ++e) {
+        const float *in = in_base + (size_t)in_slot[e] * P * PP;
+        const int code = in_code[e];
+        const float *U0 = Ubase + (code & 1) * PP, *U1 = Ubase + ((code >> 1) & 1) * PP,
+                    *U2 = Ubase + ((code >> 2) & 1) * PP;
+        float az[4], a1[6], a0[6];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) az[r] = zo < K && zc < 5 && 5 * r + zc < P ? U2[(k0 + zo) * P + 5 * r + zc] : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 6; ++r) {
+            const bool in_u = ao < P && ac < 3;
+            a1[r] = in_u ? U1[ao * P + 3 * r + ac] : 0.0f;
+            a0[r] = in_u ? U0[ao * P + 3 * r + ac] : 0.0f;
+        }
+        // z: T1[k][b][a] = sum_c U2(k0 + k, c) in[c][b][a].  (T1's last readers are a barrier back.)
+        {
+            const int j = 64 * w + lane, jc = min(j, PP - 1);
+            float x[P];
+#pragma unroll
+            for (int c = 0; c < P; ++c) x[c] = in[c * PP + jc];
+            c2p_f4 z[3];
+#pragma unroll
+            for (int g = 0; g < 3; ++g) z[g] = c2p_f4{0, 0, 0, 0};
+            t3m4_column<3, 0, 3>(az, x, z, Cs{});
+            if (j < PP)
+#pragma unroll
+                for (int k = 0; k < K; ++k) T1[k * PP + j] = z[k >> 2][k & 3];
+        }
+        __syncthreads();
+        // y: T2[k][b'][a] = sum_b U1(b', b) T1[k][b][a]
+        {
+            float x[P];
+#pragma unroll
+            for (int b = 0; b < P; ++b) x[b] = T1[kk * PP + b * P + aa];
+            c2p_f4 y[3];
+#pragma unroll
+            for (int g = 0; g < 3; ++g) y[g] = c2p_f4{0, 0, 0, 0};
+            if (low) t3m4_column<5, 0, 3>(a1, x, y, Cs{});
+            else t3m4_column<5, 3, 2>(a1, x, y, Cs{});
+            float *dst = T2 + (size_t)(kk * P + (low ? 0 : 12)) * TS + aa;
+            if (col < NC)
+#pragma unroll
+                for (int i = 0; i < 12; ++i)
+                    if (i < 6 || low) dst[i * TS] = y[i >> 2][i & 3];
+        }
+        __syncthreads();
+        // x: acc[a'] += sum_a U0(a', a) T2[k][b'][a]
+        {
+            float x[P];
+#pragma unroll
+            for (int a = 0; a < P; ++a) x[a] = T2[cc * TS + a];
+            if (low) t3m4_column<5, 0, 3>(a0, x, acc, Cs{});
+            else t3m4_column<5, 3, 2>(a0, x, acc, Cs{});
+        }
+    }
+    // [c' = k0 + k][b'][a'] is contiguous: through T1 (read last before the barrier above), 16 bytes a lane
+    if (col < NC)
+#pragma unroll
+        for (int i = 0; i < 12; ++i)
+            if (i < 6 || low) T1[col * P + (low ? 0 : 12) + i] = acc[i >> 2][i & 3];
+    __syncthreads();
+    float4 *dst = reinterpret_cast<float4 *>(out + (size_t)k0 * PP);
+    for (int i = threadIdx.x; i < NC * P / 4; i += 64 * T3m4Cfg::NW) {
+        float4 v = reinterpret_cast<const float4 *>(T1)[i];
+        if (add) {
+            const float4 o = dst[i];
+            v.x = o.x + v.x, v.y = o.y + v.y, v.z = o.z + v.z, v.w = o.w + v.w;
+        }
+        dst[i] = v;
+    }
+}
+
 // The same transform for FP64 at p = 28 on the matrix cores (v_mfma_f64_16x16x4f64,
-// operand and accumulator layout as in k_charge2proxy_mfma).  Workgroup (item, ct) computes
+// operand and accumulator layout as in k_eval_targets_mfma).  Workgroup (item, ct) computes
 // the output planes c' in [16 ct, 16 ct + 16), the item's inputs taken in slices of 4 values
 // of a:
 //   z:  T1[c'][(b, al)]  = sum_c U2(c', c) in[c][b][4 s + al]        (16 rows, 4 p columns)

@@ -1283,6 +1283,16 @@ void launch_tensor3(const Real *in, Real *out, typename Plan<Real>::Tensor3Launc
             return;
         }
     }
+    // FP32 at p = 18: matrix-core blocks unless a knob asks for a vector shape
+    if constexpr (std::is_same_v<Real, float> && P == T3m4Cfg::P) {
+        if (div == 1) {
+            hipLaunchKernelGGL(k_tensor3_m4<TRANSPOSE>, dim3(L.n_items * T3m4Cfg::slices, 1, nv), dim3(64 * T3m4Cfg::NW), 0, s,
+                               in, out, L.out.template as<int>(), L.add.template as<int>(), L.ptr.template as<int>(),
+                               L.in_slot.template as<int>(), L.in_code.template as<int>(), mats_rm, vs_in, vs_out);
+            check(hipGetLastError(), "k_tensor3_m4");
+            return;
+        }
+    }
     constexpr int KC = T3Cfg<Real, P>::KC;
     int kc = std::max(1, KC / std::max(1, div));
     while (kc > 1 && (long)L.n_items * ((P + kc - 1) / kc) < 1024) kc = (kc + 1) / 2;

@@ -203,7 +203,7 @@ struct Plan {
     int n_nf_leaves = 0, n_nf_items = 0;
     long long n_nf_steps = 0;
     DevBuf nf_trg, nf_ptr, nf_l1, nf_geom, nf_items, nf_wbox, nf_cbox, coeffs, nf_ie_base, nf_ie_ptr, nf_steps;
-    // quad-row step lists (FP32 at 6 digits): per item the row blocks from nf_wave_base[i]
+    // quad-row step lists (FP32 up to 6 digits, FP64 at 6, 9 and 12): per item the row blocks from nf_wave_base[i]
     // (K steps per row in nf_items[i].w), per (item, row) the entry slots from nf_rs_base[i]
     bool nf_rows = false;
     int nf_ne_max = 0;  // most list1 entries of a target leaf
@@ -247,7 +247,7 @@ struct Plan {
     // plans with row step lists take the vectors in passes of 16: the near field of the pass
     // (each pair's residual formed once for the 16 vectors) on s_near, the far fields on s_far
     // (the exact Fourier sum of several vectors per launch, the phases of a workgroup shared by
-    // FF_MANY_S / FF_MANY_E vectors) and the proxy / plane-wave chain of
+    // FF_MANY vectors) and the proxy / plane-wave chain of
     // several vectors per launch on s, the three beside each other and beside the next pass;
     // other plans call evaluate() per vector.  Each vector's potentials equal evaluate()'s on
     // it bit for bit.  The per-vector buffers are allocated on first use (many_ensure).
