@@ -562,18 +562,21 @@ __global__ __launch_bounds__((T3Cfg<R, P>::threads)) void k_tensor3(
             }
         }
     }
+    // [c' = k0 + k][b'][a'] is contiguous: through T1 (read last before the barrier above)
 #pragma unroll
     for (int q = 0; q < XC; ++q) {
         const int w = threadIdx.x + q * NT;
         int col, sg;
         t3_slot<SG>(w, col, sg);
         if (w < nslot && col < nk * P) {
-            R *dst = out + (size_t)k0 * PP + (size_t)col * P + sg * PS;  // [c' = k0 + k][b'][a']
 #pragma unroll
             for (int i = 0; i < PS; ++i)
-                if (sg * PS + i < P) dst[i] = add ? dst[i] + acc[q][i] : acc[q][i];
+                if (sg * PS + i < P) T1[col * P + sg * PS + i] = acc[q][i];
         }
     }
+    __syncthreads();
+    R *dst = out + (size_t)k0 * PP;
+    for (int i = threadIdx.x; i < nk * PP; i += NT) dst[i] = add ? dst[i] + T1[i] : T1[i];
 }
 
 // The same transform in FP32 at p = 18 on 4-wide matrix-core blocks (v_mfma_f32_4x4x1, see
