@@ -146,7 +146,9 @@ int pdmk_gpu_evaluate_many(void* h, int n_vec, const void* d_charges, void* d_po
 int pdmk_gpu_autotune(void* h, int repeats, double* out8);
 /// Knobs of a handle: set5 (NULL = unchanged) = {near-field wavefronts per workgroup (0 = rule,
 /// 2, 4, 8, 16), near-field late start (-1 = rule, 0, 1), proxy -> plane-wave LDS KiB (0 = rule,
-/// 16, 32, 64), plane-wave -> proxy LDS KiB (same), tensor-transform plane divisor (1, 2, 4)};
+/// 16, 32, 64), plane-wave -> proxy LDS KiB (same), tensor-transform plane divisor (1, 2, 4)}
+/// (FP32 at p = 18 runs proxy -> plane wave and the tensor transforms on matrix-core blocks at
+/// the defaults 0 and 1, on the vector kernels at the other values);
 /// get5 (NULL = not read) receives the current ones.  -1 on a NULL handle or a value outside
 /// those sets.
 int pdmk_gpu_knobs(void* h, const int* set5, int* get5);
