@@ -562,7 +562,8 @@ __global__ __launch_bounds__((T3Cfg<R, P>::threads)) void k_tensor3(
             }
         }
     }
-    // [c' = k0 + k][b'][a'] is contiguous: through T1 (read last before the barrier above)
+    // [c' = k0 + k][b'][a'] is contiguous: through T1 (read last before the barrier above).  Stores of
+    // a row a lane: N = 1e6 FP64, 4096 boxes, 205 us; through T1 166
 #pragma unroll
     for (int q = 0; q < XC; ++q) {
         const int w = threadIdx.x + q * NT;

@@ -1283,7 +1283,8 @@ void launch_tensor3(const Real *in, Real *out, typename Plan<Real>::Tensor3Launc
             return;
         }
     }
-    // FP32 at p = 18: matrix-core blocks unless a knob asks for a vector shape
+    // FP32 at p = 18: matrix-core blocks (N = 1e6, 4096 boxes 142 -> 77 us; 512 boxes 27 -> 14) unless
+    // a knob asks for a vector shape
     if constexpr (std::is_same_v<Real, float> && P == T3m4Cfg::P) {
         if (div == 1) {
             hipLaunchKernelGGL(k_tensor3_m4<TRANSPOSE>, dim3(L.n_items * T3m4Cfg::slices, 1, nv), dim3(64 * T3m4Cfg::NW), 0, s,
