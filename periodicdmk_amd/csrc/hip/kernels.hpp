@@ -3507,4 +3507,185 @@ __global__ __launch_bounds__(64) void k_nufft_interp(const double *__restrict__ 
     reduce(nb);
 }
 
+// ------------------------------------------------------------------ quasi-periodic far field
+// psi(x_u) = e^{i b.x_u} sum_m w_m S(m) e^{i m.theta_u},  S(m) = sum_l q_l e^{-i b.x_l}
+// e^{-i m.theta_l}, over the full mode box m = (i, j, k) - (ms/2, mt/2, mu/2), index
+// i + ms (j + mt k); w_m = 0 outside the window (cpp/src/dmk/pbc.cpp:249-355).  FP64.
+// Sp[y][m]: partial structure factors of the points of workgroup column y.  Per tile of tp
+// points the per-axis factors e^{-i m_d theta_d} are tabulated in LDS by recurrence
+// (tp (ms + mt + mu + 2) complex values); a thread owns QP_CHUNK consecutive i of one (j, k)
+// line and walks them by multiplying with e^{-i theta_1}, so a (point, mode) pair costs one
+// complex multiply-add.
+//
+// For FP32 trees, whose values are rounded to FP32 after this FP64 sum: k_ff_* add in another
+// order, and a value in about 2e6 falls on the other side of its rounding.  evaluate_complex()
+// at 6 digits, FP32: N = 1e3 1100 us with the walks of one thread (reduction, evaluation) one
+// load after another, 214 with them split as below; 3e4 1755 / 512; 1e5 2350 / 1145 (k_ff_*: 180,
+// 408, 695).  Bound by FP64 vector issue: k_qp_structure 560 us beside the chain at N = 1e5.
+constexpr int QP_CHUNK = 8;
+__global__ __launch_bounds__(256) void k_qp_structure(const double *__restrict__ theta, const double *__restrict__ bx,
+                                                       const double *__restrict__ q, int n, int ms, int mt, int mu, int tp,
+                                                       double2 *__restrict__ Sp) {
+    extern __shared__ double2 qp_lds[];
+    double2 *E1 = qp_lds, *E2 = E1 + tp * ms, *E3 = E2 + tp * mt, *Q = E3 + tp * mu, *Est = Q + tp;
+    const int M = ms * mt * mu, nci = (ms + QP_CHUNK - 1) / QP_CHUNK;
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool active = c < nci * mt * mu;
+    const int i0 = active ? QP_CHUNK * (c % nci) : 0, j = active ? (c / nci) % mt : 0, k = active ? c / (nci * mt) : 0;
+    double2 acc[QP_CHUNK];
+#pragma unroll
+    for (int r = 0; r < QP_CHUNK; ++r) acc[r] = make_double2(0, 0);
+    for (int p0 = blockIdx.y * tp; p0 < n; p0 += gridDim.y * tp) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < tp * 4; t += blockDim.x) {
+            const int pp = t % tp, ax = t / tp, gp = p0 + pp;
+            if (ax == 3) {  // q e^{-i b.x}
+                double sn = 0, cs = 0;
+                if (gp < n) {
+                    sincos(-bx[gp], &sn, &cs);
+                    sn *= q[gp];
+                    cs *= q[gp];
+                }
+                Q[pp] = make_double2(cs, sn);
+                continue;
+            }
+            const int cnt = ax == 0 ? ms : (ax == 1 ? mt : mu);
+            double2 *row = (ax == 0 ? E1 : (ax == 1 ? E2 : E3)) + pp * cnt;
+            const double th = gp < n ? theta[3 * (size_t)gp + ax] : 0.0;
+            double s1, c1, sl, cl;
+            sincos(th, &s1, &c1);
+            sincos(th * (cnt / 2), &sl, &cl);
+            const double2 step = make_double2(c1, -s1);  // e^{-i th}
+            if (ax == 0) Est[pp] = step;
+            double2 cur = make_double2(cl, sl);  // e^{-i (-(cnt/2)) th}
+            for (int mm = 0; mm < cnt; ++mm) {
+                row[mm] = cur;
+                cur = cmul(cur, step);
+            }
+        }
+        __syncthreads();
+        if (active) {
+            const int np = min(tp, n - p0);
+            for (int pp = 0; pp < np; ++pp) {
+                const double2 st = Est[pp];
+                double2 cur = cmul(cmul(cmul(E1[pp * ms + i0], E2[pp * mt + j]), E3[pp * mu + k]), Q[pp]);
+#pragma unroll
+                for (int r = 0; r < QP_CHUNK; ++r) {
+                    acc[r].x += cur.x;
+                    acc[r].y += cur.y;
+                    cur = cmul(cur, st);
+                }
+            }
+        }
+    }
+    if (active) {
+        const int m0 = i0 + ms * (j + mt * k);
+#pragma unroll
+        for (int r = 0; r < QP_CHUNK; ++r)
+            if (i0 + r < ms) Sp[(size_t)blockIdx.y * M + m0 + r] = acc[r];
+    }
+}
+
+// S[m] = w[m] sum_y Sp[y][m], partials added in column order, QP_AHEAD loads in flight (N = 3e4 at
+// 3 digits, 1876 columns: 584 us one at a time, 60 with 32).
+constexpr int QP_AHEAD = 32;
+__global__ __launch_bounds__(64) void k_qp_reduce(const double2 *__restrict__ Sp, int nblk, const double *__restrict__ w,
+                                                  int M, double2 *__restrict__ S) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= M) return;
+    double2 a = make_double2(0, 0);
+    int b = 0;
+    for (; b + QP_AHEAD <= nblk; b += QP_AHEAD) {
+        double2 v[QP_AHEAD];
+#pragma unroll
+        for (int i = 0; i < QP_AHEAD; ++i) v[i] = Sp[(size_t)(b + i) * M + m];
+#pragma unroll
+        for (int i = 0; i < QP_AHEAD; ++i) {
+            a.x += v[i].x;
+            a.y += v[i].y;
+        }
+    }
+    for (; b < nblk; ++b) {
+        const double2 v = Sp[(size_t)b * M + m];
+        a.x += v.x;
+        a.y += v.y;
+    }
+    S[m] = make_double2(a.x * w[m], a.y * w[m]);
+}
+
+// far[u] = psi(x_u), 64 points per workgroup.  The i axis is taken in chunks of QP_CHUNK: the
+// chunk's factors e^{i m_1 theta_1} sit in registers and serve every (j, k) line, whose factors
+// follow recurrences in e^{i theta_2}, e^{i theta_3}; the weighted structure factors are read at
+// wave-uniform addresses.  The QP_EW waves take (chunk, k) planes in turn, and wave 0 adds their
+// sums in plane order, as one wave does that walks all planes (718 us at N = 1e5, this 390 beside
+// the chain).
+constexpr int QP_EW = 8;
+__global__ __launch_bounds__(64 * QP_EW) void k_qp_eval(const double *__restrict__ theta, const double *__restrict__ bx,
+                                                        int n, int ms, int mt, int mu, const double2 *__restrict__ S,
+                                                        double2 *__restrict__ far) {
+    __shared__ double2 part[2][QP_EW][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int u = blockIdx.x * 64 + lane, uc = min(u, n - 1);
+    double2 st[3], e[3];
+    const int cnt[3] = {ms, mt, mu};
+    for (int d = 0; d < 3; ++d) {
+        const double th = theta[3 * (size_t)uc + d];
+        double sn, cs;
+        sincos(th, &sn, &cs);
+        e[d] = make_double2(cs, sn);  // e^{i th}
+        sincos(-th * (cnt[d] / 2), &sn, &cs);
+        st[d] = make_double2(cs, sn);  // e^{i (-(cnt/2)) th}
+    }
+    const int planes = (ms + QP_CHUNK - 1) / QP_CHUNK * mu;
+    int chunk = -1, kc = 0;  // the chunk in c1, the plane of c3
+    double2 acc = make_double2(0, 0), c1next = st[0], c3 = st[2], c1[QP_CHUNK];
+    for (int p0 = 0, buf = 0; p0 < planes; p0 += QP_EW, buf ^= 1) {
+        const int p = p0 + w, c = p / mu, k = p - c * mu, i0 = c * QP_CHUNK;
+        if (p < planes) {
+            while (chunk < c) {
+#pragma unroll
+                for (int r = 0; r < QP_CHUNK; ++r) {
+                    c1[r] = c1next;
+                    c1next = cmul(c1next, e[0]);
+                }
+                ++chunk;
+                kc = 0;
+                c3 = st[2];
+            }
+            for (; kc < k; ++kc) c3 = cmul(c3, e[2]);
+            const int nr = min(QP_CHUNK, ms - i0);
+            double2 acc2 = make_double2(0, 0), c2 = st[1];
+            for (int j = 0; j < mt; ++j) {
+                const double2 *row = S + ((size_t)k * mt + j) * ms + i0;
+                double2 l = make_double2(0, 0);
+#pragma unroll
+                for (int r = 0; r < QP_CHUNK; ++r) {
+                    if (r < nr) {
+                        const double2 v = row[r];
+                        l.x = fma(v.x, c1[r].x, fma(-v.y, c1[r].y, l.x));
+                        l.y = fma(v.x, c1[r].y, fma(v.y, c1[r].x, l.y));
+                    }
+                }
+                const double2 t2 = cmul(l, c2);
+                acc2.x += t2.x;
+                acc2.y += t2.y;
+                c2 = cmul(c2, e[1]);
+            }
+            part[buf][w][lane] = cmul(acc2, c3);
+        }
+        __syncthreads();
+        // (the other buffer is written meanwhile, this one again only after the next barrier)
+        if (w == 0)
+            for (int i = 0; i < min(QP_EW, planes - p0); ++i) {
+                acc.x += part[buf][i][lane].x;
+                acc.y += part[buf][i][lane].y;
+            }
+    }
+    if (w == 0 && u < n) {
+        double sn, cs;
+        sincos(bx[u], &sn, &cs);
+        far[u] = cmul(acc, make_double2(cs, sn));
+    }
+}
+
 }  // namespace pdmk::gpu

@@ -1006,8 +1006,8 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             const double *a = T.ainv;  // a11, a21, a22, a31, a32, a33
             const double dfac = 4 * M_PI / (T.psi0 * U[0] * U[4] * U[8]);
             const host::Pswf pf(T.beta);
-            std::vector<int> qm;
-            std::vector<double> wq, bx(n);
+            std::vector<int> qm;                                // modes of nonzero weight
+            std::vector<double> wq, bx(n), wf((size_t)qs * qt * qu, 0.0);  // their weights; the whole box's
             for (int k = 0; k < qu; ++k)
                 for (int j = 0; j < qt; ++j)
                     for (int i = 0; i < qs; ++i) {
@@ -1020,12 +1020,17 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                         if (x > 1) continue;
                         for (int v : {mi, mj, mk}) qm.push_back(v);
                         wq.push_back(dfac * pf(x) / kk);
+                        wf[i + (size_t)qs * (j + (size_t)qt * k)] = wq.back();
                     }
             for (int u = 0; u < n; ++u)
                 bx[u] = bloch[0] * g.r_src[3 * (size_t)u] + bloch[1] * g.r_src[3 * (size_t)u + 1] +
                         bloch[2] * g.r_src[3 * (size_t)u + 2];
-            qpf.bx.upload(bx);
-            qpf.setup(th, n, qm, wq, nullptr, 1024);
+            if constexpr (std::is_same_v<Real, float>) {
+                qpo.setup(th, bx, n, qs, qt, qu, wf);
+            } else {
+                qpf.bx.upload(bx);
+                qpf.setup(th, n, qm, wq, nullptr, 1024);
+            }
             qp_far.alloc(sizeof(double2) * (size_t)n);
             pot_dev2.alloc(2 * sizeof(Real) * (size_t)n);
         }
@@ -1452,7 +1457,8 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
     }
     if (pl.n_leaf_eval > 0) {
         // Quasi-periodic FP32 trees keep the vector kernel: evaluate_complex hands their values out
-        // as FP64 numbers, which stay the same to the last bit.
+        // in an array of FP64 numbers, each in a fixed order of sums (QpFarField).  The matrix
+        // cores add a, b and c in another order: a third of the values one FP32 step away.
         constexpr bool kMfma = P >= 18 && (P <= 18 || std::is_same_v<Real, double>);
         bool mfma = kMfma;
         if constexpr (std::is_same_v<Real, float>) mfma = kMfma && !pl.qp;
@@ -1971,6 +1977,40 @@ int Plan<Real>::kernel_times(double *avg_ms, int *n_calls) {
     return nc;
 }
 
+void QpFarField::setup(const std::vector<double> &theta_host, const std::vector<double> &bx_host, int n_points,
+                       int ms_, int mt_, int mu_, const std::vector<double> &w_full) {
+    n = n_points;
+    ms = ms_;
+    mt = mt_;
+    mu = mu_;
+    M = ms * mt * mu;
+    theta.upload(theta_host);
+    bx.upload(bx_host);
+    w.upload(w_full);
+    // points per LDS tile: up to 16 within 48 KB of tables; point columns: enough workgroups
+    // to fill the GPU, partials M complex each
+    tp = std::max(1, std::min(16, (int)((48 << 10) / (sizeof(double2) * (size_t)(ms + mt + mu + 2)))));
+    const int cblk = (((ms + QP_CHUNK - 1) / QP_CHUNK) * mt * mu + 255) / 256;
+    nblk = std::max(1, std::min((n + tp - 1) / tp, std::max(1, 4096 / cblk)));
+    Sp.alloc(sizeof(double2) * (size_t)nblk * M);
+    S.alloc(sizeof(double2) * (size_t)M);
+}
+
+void QpFarField::run(const double *d_q, double2 *d_out, hipStream_t s) const {
+    if (n == 0) return;
+    const size_t lds = sizeof(double2) * (size_t)tp * (ms + mt + mu + 2);
+    const int nch = ((ms + QP_CHUNK - 1) / QP_CHUNK) * mt * mu;
+    hipLaunchKernelGGL(k_qp_structure, dim3((nch + 255) / 256, nblk), dim3(256), lds, s, theta.as<double>(), bx.as<double>(),
+                       d_q, n, ms, mt, mu, tp, Sp.as<double2>());
+    check(hipGetLastError(), "k_qp_structure");
+    hipLaunchKernelGGL(k_qp_reduce, dim3((M + 63) / 64), dim3(64), 0, s, Sp.as<double2>(), nblk, w.as<double>(), M,
+                       S.as<double2>());
+    check(hipGetLastError(), "k_qp_reduce");
+    hipLaunchKernelGGL(k_qp_eval, dim3((n + 63) / 64), dim3(64 * QP_EW), 0, s, theta.as<double>(), bx.as<double>(), n, ms, mt,
+                       mu, S.as<double2>(), d_out);
+    check(hipGetLastError(), "k_qp_eval");
+}
+
 template <typename Real>
 void Plan<Real>::evaluate_complex(const double *d_q, Real *d_out, hipStream_t s, int stages) {
     if (!qp) throw std::logic_error("evaluate_complex: bloch not set at construction");
@@ -1984,7 +2024,10 @@ void Plan<Real>::evaluate_complex(const double *d_q, Real *d_out, hipStream_t s,
     check(hipEventRecord(e_in, s), "hipEventRecord");
     if (!single_stream) check(hipStreamWaitEvent(sf, e_in, 0), "hipStreamWaitEvent");
     mark(0, 0, sf);
-    if (stages & 8) qpf.run(d_q, qp_far.as<double>(), sf);
+    if (stages & 8) {
+        if constexpr (std::is_same_v<Real, float>) qpo.run(d_q, qp_far.as<double2>(), sf);
+        else qpf.run(d_q, qp_far.as<double>(), sf);
+    }
     mark(0, 1, sf);
     check(hipEventRecord(e_far, sf), "hipEventRecord");
     mark(1, 0, s);

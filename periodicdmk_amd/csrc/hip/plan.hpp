@@ -123,6 +123,17 @@ struct NufftFarField {
     void run(const double *d_q, double *d_out, hipStream_t s) const;  // enqueue only
 };
 
+// The quasi-periodic sum in a fixed order, on the vector ALUs: wave vectors 2 pi U^{-T} m + b over
+// the full mode box, out[u] complex.  FP32 trees use it: they round each value to FP32 from the
+// FP64 sum, so a sum in another order (FourierSum) moves a value in about 2e6 by a whole FP32 step.
+struct QpFarField {
+    int n = 0, ms = 0, mt = 0, mu = 0, M = 0, nblk = 0, tp = 0;
+    DevBuf theta, bx, w, Sp, S;
+    void setup(const std::vector<double> &theta_host, const std::vector<double> &bx_host, int n_points, int ms_,
+               int mt_, int mu_, const std::vector<double> &w_full);
+    void run(const double *d_q, double2 *d_out, hipStream_t s) const;  // enqueue only
+};
+
 // Launch shapes of evaluate() the autotuner chooses among (0 / -1 = the built-in rule).
 struct Knobs {
     int near_wpb = 0;    // near-field wavefronts per workgroup: 0 (4, or 16 for a late start), 4, 8, 16
@@ -280,14 +291,15 @@ struct Plan {
     // per point in user order.  The charges times the real and the imaginary part of each image's
     // phase are two real vectors: one near-field launch for both, the proxy / plane-wave chain
     // for qp_nv vectors per launch (2 below p = 28 when a second set of chain buffers fits, else
-    // one after the other), beside the quasi-periodic far field on s_far; the self correction
-    // goes to the real part.
+    // one after the other), beside the quasi-periodic far field on s_far (FP32: qpo, FP64: qpf); the
+    // self correction goes to the real part.
     bool qp = false;
     double bloch[3] = {0, 0, 0};
     int qp_nv = 1;
     DevBuf src_phase;   // (cos, sin) of b.R per sorted source (R: the image's lattice translation)
     DevBuf qp_src;      // the sources twice (nsall + NF_CHUNK + 1 apart), one copy per component
     FourierSum qpf;
+    QpFarField qpo;
     DevBuf qp_far;      // complex far field, user order
     DevBuf pot_dev2;    // 2N Real for the host-buffer path
     void evaluate_complex(const double *d_q, Real *d_out, hipStream_t s, int stages = 15);

@@ -1,0 +1,52 @@
+"""The quasi-periodic far field.
+
+* FP32 trees return their values rounded to FP32 from FP64 sums in a fixed order (k_qp_structure,
+  k_qp_reduce, k_qp_eval), so that a value does not depend on how the sum is split: the five
+  values below lie within an FP64 rounding of the middle between two FP32 numbers (3e6 values
+  per tree searched), and a sum in another order gives the other one of the two.  Recorded on
+  gfx950, compared exactly.
+* Against the oracle's direct sum at the edges of the launch shapes: point counts around a
+  workgroup's 64 points, counts of partial sums around the reduction's 32 loads, mode chunks with
+  a remainder, unequal axes.  FP64 to 1e-12 (each phase is one sincos and at most 70 complex
+  products, 70 * 2 * 2^-53 * 3 axes ~ 5e-14, in both directions), FP32 to the rounding of the
+  result, 2^-23.
+"""
+import numpy as np
+import pytest
+
+from periodicdmk_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+B = np.array([2.0, -1.0, 0.5])
+CELLS = {"cubic": W.cubic_cell(), "triclinic": W.triclinic_cell(), "long": np.diag([0.5, 1.0, 2.3])}
+
+
+@pytest.mark.parametrize("digits,n,values", [
+    (4, 30011, {(30, 36419): "-0x1.091a5cp-13", (51, 11992): "0x1.17635ap-18", (113, 40203): "-0x1.36c4c6p-11"}),
+    (6, 20011, {(1, 2132): "-0x1.1e9d54p-19", (108, 35977): "0x1.e3ffb2p-12"}),
+])
+def test_fp32_values_of_the_fixed_order(pdmk, cuda, digits, n, values):
+    cell = W.cubic_cell()
+    s = pdmk.PDMKSolver(cell, W.uniform_positions(n, 41, cell), n_digits=digits, n_per_leaf=300, nz=4,
+                        precision="float", bloch=B)
+    for (seed, i), v in values.items():
+        far = s.run_complex_stages(2.0 * W.uniform01(1000 + seed, n) - 1.0, 8)
+        assert far.view(np.float64)[i] == float.fromhex(v), (seed, i)
+    s.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 513, 1041])
+@pytest.mark.parametrize("cell,digits", [("cubic", 3), ("cubic", 6), ("triclinic", 6), ("long", 6), ("long", 9)])
+def test_far_stage_edges(pdmk, oracle_mod, cuda, cell, digits, n):
+    c = CELLS[cell]
+    pos = W.uniform_positions(n, 17 + n, c)
+    q = 2.0 * W.uniform01(19 + n, n) - 1.0
+    o = oracle_mod.OracleTree(c, pos, digits, 300, 4, precision="double")
+    ref = o.evaluate_complex(q, B, 8)
+    o.close()
+    for precision, tol in (("double", 1e-12), ("float", 2.0 ** -23)):
+        s = pdmk.PDMKSolver(c, pos, n_digits=digits, n_per_leaf=300, nz=4, precision=precision, bloch=B)
+        got = s.run_complex_stages(q, 8)
+        s.close()
+        assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref), (precision, np.linalg.norm(got - ref))
