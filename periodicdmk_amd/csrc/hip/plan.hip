@@ -1025,7 +1025,8 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             for (int u = 0; u < n; ++u)
                 bx[u] = bloch[0] * g.r_src[3 * (size_t)u] + bloch[1] * g.r_src[3 * (size_t)u + 1] +
                         bloch[2] * g.r_src[3 * (size_t)u + 2];
-            if constexpr (std::is_same_v<Real, float>) {
+            qp_fixed = std::is_same_v<Real, float> || !FourierSum::fits(qs / 2, qt / 2, qu / 2);
+            if (qp_fixed) {
                 qpo.setup(th, bx, n, qs, qt, qu, wf);
             } else {
                 qpf.bx.upload(bx);
@@ -2025,7 +2026,7 @@ void Plan<Real>::evaluate_complex(const double *d_q, Real *d_out, hipStream_t s,
     if (!single_stream) check(hipStreamWaitEvent(sf, e_in, 0), "hipStreamWaitEvent");
     mark(0, 0, sf);
     if (stages & 8) {
-        if constexpr (std::is_same_v<Real, float>) qpo.run(d_q, qp_far.as<double2>(), sf);
+        if (qp_fixed) qpo.run(d_q, qp_far.as<double2>(), sf);
         else qpf.run(d_q, qp_far.as<double>(), sf);
     }
     mark(0, 1, sf);
@@ -2093,6 +2094,13 @@ void Plan<Real>::evaluate_complex_host(const double *q, Real *out) {
     check(hipMemcpyAsync(out, pot_dev2.p, 2 * sizeof(Real) * (size_t)n, hipMemcpyDeviceToHost, stream),
           "hipMemcpyAsync D2H");
     check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+}
+
+bool FourierSum::fits(int i_max, int j_max, int k_max) {
+    int dev = 0, lds = 0;
+    check(hipGetDevice(&dev), "hipGetDevice");
+    check(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev), "hipDeviceGetAttribute");
+    return FfDims{i_max, j_max, k_max}.lds_bytes(16) + 2048 <= (size_t)lds;  // (2048: the kernels' own arrays)
 }
 
 void FourierSum::setup(const std::vector<double> &theta_host, int n_points, const std::vector<int> &M,

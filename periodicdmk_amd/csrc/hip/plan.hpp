@@ -90,6 +90,9 @@ struct FourierSum {
     double *S_d = nullptr;
     void setup(const std::vector<double> &theta_host, int n_points, const std::vector<int> &mode_ijk,
                const std::vector<double> &mode_w, Arena *arena = nullptr, int max_blocks = 2048);
+    // whether the tables of the smallest point tile (16) fit a workgroup's LDS for modes up to these
+    // indices: 256 bytes per index, up to i_max + j_max + k_max = 628 within 160 KB
+    static bool fits(int i_max, int j_max, int k_max);
     void run(const double *d_q, double *d_out, hipStream_t s) const;  // enqueue only
     // S(m) from the setup points, then out[t] at n_eval other points (theta_eval[3t + d],
     // device, same convention); enqueue only
@@ -126,6 +129,8 @@ struct NufftFarField {
 // The quasi-periodic sum in a fixed order, on the vector ALUs: wave vectors 2 pi U^{-T} m + b over
 // the full mode box, out[u] complex.  FP32 trees use it: they round each value to FP32 from the
 // FP64 sum, so a sum in another order (FourierSum) moves a value in about 2e6 by a whole FP32 step.
+// FP64 trees use it on long cells, whose mode box FourierSum's tables do not fit (its own take
+// fewer points per tile, down to one).
 struct QpFarField {
     int n = 0, ms = 0, mt = 0, mu = 0, M = 0, nblk = 0, tp = 0;
     DevBuf theta, bx, w, Sp, S;
@@ -291,8 +296,8 @@ struct Plan {
     // per point in user order.  The charges times the real and the imaginary part of each image's
     // phase are two real vectors: one near-field launch for both, the proxy / plane-wave chain
     // for qp_nv vectors per launch (2 below p = 28 when a second set of chain buffers fits, else
-    // one after the other), beside the quasi-periodic far field on s_far (FP32: qpo, FP64: qpf); the
-    // self correction goes to the real part.
+    // one after the other), beside the quasi-periodic far field on s_far (qpo if qp_fixed, else
+    // qpf); the self correction goes to the real part.
     bool qp = false;
     double bloch[3] = {0, 0, 0};
     int qp_nv = 1;
@@ -300,6 +305,7 @@ struct Plan {
     DevBuf qp_src;      // the sources twice (nsall + NF_CHUNK + 1 apart), one copy per component
     FourierSum qpf;
     QpFarField qpo;
+    bool qp_fixed = false;
     DevBuf qp_far;      // complex far field, user order
     DevBuf pot_dev2;    // 2N Real for the host-buffer path
     void evaluate_complex(const double *d_q, Real *d_out, hipStream_t s, int stages = 15);

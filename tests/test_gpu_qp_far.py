@@ -10,6 +10,9 @@
   a remainder, unequal axes.  FP64 to 1e-12 (each phase is one sincos and at most 70 complex
   products, 70 * 2 * 2^-53 * 3 axes ~ 5e-14, in both directions), FP32 to the rounding of the
   result, 2^-23.
+* On a 1 x 1 x 90 cell the mode box is too long for the matrix-core sum's tables (256 bytes of LDS
+  per index of i + j + k, 160 KB): both precisions take the fixed order.  Up to 821 products along
+  the long axis: 821 * 2 * 2^-53 in both directions, below 1e-12 as well.
 """
 import numpy as np
 import pytest
@@ -50,3 +53,18 @@ def test_far_stage_edges(pdmk, oracle_mod, cuda, cell, digits, n):
         got = s.run_complex_stages(q, 8)
         s.close()
         assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref), (precision, np.linalg.norm(got - ref))
+
+
+@pytest.mark.parametrize("precision,tol,tol_all", [("double", 1e-12, 1e-12), ("float", 2.0 ** -23, 1e-5)])
+def test_long_cell(pdmk, oracle_mod, cuda, precision, tol, tol_all):
+    c, n = np.diag([1.0, 1.0, 90.0]), 130
+    pos = W.uniform_positions(n, 3, c)
+    q = 2.0 * W.uniform01(4, n) - 1.0
+    o = oracle_mod.OracleTree(c, pos, 6, 300, 4, precision="double")
+    s = pdmk.PDMKSolver(c, pos, n_digits=6, n_per_leaf=300, nz=4, precision=precision, bloch=B)
+    far, full = s.run_complex_stages(q, 8), s.evaluate_complex(q)
+    s.close()
+    ref, ref_full = o.evaluate_complex(q, B, 8), o.evaluate_complex(q, B)
+    o.close()
+    assert np.linalg.norm(far - ref) <= tol * np.linalg.norm(ref)
+    assert np.linalg.norm(full - ref_full) <= tol_all * np.linalg.norm(ref_full)
