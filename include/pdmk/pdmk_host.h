@@ -29,6 +29,14 @@ int pdmk_host_tables(int n_digits, double rc, int n_levels, const double* umat, 
 /// psi_0^c(x) for |x| <= 1 as computed by the library (unit L2 norm on [-1,1], psi(0) > 0).
 double pdmk_host_pswf(double c, double x);
 
+/// Near-field row step lists of one item cut in n_parts parts (counts[16 e + g]: steps of row g
+/// in list entry e): begin_end_steps[3 p ..] = {first entry, one past the last, steps per row}.
+int pdmk_host_row_parts(const int* counts, int n_entries, int n_parts, int* begin_end_steps);
+
+/// 1 if step lists of `indices` ints can be built beside `others` more with free_bytes of
+/// device memory (32-bit positions, a quarter of the memory), else 0.
+int pdmk_host_row_lists_fit(long long indices, long long others, unsigned long long free_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -90,6 +90,8 @@ def lib():
                                                 C.POINTER(C.c_ulonglong), C.POINTER(C.c_uint)]),
         "pdmk_campaign_read": (C.c_int, [C.c_char_p, dp, C.POINTER(C.c_uint), dp, dp, dp]),
         "pdmk_host_pswf": (C.c_double, [C.c_double, C.c_double]),
+        "pdmk_host_row_parts": (C.c_int, [ip, C.c_int, C.c_int, ip]),
+        "pdmk_host_row_lists_fit": (C.c_int, [C.c_longlong, C.c_longlong, C.c_ulonglong]),
     }
     for name, (res, args) in sig.items():
         f = getattr(L, name)

@@ -884,7 +884,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
             if (nf_rows) {
                 nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp);
-                if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c);
+                if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c, total, mem_free);
             }
         }
         if (n_nf_items > 0 && nf_rows) {
@@ -1146,10 +1146,12 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
 
 // Row lists of the items in nf_parts parts each: list1 entries in order, cut where the parts
 // hold about the same steps (rows summed); per part the rows' steps and slots as in the
-// undivided lists.  c: steps per (item, entry, row).
+// undivided lists.  c: steps per (item, entry, row).  The parts' rows are padded one by one, so
+// that their lists may be several times the undivided ones (`total` indices): one part per item
+// where they pass 32-bit positions or, with those, a quarter of the free memory.
 template <typename Real>
 void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vector<int> &ptr, const std::vector<int> &ieb,
-                                  const std::vector<int> &c) {
+                                  const std::vector<int> &c, long long total, size_t mem_free) {
     const int S = nf_parts, n_sub = n_nf_items * S;
     std::vector<int4> items(n_sub);
     std::vector<int2> range(n_sub);
@@ -1158,26 +1160,11 @@ void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vecto
     host_parallel(n_nf_items, [&](int i0, int i1) {
         for (int i = i0; i < i1; ++i) {
             const int ne = ptr[itv[i].z + 1] - ptr[itv[i].z];
-            const int *ci = &c[(size_t)ieb[i] * NF_ROWS];
-            std::vector<long> cum(ne + 1, 0);
-            for (int e = 0; e < ne; ++e) {
-                long t = 0;
-                for (int g = 0; g < NF_ROWS; ++g) t += ci[(size_t)e * NF_ROWS + g];
-                cum[e + 1] = cum[e] + t;
-            }
-            for (int p = 0, e = 0; p < S; ++p) {
-                const int e0 = e;
-                const double stop = (double)cum[ne] * (p + 1) / S;
-                // the boundary nearest to an even share
-                while (e < ne && (p == S - 1 || 0.5 * ((double)cum[e] + (double)cum[e + 1]) <= stop)) ++e;
-                range[(size_t)i * S + p] = make_int2(e0, e);
-                int kmax = 0;
-                for (int g = 0; g < NF_ROWS; ++g) {
-                    int k = 0;
-                    for (int x = e0; x < e; ++x) k += ci[(size_t)x * NF_ROWS + g];
-                    kmax = std::max(kmax, k);
-                }
-                items[(size_t)i * S + p] = make_int4(itv[i].x, itv[i].y, itv[i].z, (kmax + 3) & ~3);
+            host::RowPart part[8];  // S is 4 or 8
+            host::cut_row_lists(&c[(size_t)ieb[i] * NF_ROWS], ne, NF_ROWS, S, part);
+            for (int p = 0; p < S; ++p) {
+                range[(size_t)i * S + p] = make_int2(part[p].begin, part[p].end);
+                items[(size_t)i * S + p] = make_int4(itv[i].x, itv[i].y, itv[i].z, part[p].steps);
             }
         }
     });
@@ -1186,6 +1173,10 @@ void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vecto
         rsb[k + 1] = rsb[k] + range[k].y - range[k].x + 1;
         wb[k] = np_total;
         np_total += (long long)items[k].w * NF_ROWS;
+    }
+    if (!host::row_lists_fit(np_total + NF_ROW_PAD, total + NF_ROW_PAD, mem_free)) {
+        nf_parts = 1;
+        return;
     }
     std::vector<int> slot((size_t)rsb[n_sub] * NF_ROWS);
     host_parallel(n_nf_items, [&](int i0, int i1) {

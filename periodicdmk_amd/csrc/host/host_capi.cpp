@@ -81,4 +81,21 @@ int pdmk_host_tables(int n_digits, double rc, int n_levels, const double *umat, 
 
 double pdmk_host_pswf(double c, double x) { return Pswf(c)(x); }
 
+int pdmk_host_row_parts(const int *counts, int n_entries, int n_parts, int *begin_end_steps) {
+    if (!counts || !begin_end_steps || n_entries < 0 || n_parts < 1) return -1;
+    try {
+        std::vector<RowPart> p(n_parts);
+        cut_row_lists(counts, n_entries, 16, n_parts, p.data());
+        std::memcpy(begin_end_steps, p.data(), sizeof(RowPart) * p.size());
+        return 0;
+    } catch (const std::exception &e) {
+        std::fprintf(stderr, "pdmk_host_row_parts: %s\n", e.what());
+        return -1;
+    }
+}
+
+int pdmk_host_row_lists_fit(long long indices, long long others, unsigned long long free_bytes) {
+    return row_lists_fit(indices, others, free_bytes) ? 1 : 0;
+}
+
 }  // extern "C"

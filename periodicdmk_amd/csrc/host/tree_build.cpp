@@ -473,4 +473,29 @@ CubicCover cubic_cover(const double *cell, int nz) {
     return c;
 }
 
+void cut_row_lists(const int *c, int n_entries, int n_rows, int n_parts, RowPart *out) {
+    std::vector<long> cum(n_entries + 1, 0);
+    for (int e = 0; e < n_entries; ++e) {
+        long s = 0;
+        for (int g = 0; g < n_rows; ++g) s += c[(size_t)e * n_rows + g];
+        cum[e + 1] = cum[e] + s;
+    }
+    for (int p = 0, e = 0; p < n_parts; ++p) {
+        const int e0 = e;
+        const double stop = (double)cum[n_entries] * (p + 1) / n_parts;
+        while (e < n_entries && (p == n_parts - 1 || 0.5 * ((double)cum[e] + (double)cum[e + 1]) <= stop)) ++e;
+        int longest = 0;
+        for (int g = 0; g < n_rows; ++g) {
+            int k = 0;
+            for (int x = e0; x < e; ++x) k += c[(size_t)x * n_rows + g];
+            longest = std::max(longest, k);
+        }
+        out[p] = {e0, e, (longest + 3) & ~3};
+    }
+}
+
+bool row_lists_fit(long long indices, long long others, unsigned long long free_bytes) {
+    return indices <= 0x7fffffffLL && (double)(indices + others) * sizeof(int) <= 0.25 * (double)free_bytes;
+}
+
 }  // namespace pdmk::host

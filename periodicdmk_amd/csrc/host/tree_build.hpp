@@ -116,4 +116,15 @@ struct PointBackend {
 Tree build_tree(const Geometry &g, int n_per_leaf);  // points on the host
 Tree build_tree_with(const Geometry &g, int n_per_leaf, PointBackend &points);
 
+// Near-field row step lists of one item cut in n_parts parts: list1 entries begin .. end - 1 of
+// part p, the boundaries nearest to even shares of the steps (rows summed), and the steps of its
+// longest row, rounded up to 4 (every row of a part is padded to it).  c[e n_rows + g]: steps of
+// row g in entry e.
+struct RowPart { int begin, end, steps; };
+void cut_row_lists(const int *c, int n_entries, int n_rows, int n_parts, RowPart *out);
+
+// Whether step lists of `indices` ints can be built beside `others` more: positions within
+// 32-bit integers, and at most a quarter of the free device memory for both.
+bool row_lists_fit(long long indices, long long others, unsigned long long free_bytes);
+
 }  // namespace pdmk::host
