@@ -1767,7 +1767,7 @@ template <class R, int P> struct EvMfmaCfg {
     static constexpr int NW = 4;
     static constexpr int RH = P >= 38 ? 4 : (P >= 28 ? 2 : 1);  // passes over the leaf's targets
     static constexpr int MT = (RT + NW * RH - 1) / (NW * RH);  // (c, b) tiles per wave and pass
-    static constexpr int TT = P < 28 ? 2 : 2;   // target tiles per stage
+    static constexpr int TT = 2;                   // target tiles per stage
     static constexpr int NT = 16 * TT;             // targets per stage
     static constexpr int PA = (P + 3) / 4 * 4;
     // LDS row strides, in elements: odd, so that the 32 threads that write their targets' rows in

@@ -682,10 +682,17 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     {
         std::vector<int> ld, lt;
         std::vector<Real> lg;
-        // a leaf's targets in pieces of at most 1/1024 of all targets (whole stages of 32), so that
-        // a few large leaves do not set the time (N = 3e4, 6 digits: 9 of 449 leaves hold 440
-        // targets, the others 60: 44 -> 14 us)
-        const int piece = std::max(32, (n / 1024 + 31) / 32 * 32);
+        // Quasi-periodic FP32 trees keep the vector kernel: evaluate_complex hands their values out
+        // in an array of FP64 numbers, each in a fixed order of sums (QpFarField).  The matrix
+        // cores add a, b and c in another order: a third of the values one FP32 step away.
+        eval_mfma = (p == 18 || (p > 18 && std::is_same_v<Real, double>)) && !(qp && std::is_same_v<Real, float>);
+        // matrix cores: a leaf's targets in pieces of at most 1/1024 of all targets (whole stages of
+        // 32), so that a few large leaves do not set the time (N = 3e4, 6 digits: 9 of 449 leaves
+        // hold 440 targets, the others 60: 44 -> 14 us).  Vector kernel: in whole passes, whose time is
+        // the same for 32 targets as for 256 (evaluate(), FP32 9 digits, pieces as above / of 256 / whole
+        // leaves: N = 2e4 1177 / 1128 / 1126 us, 1e5 1530 / 1478 / 1484, clustered 1e4 1393 / 1392 / 1604;
+        // quasi-periodic 6 digits 3e4 427 / 382 / 379, 1e5 985 / 949 / 950)
+        const int piece = eval_mfma ? std::max(32, (n / 1024 + 31) / 32 * 32) : EV_THREADS * EV_TPT;
         for (int b = 0; b < nboxes; ++b) {
             if (!(t.tpeval[b] && t.trg_count[b] > 0)) continue;
             for (int t0 = 0; t0 < t.trg_count[b]; t0 += piece) {
@@ -1448,13 +1455,8 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
                                        pl.t3_mfma, nv, B.s_down, B.s_down);
     }
     if (pl.n_leaf_eval > 0) {
-        // Quasi-periodic FP32 trees keep the vector kernel: evaluate_complex hands their values out
-        // in an array of FP64 numbers, each in a fixed order of sums (QpFarField).  The matrix
-        // cores add a, b and c in another order: a third of the values one FP32 step away.
-        constexpr bool kMfma = P >= 18 && (P <= 18 || std::is_same_v<Real, double>);
-        bool mfma = kMfma;
-        if constexpr (std::is_same_v<Real, float>) mfma = kMfma && !pl.qp;
-        if (mfma) {
+        constexpr bool kMfma = P == 18 || (P > 18 && std::is_same_v<Real, double>);
+        if (pl.eval_mfma) {
             if constexpr (kMfma) {
                 hipLaunchKernelGGL((k_eval_targets_mfma<Real, P>), dim3(pl.n_leaf_eval, 1, nv),
                                    dim3(64 * EvMfmaCfg<Real, P>::NW), 0, s, B.down, pl.leaf_down.template as<int>(),

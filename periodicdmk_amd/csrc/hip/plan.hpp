@@ -186,6 +186,7 @@ struct Plan {
     // before the first plane wave is formed, on the same stream).
     bool pw_by_level = false;
     bool shift_groups = true;  // k_pw_shift_grp (p >= 28; PDMK_SHIFT_GROUPS=0 / 1 forces either)
+    bool eval_mfma = false;  // target evaluation by k_eval_targets_mfma (else k_eval_targets)
     bool t3_mfma = true;  // FP64 tensor transforms at p = 28 on the matrix cores (PDMK_T3_MFMA=0: vector ALUs)
     // several workgroups per box in FP64 charge -> proxy, for trees with fewer than
     // kC2pSplitBoxes proxy slots (the same sums; PDMK_C2P_WIDE=0 / 1 forces)
