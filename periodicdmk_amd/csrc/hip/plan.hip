@@ -1632,10 +1632,13 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     // after the other; otherwise the far field and the near field run on their own streams
     // beside the transform chain and join before the final combination
     // (small trees too: the eight event calls of the fork and join take the host longer than the
-    // stages beside each other save.  One stream against three, us per call: 3 digits N = 1e3
-    // 51 / 75, 5e3 73 / 104; 6 digits FP32 1e3 72 / 105, 2e3 78 / 76; FP64 1e3 88 / 107, 2e3
-    // 96 / 80; 9 digits never)
-    const bool small = p < 28 && (long)n * (p == 9 ? 1 : (sizeof(Real) == 4 ? 4 : 6)) <= 6000;
+    // stages beside each other save.  One stream against three, us per call: FP32 3 digits N = 1e3
+    // 54 / 93, 6e3 76 / 95, 1e4 95 / 93; 6 digits 1e3 72 / 105, 2e3 100 / 95; FP64, whose near field
+    // takes longer, 3 digits 1e3 89 / 97, 1500 101 / 99, 4e3 173 / 157; 6 digits 1e3 88 / 107, 2e3
+    // 134 / 118; 4 and 5 digits (p = 18, one list per wavefront) 500 137 / 112, 1e3 152 / 116; 9 digits
+    // never)
+    const bool f32 = sizeof(Real) == 4;
+    const bool small = p == 9 ? n <= (f32 ? 6000 : 1400) : p == 18 && (f32 || nf_rows) && n <= (f32 ? 1500 : 1000);
     const bool serial = times_ms != nullptr || single_stream || small;
     hipStream_t sf = serial ? s : s_far, sn = serial ? s : s_near;
     if (!serial) {
