@@ -168,7 +168,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
     for (auto &e : ev) check(hipEventCreate(&e), "hipEventCreate");
     check(hipStreamCreate(&s_far), "hipStreamCreate");
     check(hipStreamCreate(&s_near), "hipStreamCreate");
-    for (hipEvent_t *e : {&e_in, &e_gather, &e_far, &e_near, &e_up})
+    for (hipEvent_t *e : {&e_in, &e_gather, &e_far, &e_near, &e_near0, &e_up})
         check(hipEventCreateWithFlags(e, hipEventDisableTiming), "hipEventCreate");
     using clk = std::chrono::steady_clock;
     const auto ms_since = [](clk::time_point a) { return std::chrono::duration<double, std::milli>(clk::now() - a).count(); };
@@ -1221,7 +1221,7 @@ void Plan<Real>::release_handles() {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
     }
-    for (hipEvent_t *e : {&e_in, &e_gather, &e_far, &e_near, &e_up}) {
+    for (hipEvent_t *e : {&e_in, &e_gather, &e_far, &e_near, &e_near0, &e_up}) {
         if (*e) (void)hipEventDestroy(*e);
         *e = nullptr;
     }
@@ -1681,7 +1681,18 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     // field cut into two launches, is slower at 6 digits; the late start is faster at 9; a
     // start after the whole chain was slower at 6 and 9 digits, FP32 and FP64.)
     e_upward = near_late ? e_up : nullptr;
+    // FP64, one wave per item and few items: the near field's workgroups go out before the chain's
+    // first.  Charge -> proxy, two workgroups of 7 waves on some CUs and one on others, would leave
+    // them the latter only: two on one CU, none on the next, and twice their time alone.  (The
+    // chain waits for what the near field waits for, on the near field's stream.)  evaluate(), us,
+    // without / with: 3 digits N = 6e4 (1311 items) 480 / 344, 1e5 565 / 499, 1.5e5 (2723) 926 / 831; 5
+    // digits 2e4 (377) 702 / 610, 1e5 998 / 844; 6 digits 1e5 779 / 672, cubic 611 / 527.  Same time from
+    // 7000 items on; with 4 or 8 waves per item it is slower (6 digits 4.5e4 374 / 428), and
+    // below 300 items too (5 digits 1e4 364 / 381)
+    const bool near_first = !f32 && !serial && !near_late && nf_parts == 1 && n_nf_items >= 320 && n_nf_items <= 4096;
+    if (near_first) check(hipEventRecord(e_near0, sn), "hipEventRecord");
     if (!serial && !near_late) near();
+    if (near_first) check(hipStreamWaitEvent(s, e_near0, 0), "hipStreamWaitEvent");
     mark(2, 0, s);
     if (stages & 1) {
         run_chain(*this, s, own_chain(*this));

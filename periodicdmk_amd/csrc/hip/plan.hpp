@@ -165,7 +165,8 @@ struct Plan {
     // concurrent evaluate(): far field and near field on their own streams (default
     // priority), joined before the final combination
     hipStream_t s_far = nullptr, s_near = nullptr;
-    hipEvent_t e_in = nullptr, e_gather = nullptr, e_far = nullptr, e_near = nullptr, e_up = nullptr;
+    hipEvent_t e_in = nullptr, e_gather = nullptr, e_far = nullptr, e_near = nullptr, e_near0 = nullptr,
+               e_up = nullptr;
     hipEvent_t e_upward = nullptr;  // when set, recorded by the transform chain after the upward pass
 
     // O(N) data
