@@ -816,6 +816,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                   !(rows_env && rows_env[0] == '0');
         std::vector<long long> wbase;
         std::vector<int> rsb, rend;
+        bool whole_lists = true;  // the undivided row lists are built
         long long total = 0;
         unsigned long long np = 0;
         const dim3 grid((n_nf_items + 3) / 4);
@@ -846,14 +847,19 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                 rsb[i] = n_slots;
                 n_slots += ne + 1;
             }
-            rend.assign((size_t)n_slots * NF_ROWS, 0);
+            // Trees cut in parts walk the parts' lists only, but for the many-vector pass of FP32
+            // trees at 6 digits (construction of N = 3e4 with both lists / the parts only: 3 digits 19.6 /
+            // 17.5 ms, FP64 6 digits 28 / 25, quasi-periodic 3 digits 25 / 20)
+            nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp);
+            whole_lists = nf_parts == 1 || (std::is_same<Real, float>::value && nc == 12 && !qp);
             // items own disjoint slot ranges: rows of all items on the host threads
-            host_parallel(n_nf_items, [&](int i0, int i1) {
+            auto item_rows = [&](int i0, int i1) {
                 for (int i = i0; i < i1; ++i) {
                     const int ne = ptr[itv[i].z + 1] - ptr[itv[i].z];
                     // slot = (end step << 8) | entry ordinal; unused slots hold the terminator
-                    std::fill(rend.begin() + (size_t)rsb[i] * NF_ROWS, rend.begin() + (size_t)(rsb[i] + ne + 1) * NF_ROWS,
-                              (0x7fffff << 8) | std::min(ne, 255));
+                    if (whole_lists)
+                        std::fill(rend.begin() + (size_t)rsb[i] * NF_ROWS, rend.begin() + (size_t)(rsb[i] + ne + 1) * NF_ROWS,
+                                  (0x7fffff << 8) | std::min(ne, 255));
                     int kmax = 0;
                     for (int g = 0; g < NF_ROWS; ++g) {
                         int k = 0, sl = 0;
@@ -861,14 +867,19 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
                             const int ce = c[(size_t)(ieb[i] + e) * NF_ROWS + g];
                             if (ce == 0) continue;
                             k += ce;
-                            rend[(size_t)(rsb[i] + sl) * NF_ROWS + g] = (std::min(k, 0x7fffff) << 8) | e;
+                            if (whole_lists) rend[(size_t)(rsb[i] + sl) * NF_ROWS + g] = (std::min(k, 0x7fffff) << 8) | e;
                             ++sl;
                         }
                         kmax = std::max(kmax, k);
                     }
                     itv[i].w = (kmax + 3) & ~3;  // K
                 }
-            });
+            };
+            auto all_rows = [&]() {
+                if (whole_lists) rend.assign((size_t)n_slots * NF_ROWS, 0);
+                host_parallel(n_nf_items, item_rows);
+            };
+            all_rows();
             for (int i = 0; i < n_nf_items; ++i) {
                 k_item_max = std::max(k_item_max, itv[i].w);
                 wbase[i] = total;
@@ -889,30 +900,34 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             size_t mem_free = 0, mem_total = 0;
             check(hipMemGetInfo(&mem_free, &mem_total), "hipMemGetInfo");
             if ((double)(total + NF_ROW_PAD) * sizeof(int) > 0.25 * (double)mem_free) nf_rows = false;
-            if (nf_rows) {
-                nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp);
-                if (nf_parts > 1) build_near_parts(itv, ptr, ieb, c, total, mem_free);
+            if (nf_rows && nf_parts > 1) build_near_parts(itv, ptr, ieb, c, whole_lists ? total + NF_ROW_PAD : 0, mem_free);
+            if (!nf_rows) nf_parts = 1;
+            if (nf_rows && nf_parts == 1 && !whole_lists) {  // the parts did not fit
+                whole_lists = true;
+                all_rows();
             }
         }
         if (n_nf_items > 0 && nf_rows) {
             nf_items.upload(itv);
-            nf_rs_base.upload(rsb);
-            nf_rslot.upload(rend);
-            nf_wave_base.upload(wbase);
             // the padding points at the sentinel source (far from every target)
             const int sentinel = nsall + NF_CHUNK;
-            nf_row_steps.alloc(sizeof(int) * (size_t)(total + NF_ROW_PAD));
-            const long long n_fill = total + NF_ROW_PAD;
-            hipLaunchKernelGGL(k_fill<int>, dim3((unsigned)((n_fill + 255) / 256)), dim3(256), 0, stream,
-                               nf_row_steps.as<int>(), sentinel, (int)n_fill);
-            check(hipGetLastError(), "k_fill row steps");
-            hipLaunchKernelGGL((k_near_rows_build<Real, 1>), grid, dim3(256), 0, stream, src.as<P4<Real>>(),
-                               trg.as<P4<Real>>(), nf_items.as<int4>(), nf_wbox.as<P4<Real>>(),
-                               nf_ptr.as<int>(), nf_l1.as<NfEntry>(), nf_geom.as<P4<Real>>(),
-                               nf_cbox.as<P4<Real>>(), nf_ie_base.as<int>(), (int *)nullptr,
-                               nf_wave_base.as<long long>(), nf_row_steps.as<int>(), (unsigned long long *)nullptr,
-                               n_nf_items);
-            check(hipGetLastError(), "k_near_rows_build write");
+            if (whole_lists) {
+                nf_rs_base.upload(rsb);
+                nf_rslot.upload(rend);
+                nf_wave_base.upload(wbase);
+                nf_row_steps.alloc(sizeof(int) * (size_t)(total + NF_ROW_PAD));
+                const long long n_fill = total + NF_ROW_PAD;
+                hipLaunchKernelGGL(k_fill<int>, dim3((unsigned)((n_fill + 255) / 256)), dim3(256), 0, stream,
+                                   nf_row_steps.as<int>(), sentinel, (int)n_fill);
+                check(hipGetLastError(), "k_fill row steps");
+                hipLaunchKernelGGL((k_near_rows_build<Real, 1>), grid, dim3(256), 0, stream, src.as<P4<Real>>(),
+                                   trg.as<P4<Real>>(), nf_items.as<int4>(), nf_wbox.as<P4<Real>>(),
+                                   nf_ptr.as<int>(), nf_l1.as<NfEntry>(), nf_geom.as<P4<Real>>(),
+                                   nf_cbox.as<P4<Real>>(), nf_ie_base.as<int>(), (int *)nullptr,
+                                   nf_wave_base.as<long long>(), nf_row_steps.as<int>(), (unsigned long long *)nullptr,
+                                   n_nf_items);
+                check(hipGetLastError(), "k_near_rows_build write");
+            }
             if (nf_parts > 1) {
                 const int n_sub = n_nf_items * nf_parts;
                 hipLaunchKernelGGL(k_fill<int>, dim3((unsigned)((np_total + NF_ROW_PAD + 255) / 256)), dim3(256), 0, stream,
@@ -1154,11 +1169,11 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
 // Row lists of the items in nf_parts parts each: list1 entries in order, cut where the parts
 // hold about the same steps (rows summed); per part the rows' steps and slots as in the
 // undivided lists.  c: steps per (item, entry, row).  The parts' rows are padded one by one, so
-// that their lists may be several times the undivided ones (`total` indices): one part per item
-// where they pass 32-bit positions or, with those, a quarter of the free memory.
+// that their lists may be several times the undivided ones: one part per item where they pass 32-bit
+// positions or, with `others` indices beside them, a quarter of the free memory.
 template <typename Real>
 void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vector<int> &ptr, const std::vector<int> &ieb,
-                                  const std::vector<int> &c, long long total, size_t mem_free) {
+                                  const std::vector<int> &c, long long others, size_t mem_free) {
     const int S = nf_parts, n_sub = n_nf_items * S;
     std::vector<int4> items(n_sub);
     std::vector<int2> range(n_sub);
@@ -1181,7 +1196,7 @@ void Plan<Real>::build_near_parts(const std::vector<int4> &itv, const std::vecto
         wb[k] = np_total;
         np_total += (long long)items[k].w * NF_ROWS;
     }
-    if (!host::row_lists_fit(np_total + NF_ROW_PAD, total + NF_ROW_PAD, mem_free)) {
+    if (!host::row_lists_fit(np_total + NF_ROW_PAD, others, mem_free)) {
         nf_parts = 1;
         return;
     }

@@ -232,7 +232,7 @@ struct Plan {
     long long np_total = 0;
     DevBuf np_items, np_range, np_rs_base, np_rslot, np_wave_base, np_steps;
     void build_near_parts(const std::vector<int4> &itv, const std::vector<int> &ptr, const std::vector<int> &ieb,
-                          const std::vector<int> &c, long long total, size_t mem_free);
+                          const std::vector<int> &c, long long others, size_t mem_free);
     // far field: exact Fourier sum, or the NUFFT for large N x modes
     int far_nufft = 0;
     FourierSum ff;
