@@ -1157,8 +1157,11 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
         std::lock_guard<std::mutex> lock(tune_mu);
         tune_cache_load();
         auto it = tune_cache.find(tune_key());
+        const bool own = it != tune_cache.end();
+        if (!own) it = tune_cache.find(tune_key(false));
         if (it != tune_cache.end()) {
             knobs = it->second;
+            if (!own) knobs.p2pw_bk = Knobs{}.p2pw_bk, knobs.t3_div = Knobs{}.t3_div;
             knobs_cached = true;
         }
     }
@@ -1891,15 +1894,19 @@ void tune_cache_clear() {
     tune_file_read = true;  // the file is not read again
 }
 
+// FP32 plans at p = 18 take matrix-core kernels unless p2pw_bk or t3_div asks for a vector kernel's
+// shape, so their entries have a key of their own (":m4").  One under the key without it was tuned
+// among the vector kernels: its other knobs still hold.
 template <typename Real>
-std::string Plan<Real>::tune_key() const {
+std::string Plan<Real>::tune_key(bool m4) const {
     int dev = 0;
     hipDeviceProp_t prop{};
     check(hipGetDevice(&dev), "hipGetDevice");
     check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
     return std::string(prop.gcnArchName) + "/" + std::to_string(prop.multiProcessorCount) + ":p" + std::to_string(p) +
            ":r" + std::to_string(sizeof(Real)) + ":n" + std::to_string(log2_bucket(n)) + ":b" +
-           std::to_string(log2_bucket((long long)n_up + 1)) + ":w" + std::to_string(log2_bucket((long long)n_nf_items + 1));
+           std::to_string(log2_bucket((long long)n_up + 1)) + ":w" + std::to_string(log2_bucket((long long)n_nf_items + 1)) +
+           (m4 && std::is_same_v<Real, float> && p == T3m4Cfg::P ? ":m4" : "");
 }
 
 template <typename Real>

@@ -291,7 +291,7 @@ struct Plan {
     // faster), stores the result in the cache and returns {ms default, ms tuned}.
     Knobs knobs;
     bool knobs_cached = false;
-    std::string tune_key() const;
+    std::string tune_key(bool m4 = true) const;
     void autotune(int repeats, double *ms_default, double *ms_tuned);
 
     // Quasi-periodic evaluate (bloch given at construction): d_out holds 2N Real, (Re, Im)
