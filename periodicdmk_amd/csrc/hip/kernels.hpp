@@ -1021,7 +1021,7 @@ __device__ __forceinline__ void p2pw4_z(const float *a, const float *x, c2p_f4 *
 }
 __global__ __launch_bounds__(64 * P2pw4Cfg::NW, 2) void k_proxy2pw_m4(const float *__restrict__ proxy,
                                                                       Cx<float> *__restrict__ pw_out,
-                                                                      const float *__restrict__ F, int slot0, int n_boxes,
+                                                                      const float *__restrict__ F, int slot0,
                                                                       long long vs_in, long long vs_out) {
     chain_priority();
     proxy += (long long)blockIdx.z * vs_in;
@@ -2251,7 +2251,7 @@ __global__ __launch_bounds__(1024) void k_near_rows(const P4<float> *__restrict_
                                                    const NfEntry *__restrict__ l1 = nullptr) {
     extern __shared__ float4 nf_lds[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = S > 1 ? (int)blockIdx.x * S + w
+    const int item = S > 1 ? (item0 + (int)blockIdx.x) * S + w
                            : item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
     if (S == 1 && item >= item1) return;  // whole wavefront (no workgroup barrier below)
     const int lane = threadIdx.x & 63, g = lane >> 2;
@@ -2630,7 +2630,7 @@ __global__ __launch_bounds__(1024) void k_near_rows64(const P4<double> *__restri
     pot_sorted += (long long)blockIdx.z * vs_pot;
     extern __shared__ double2 nf_lds64[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = S > 1 ? (int)blockIdx.x * S + w
+    const int item = S > 1 ? (item0 + (int)blockIdx.x) * S + w
                            : item0 + xcd_block(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
     if (S == 1 && item >= item1) return;  // whole wavefront (no workgroup barrier below)
     const int lane = threadIdx.x & 63, g = lane >> 2;

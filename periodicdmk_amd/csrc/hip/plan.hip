@@ -1393,7 +1393,7 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
         if constexpr (std::is_same_v<Real, float> && P == P2pw4Cfg::P && NPW == P2pw4Cfg::NPW) {
             if (pl.knobs.p2pw_bk == 0) {
                 hipLaunchKernelGGL(k_proxy2pw_m4, dim3(count * P2pw4Cfg::slices, 1, nv), dim3(64 * P2pw4Cfg::NW), 0, s, B.up,
-                                   B.pw, pl.poly2pw_f.template as<float>(), slot0, count, B.s_up, B.s_pw);
+                                   B.pw, pl.poly2pw_f.template as<float>(), slot0, B.s_up, B.s_pw);
                 check(hipGetLastError(), "k_proxy2pw_m4");
                 return;
             }
