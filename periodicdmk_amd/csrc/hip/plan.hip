@@ -125,12 +125,17 @@ template <class Real> size_t near_parts_lds(int S, int ne_max, int nc, int pair 
 // 118 / 181, 115 / 187; 2048 items (1.2e5) 329 / 511, 247 / 413, 258 / 453; 4096 items (2.5e5)
 // 206 / 331, 224 / 500, -.  Beside the chain the extra waves cost it more than the near field
 // gains from about 2000 items on (2249 items, FP64: near field 793 -> 682 us, evaluate() 810 ->
-// 843): 8 waves up to 256 items, 4 up to 1280 (2560 for quasi-periodic trees, whose near field
-// forms both components: N = 1e5, 1834 items, 1017 -> 867 us per call), within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or
-// 8 forces a count).
+// 843): 8 waves up to 256 items, 4 up to 1280, within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or 8
+// forces a count).
+// Quasi-periodic trees (a second chain and a longer far field beside it), us per call with 1 / 4
+// waves: FP32 6 digits 380 items 428 / 326, 596 566 / 496, 708 414 / 425, 1829 931 / 954; FP64 6 digits
+// 380 583 / 387, 616 433 / 414, 708 400 / 428, 1829 990 / 1001: 4 up to 700.  FP32 at p = 9, whose
+// chain is short: 1020 items 220 / 232, 1923 514 / 455, 2728 901 / 702, 4173 1374 / 1065, 7566 815 /
+// 834: 4 up to 4800.
 template <class Real> int near_parts(int n_items, int ne_max, int nc, bool qp) {
     const int pair = qp && std::is_same<Real, float>::value ? 2 : 1;
-    int S = n_items <= 256 ? 8 : (n_items <= (qp ? 2560 : 1280) ? 4 : 1);
+    const int most = !qp ? 1280 : (std::is_same<Real, float>::value && nc <= 6 ? 4800 : 700);
+    int S = n_items <= 256 ? 8 : (n_items <= most ? 4 : 1);
     if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
         const int v = std::atoi(e);
         S = v >= 8 ? 8 : (v >= 4 ? 4 : 1);
