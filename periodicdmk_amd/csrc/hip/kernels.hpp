@@ -3520,8 +3520,8 @@ __global__ __launch_bounds__(64) void k_nufft_interp(const double *__restrict__ 
 // For FP32 trees, whose values are rounded to FP32 after this FP64 sum: k_ff_* add in another
 // order, and a value in about 2e6 falls on the other side of its rounding.  evaluate_complex()
 // at 6 digits, FP32: N = 1e3 1100 us with the walks of one thread (reduction, evaluation) one
-// load after another, 214 with them split as below; 3e4 1755 / 512; 1e5 2350 / 1145 (k_ff_*: 180,
-// 408, 695).  Bound by FP64 vector issue: k_qp_structure 560 us beside the chain at N = 1e5.
+// load after another, 214 with them split as below; 3e4 1755 / 470; 1e5 2370 / 1050 (k_ff_*: 180,
+// 408, 670).  Bound by FP64 vector issue: k_qp_structure 520 us beside the chain at N = 1e5.
 constexpr int QP_CHUNK = 8;
 __global__ __launch_bounds__(256) void k_qp_structure(const double *__restrict__ theta, const double *__restrict__ bx,
                                                        const double *__restrict__ q, int n, int ms, int mt, int mu, int tp,
@@ -3617,7 +3617,7 @@ __global__ __launch_bounds__(64) void k_qp_reduce(const double2 *__restrict__ Sp
 // chunk's factors e^{i m_1 theta_1} sit in registers and serve every (j, k) line, whose factors
 // follow recurrences in e^{i theta_2}, e^{i theta_3}; the weighted structure factors are read at
 // wave-uniform addresses.  The QP_EW waves take (chunk, k) planes in turn, and wave 0 adds their
-// sums in plane order, as one wave does that walks all planes (718 us at N = 1e5, this 390 beside
+// sums in plane order, as one wave does that walks all planes (718 us at N = 1e5, this 350 beside
 // the chain).
 constexpr int QP_EW = 8;
 __global__ __launch_bounds__(64 * QP_EW) void k_qp_eval(const double *__restrict__ theta, const double *__restrict__ bx,
