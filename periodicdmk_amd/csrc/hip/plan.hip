@@ -123,18 +123,26 @@ template <class Real> size_t near_parts_lds(int S, int ne_max, int nc, int pair 
 // 4 and 8: 64 items (N = 1e3) 50 / 59 us, 40 / 43, 36 / 39; 192 items (1e4) 174 / 242 us,
 // 86 / 117, 73 / 96; 512 items (3e4) 152 / 212, 82 / 111, 75 / 110; 1024 items (6e4) 167 / 243,
 // 118 / 181, 115 / 187; 2048 items (1.2e5) 329 / 511, 247 / 413, 258 / 453; 4096 items (2.5e5)
-// 206 / 331, 224 / 500, -.  Beside the chain the extra waves cost it more than the near field
-// gains from about 2000 items on (2249 items, FP64: near field 793 -> 682 us, evaluate() 810 ->
-// 843): 8 waves up to 256 items, 4 up to 1280, within 64 KiB of LDS (PDMK_NEAR_PARTS = 1, 4 or 8
-// forces a count).
+// 206 / 331, 224 / 500, -.  8 waves up to 256 items, 4 up to 1280, within 64 KiB of LDS
+// (PDMK_NEAR_PARTS = 1, 4 or 8 forces a count).
+// From there to 4800 items one wave each fills the chip about once, and what runs beside it leaves
+// some waves behind the others.  4 waves pay where the near field outweighs the chain, and cost up
+// to 7% where the chain does: they are taken for items with long lists (256 sources in support per
+// target) and, at p >= 18, for 1.2e5 pairs per proxy slot.  evaluate(), us, 1 / 4 waves (503 trees of 4e4 to
+// 2.5e5 points, 100 to 400 per leaf, cubic, triclinic and clustered, at 3, 6, 9 and 12 digits; this
+// choice is 0.4% above the better of the two in the mean, always one wave 3.9%):
+// cubic N = 2e5 (3393 items, 64 slots) FP64 6 digits 1467 / 1114, FP32 884 / 659, 9 digits 1932 / 1772,
+// triclinic (3538, 432 slots) 1491 / 1367; short lists, N = 1.3e5 (4012 items, 576 slots) 845 / 899;
+// many slots, N = 2.5e5 (4384, 3278 slots) 2182 / 2334.
 // Quasi-periodic trees (a second chain and a longer far field beside it), us per call with 1 / 4
 // waves: FP32 6 digits 380 items 428 / 326, 596 566 / 496, 708 414 / 425, 1829 931 / 954; FP64 6 digits
 // 380 583 / 387, 616 433 / 414, 708 400 / 428, 1829 990 / 1001: 4 up to 700.  FP32 at p = 9, whose
 // chain is short: 1020 items 220 / 232, 1923 514 / 455, 2728 901 / 702, 4173 1374 / 1065, 7566 815 /
 // 834: 4 up to 4800.
-template <class Real> int near_parts(int n_items, int ne_max, int nc, bool qp) {
+template <class Real> int near_parts(int n_items, int ne_max, int nc, bool qp, int n_targets, double pairs, int n_slots) {
     const int pair = qp && std::is_same<Real, float>::value ? 2 : 1;
-    const int most = !qp ? 1280 : (std::is_same<Real, float>::value && nc <= 6 ? 4800 : 700);
+    const bool heavy = pairs >= 256.0 * n_targets && (nc <= 6 || pairs >= 1.2e5 * n_slots);
+    const int most = qp ? (std::is_same<Real, float>::value && nc <= 6 ? 4800 : 700) : (heavy ? 4800 : 1280);
     int S = n_items <= 256 ? 8 : (n_items <= most ? 4 : 1);
     if (const char *e = std::getenv("PDMK_NEAR_PARTS")) {
         const int v = std::atoi(e);
@@ -855,7 +863,7 @@ Plan<Real>::Plan(const double *cell, const double *pos, int N, int n_digits_user
             // Trees cut in parts walk the parts' lists only, but for the many-vector pass of FP32
             // trees at 6 digits (construction of N = 3e4 with both lists / the parts only: 3 digits 19.6 /
             // 17.5 ms, FP64 6 digits 28 / 25, quasi-periodic 3 digits 25 / 20)
-            nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp);
+            nf_parts = near_parts<Real>(n_nf_items, nf_ne_max, nc, qp, n, (double)np, n_up);
             whole_lists = nf_parts == 1 || (std::is_same<Real, float>::value && nc == 12 && !qp);
             // items own disjoint slot ranges: rows of all items on the host threads
             auto item_rows = [&](int i0, int i1) {
