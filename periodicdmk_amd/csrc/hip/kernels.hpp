@@ -192,8 +192,10 @@ template <class R, int P> struct C2pCfg {
     static constexpr int CW = F32 ? 64 : 16;              // columns of a tile
     static constexpr int CT = (CB + CW - 1) / CW;         // column tiles
     // waves per workgroup.  FP64 at p = 28, 38: 4, one per SIMD, and two workgroups or more per CU
-    // (7 waves of 7 tiles: N = 1e6 9 digits 1012 us, clustered 8942; 5 waves: 1304)
-    static constexpr int NW = F32 ? (CT > 16 ? (CT + 1) / 2 : CT) : (P <= 18 ? 7 : 4);
+    // (7 waves of 7 tiles: N = 1e6 9 digits 1012 us, clustered 8942; 5 waves: 1304).  FP64 at p = 9: 3
+    // waves of 2 tiles, which find room beside the near field; workgroups of 7 waited for it (N = 2e5,
+    // 3888 boxes: evaluate() 571 -> 481 us; 1.5e5, 576 boxes 338 -> 306)
+    static constexpr int NW = F32 ? (CT > 16 ? (CT + 1) / 2 : CT) : (P == 9 ? 3 : (P == 18 ? 7 : 4));
     static constexpr int parts(int tpw) { return (CT + NW * tpw - 1) / (NW * tpw); }  // workgroups per box
     static constexpr int SPA = F32 ? 64 / PX : 4;         // sources per A register / product
     static constexpr int TS = F32 ? 60 / SPA * SPA : 32;  // sources per table

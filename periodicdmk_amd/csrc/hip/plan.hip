@@ -1356,10 +1356,11 @@ void launch_transforms(Plan<Real> &pl, hipStream_t s, const ChainBufs<Real> &B) 
                                pl.rng_off.template as<Real>(), B.up, B.qv, B.qv_ld, B.s_up, B.s_src);
             check(hipGetLastError(), "k_charge2proxy");
         };
-        // FP64: a box's column tiles in 1, 2 or 4 workgroups (p = 18, 28, 38), or in 3, 5 or 8 where
-        // the boxes alone leave CUs idle (64 boxes, N = 3e4: 6 digits 52 -> 29 us, 9 digits 81 -> 69)
+        // FP64: a box's column tiles in 1, 1, 2 or 4 workgroups (p = 9, 18, 28, 38), or in 3, 5 or 8 (p = 18,
+        // 28, 38) where the boxes alone leave CUs idle (64 boxes, N = 3e4: 6 digits 52 -> 29 us, 9 digits 81 -> 69)
         constexpr bool F64 = std::is_same_v<Real, double>;
-        constexpr int T_FEW = !F64 || P == 9 ? 1 : (P == 18 ? 3 : (P == 28 ? 7 : 6)), T_MANY = !F64 || P <= 18 ? 1 : 3;
+        constexpr int T_FEW = !F64 ? 1 : (P == 9 ? 2 : (P == 18 ? 3 : (P == 28 ? 7 : 6))),
+                      T_MANY = P == 9 ? T_FEW : (!F64 || P == 18 ? 1 : 3);
         if (T_MANY != T_FEW && pl.c2p_split) c2p(std::integral_constant<int, T_MANY>{});
         else c2p(std::integral_constant<int, T_FEW>{});
     }
