@@ -1700,7 +1700,11 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
         check(hipStreamWaitEvent(sn, e_gather, 0), "hipStreamWaitEvent");
     }
     const bool near_late = !serial && (knobs.near_late >= 0 ? knobs.near_late == 1 : p >= 28);
-    const int wpb = knobs.near_wpb > 0 ? knobs.near_wpb : (near_late ? 16 : 4);
+    // (2 items per workgroup at p = 18 in FP64 on wavefront lists where few boxes keep charge ->
+    // proxy on some of the CUs: 5 digits, cubic, N = 2e5 (3399 items, 172 slots) 1842 -> 1630 us; N = 6e4 (1098
+    // items) 435 -> 448)
+    const bool few_boxes = !f32 && p == 18 && !nf_rows && c2p_split && n_nf_items >= 2000;
+    const int wpb = knobs.near_wpb > 0 ? knobs.near_wpb : (near_late ? 16 : (few_boxes ? 2 : 4));
     auto near = [&]() {
         mark(3, 0, sn);
         if (stages & 2) near_field(sn, wpb);
@@ -1713,15 +1717,14 @@ void Plan<Real>::evaluate(const double *d_q, Real *d_pot, hipStream_t s, int sta
     // field cut into two launches, is slower at 6 digits; the late start is faster at 9; a
     // start after the whole chain was slower at 6 and 9 digits, FP32 and FP64.)
     e_upward = near_late ? e_up : nullptr;
-    // FP64, one wave per item and few items: the near field's workgroups go out before the chain's
-    // first.  Charge -> proxy, two workgroups of 7 waves on some CUs and one on others, would leave
-    // them the latter only: two on one CU, none on the next, and twice their time alone.  (The
-    // chain waits for what the near field waits for, on the near field's stream.)  evaluate(), us,
-    // without / with: 3 digits N = 6e4 (1311 items) 480 / 344, 1e5 565 / 499, 1.5e5 (2723) 926 / 831; 5
-    // digits 2e4 (377) 702 / 610, 1e5 998 / 844; 6 digits 1e5 779 / 672, cubic 611 / 527.  Same time from
-    // 7000 items on; with 4 or 8 waves per item it is slower (6 digits 4.5e4 374 / 428), and
-    // below 300 items too (5 digits 1e4 364 / 381)
-    const bool near_first = !f32 && !serial && !near_late && nf_parts == 1 && n_nf_items >= 320 && n_nf_items <= 4096;
+    // FP64 on wavefront lists and few items: the near field's workgroups go out before the chain's
+    // first.  Charge -> proxy, two workgroups on some CUs and one on others, would leave them the
+    // latter only: two on one CU, none on the next, and twice their time alone.  (The chain waits for
+    // what the near field waits for, on the near field's stream.)  evaluate(), us, without / with:
+    // 3 digits N = 1e5 (1919 items) 549 / 505, 1.5e5 (2723) 1041 / 854, cubic 2.3e5 (4231) 1275 / 1192; 5
+    // digits 2e4 (377) 701 / 611, 6e4 647 / 537, 1e5 984 / 835.  Same time from 5000 items on; below 300
+    // slower (5 digits 1e4 364 / 381), and so for row lists in parts (6 digits 4.5e4 374 / 428)
+    const bool near_first = !f32 && !serial && !near_late && !nf_rows && n_nf_items >= 320 && n_nf_items <= 8192;
     if (near_first) check(hipEventRecord(e_near0, sn), "hipEventRecord");
     if (!serial && !near_late) near();
     if (near_first) check(hipStreamWaitEvent(s, e_near0, 0), "hipStreamWaitEvent");
